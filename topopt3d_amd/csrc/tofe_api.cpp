@@ -2104,6 +2104,11 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       np = std::max(np, level_blocks<double>(c.get(), l));
       np = std::max(np, level_blocks<float>(c.get(), l));
     }
+    if (c->ke_wht && !c->fine_mfma) {  // any z-chunk length tofe_autotune may choose
+      FineOp<double> f = fine_of<double>(c.get());
+      f.zlen = 1;
+      np = std::max(np, fine_wht_blocks<double>(f));
+    }
     c->npart = np;
     c->partial.alloc(np);
     c->partial2.alloc(np);
