@@ -314,16 +314,21 @@ WhtGrid wht_grid(const FineOp<T> &op)
 
 int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide)
 {
-  // every step forms a full element layer, so a chunk of zlen node planes costs zlen + 1
-  // steps; the launch lasts about ceil(blocks / CUs) block-times once `hide` blocks per CU
-  // are resident (the larger chunk wins ties)
+  // A block lasts a fixed start (the first two planes and the launch itself, about two and a
+  // half steps) and zlen + 1 steps, since the chunk's lowest element layer is formed too; with m
+  // blocks on the busiest CU the launch takes a time proportional to m + hide, `hide` being the
+  // blocks whose latencies overlap for free.  Measured on MI355X over 24x12x12 to 192x96x96
+  // elements (us per apply, FP64 / FP32): one step more costs 1.33 / 1.15 on a grid of one block
+  // per CU; 24x12x12 5.1 / 4.6 at zlen 1 and 9.1 / 8.0 at 4; 96x48x48 13.5 / 9.3 at 1, 11.2 / 8.4
+  // at 2, 13.0 / 9.8 at 4; 128x64x64 17.0 / 12.3 at 3; 192x96x96 fastest at 7.  The larger chunk
+  // wins ties.
   const int tiles = ((nx + 1 + WN - 1) / WN) * ((ny + 1 + WN - 1) / WN);
   int best = 8;
   double best_cost = 1e300;
   ncu = std::max(ncu, 1);
-  for (int zl = 4; zl <= 24; ++zl) {
+  for (int zl = 1; zl <= 24; ++zl) {
     const int nb = tiles * ((nz + 1 + zl - 1) / zl);
-    const double cost = (zl + 1.0) * std::max((nb + ncu - 1) / ncu, hide);
+    const double cost = (zl + 3.0) * ((nb + ncu - 1) / ncu + hide);
     if (cost < best_cost - 1e-9 || (cost < best_cost + 1e-9 && zl > best)) {
       best_cost = cost;
       best = zl;

@@ -1876,8 +1876,8 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       TOFE_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
       c->fine_tile = fine_tile_choose(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 3);
       c->fine_tile32 = fine_tile_choose(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 6);
-      c->wht_zlen = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 3);
-      c->wht_zlen32 = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 5);
+      c->wht_zlen = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 2);
+      c->wht_zlen32 = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 4);
       if (const char *wz = std::getenv("TOFE_FINE_WHT_Z")) {
         int z64 = 0, z32 = 0;
         if (std::sscanf(wz, "%d:%d", &z64, &z32) != 2 || z64 < 1 || z64 > 64 || z32 < 1 || z32 > 64)

@@ -88,7 +88,8 @@ struct FineTile {
   int tile, zlen;
 };
 FineTile fine_tile_choose(int nx, int ny, int nz, int ncu, int hide);
-// Element-centric fine operator in the Walsh-Hadamard basis of KE (k_fine_wht).
+// Element-centric fine operator in the Walsh-Hadamard basis of KE (k_fine_wht); hide: blocks per CU
+// that overlap for free (measured: 2 for FP64, 4 for FP32).
 int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide);
 template <typename T>
 int fine_wht_blocks(const FineOp<T> &op);
