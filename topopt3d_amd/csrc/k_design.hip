@@ -9,6 +9,10 @@
 // sequential non-FMA evaluation of the reference formulas.
 #include "k_common.hpp"
 
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+
 // Keep every multiply and add separately rounded (no fused multiply-add) in this file.
 #pragma clang fp contract(off)
 
@@ -190,62 +194,179 @@ __global__ __launch_bounds__(NT) void k_rfilter_T(FilterTemplate t, const double
 // MatIntFnc after the filters (Material_Interpolation.cpp:54-116): rhoq = (q/vdMin)(1-rho)^(q-1);
 // z = rho y; dEsdz = z^(p-1); Es = dEsdz z; dEsdz *= p; dEdz = (1-eps) dEsdz;
 // E = eps + (1-eps) Es; then SIMP_CUT / SIMP_LOGISTIC modify Es and dEsdz only.
-// y == nullptr means the plain density filter (y = 1, written to yout).
-__global__ void k_simp(const double *__restrict__ rho, const double *y_in, int64_t ne,
-                       SimpParams sp, double *yout, double *rhoq, double *E, double *dEdz,
-                       double *Es, double *dEsdz, float *E32)
+__device__ inline void simp_one(int64_t i, double r, double y, const SimpParams &sp,
+                                const SimpOut &o)
 {
   const double sc = sp.vd_penal / sp.vd_min;
+  o.rhoq[i] = vecpow1(1.0 + -1 * r, sp.vd_penal - 1) * sc;
+  const double z = r * y;
+  double d = vecpow1(z, sp.penal - 1);
+  double es = d * z;
+  d = d * sp.penal;
+  const double e = sp.eps + (1 - sp.eps) * es;
+  o.dEdz[i] = d * (1 - sp.eps);
+  o.E[i] = e;
+  if (o.E32) o.E32[i] = (float)e;
+  if (sp.interp == TOFE_INTERP_SIMP_CUT) {
+    const double cut = (z > sp.p0) ? 1.0 : 0.0;
+    es = es * cut;
+    d = d * cut;
+  } else if (sp.interp == TOFE_INTERP_SIMP_LOGISTIC) {
+    const double denom = 1 + exp(sp.p0 * (sp.p1 - z));
+    es = es / denom;
+    d = (d + (es * sp.p0) * (1 - 1 / denom)) / denom;
+  }
+  o.Es[i] = es;
+  o.dEsdz[i] = d;
+}
+
+// y_in == nullptr means the plain density filter (y = 1, written to o.y).
+__global__ void k_simp(const double *__restrict__ rho, const double *y_in, int64_t ne,
+                       SimpParams sp, SimpOut o)
+{
   for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < ne; i += (int64_t)gridDim.x * NT) {
-    const double r = rho[i];
     const double y = y_in ? y_in[i] : 1.0;
-    if (!y_in) yout[i] = 1.0;
-    rhoq[i] = vecpow1(1.0 + -1 * r, sp.vd_penal - 1) * sc;
-    const double z = r * y;
-    double d = vecpow1(z, sp.penal - 1);
-    double es = d * z;
-    d = d * sp.penal;
-    const double e = sp.eps + (1 - sp.eps) * es;
-    dEdz[i] = d * (1 - sp.eps);
-    E[i] = e;
-    if (E32) E32[i] = (float)e;
-    if (sp.interp == TOFE_INTERP_SIMP_CUT) {
-      const double cut = (z > sp.p0) ? 1.0 : 0.0;
-      es = es * cut;
-      d = d * cut;
-    } else if (sp.interp == TOFE_INTERP_SIMP_LOGISTIC) {
-      const double denom = 1 + exp(sp.p0 * (sp.p1 - z));
-      es = es / denom;
-      d = (d + (es * sp.p0) * (1 - 1 / denom)) / denom;
-    }
-    Es[i] = es;
-    dEsdz[i] = d;
+    if (!y_in) o.y[i] = 1.0;
+    simp_one(i, rho[i], y, sp, o);
   }
 }
 
 // Chain_Filter middle step (Material_Interpolation.cpp:168-179):
-// out = dfdE .* y - rhoq .* ((y < 1) .* RtT), RtT = R^T(dfdE .* rho) (or nullptr: no R term)
+// out = dfdE .* y - rhoq .* ((y < 1) .* RtT), RtT = R^T(dfdE .* rho)
+__device__ inline double chain_mid_one(double g, double y, double rhoq, double rt)
+{
+  const double b = g * y;
+  const double mask = (y < 1.0) ? 1.0 : 0.0;
+  double a = rt * mask;
+  a = rhoq * a;
+  return b - a;
+}
+
 __global__ void k_chain_mid(const double *__restrict__ dfdE, const double *__restrict__ y,
                             const double *__restrict__ rhoq, const double *__restrict__ RtT,
                             double *out, int64_t ne)
 {
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < ne; i += (int64_t)gridDim.x * NT) {
-    const double b = dfdE[i] * y[i];
-    if (RtT) {
-      const double mask = (y[i] < 1.0) ? 1.0 : 0.0;
-      double a = RtT[i] * mask;
-      a = rhoq[i] * a;
-      out[i] = b - a;
-    } else {
-      out[i] = b;
-    }
-  }
+  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < ne; i += (int64_t)gridDim.x * NT)
+    out[i] = chain_mid_one(dfdE[i], y[i], rhoq[i], RtT[i]);
 }
 
 __global__ void k_mul(const double *__restrict__ a, const double *__restrict__ b, double *c, int64_t n)
 {
   for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT)
     c[i] = a[i] * b[i];
+}
+
+// Filters with a radius of up to kFilterTileMax elements, tiled through LDS.
+//
+// A block of 512 threads forms a tile of 32 x 8 x (2 RZ) outputs from one staged box of the
+// source, H elements wider on every side (zero outside the mesh: a zero term leaves a partial
+// sum as it is, for the sums start at +0 or at a value >= 0).  Every thread then walks the
+// neighbour list once, in its ascending order, for RZ outputs: one scalar load of the entry's
+// LDS offset and weight serves the wavefront, and a term costs one LDS read (two in the
+// transpose, which scales by the source's row sum) and its separately rounded operations, in
+// place of three LDS reads, three bounds checks and a gather.  The transpose visits the rows
+// e - off in ascending order; the neighbour list is symmetric with equal weights, so that is
+// the same walk.  Bound: the LDS reads, 8 bytes a term; the 32-wide rows are read without bank
+// conflicts, and z is the axis of the RZ outputs because their offsets are then immediates.
+// H is a template argument for the same reason.
+constexpr int FTX = 32, FTY = 8, FNT = 512;
+enum FiltMode : int { FM_APPLY = 0, FM_T = 1, FM_RADD = 2, FM_RT = 3 };
+// FE_PLAIN: out; FE_SIMP: rho (or y) and the interpolation; FE_VOID: rho and z = (1 - rho)^q
+enum FiltEpi : int { FE_PLAIN = 0, FE_SIMP = 1, FE_VOID = 2 };
+
+struct FilterArgs {
+  FilterTemplate t;
+  const double *src = nullptr;  // x; g; z = (1 - rho)^q; dfdE
+  const double *inv = nullptr;  // reciprocal row sums (FM_APPLY, FM_T)
+  const double *add = nullptr;  // FM_RADD: REdge
+  double scale = 0;             // FM_RADD: 1 / vdMin
+  const double *rho = nullptr;  // FM_RADD with FE_SIMP; FM_RT: the factor of dfdE
+  const double *y = nullptr, *rhoq = nullptr;  // FM_RT
+  double *out = nullptr;        // rho; P^T g; y; the chain rule's middle step
+  double *copy = nullptr;       // FM_APPLY: where x itself is kept (null: nowhere)
+  double *zt = nullptr;         // FE_VOID
+  SimpParams sp;
+  SimpOut so;
+};
+
+// planes of outputs per thread: two, or one where two would not fit the LDS
+constexpr int filter_rz(int H, int mode) { return (mode == FM_T && H >= 5) ? 1 : 2; }
+
+template <int H, int MODE, int EPI>
+__global__ __launch_bounds__(FNT) void k_filter_tile(FilterArgs a)
+{
+  constexpr int RZ = filter_rz(H, MODE);
+  constexpr int PX = FTX + 2 * H, PY = FTY + 2 * H, PZ = 2 * RZ + 2 * H, PL = PX * PY;
+  __shared__ double sv[PL * PZ];
+  __shared__ double si[MODE == FM_T ? PL * PZ : 1];
+  const int nx = a.t.nx, ny = a.t.ny, nz = a.t.nz;
+  const int bx = blockIdx.x * FTX, by = blockIdx.y * FTY, bz = blockIdx.z * (2 * RZ);
+  for (int v = threadIdx.x; v < PL * PZ; v += FNT) {
+    const int lz = v / PL, r = v - lz * PL, ly = r / PX, lx = r - ly * PX;
+    const int gx = bx - H + lx, gy = by - H + ly, gz = bz - H + lz;
+    const bool in = gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz;
+    const int64_t n = in ? gx + (int64_t)nx * (gy + (int64_t)ny * gz) : 0;
+    double x = in ? a.src[n] : 0.0;
+    if constexpr (MODE == FM_RT) x = in ? x * a.rho[n] : 0.0;
+    sv[v] = x;
+    if constexpr (MODE == FM_T) si[v] = in ? a.inv[n] : 0.0;
+  }
+  __syncthreads();
+  const int tx = threadIdx.x % FTX, ty = (threadIdx.x / FTX) % FTY, tz = threadIdx.x / (FTX * FTY);
+  const int gx = bx + tx, gy = by + ty, z0 = bz + tz * RZ;
+  if (gx >= nx || gy >= ny || z0 >= nz) return;
+  const int base = (tz * RZ * PY + ty) * PX + tx;  // the box corner of the first output
+  int64_t el[RZ];
+  double s[RZ], ie[RZ];
+#pragma unroll
+  for (int r = 0; r < RZ; ++r) {
+    el[r] = gx + (int64_t)nx * (gy + (int64_t)ny * min(z0 + r, nz - 1));
+    s[r] = 0.0;
+    ie[r] = 0.0;
+    if constexpr (MODE == FM_APPLY) ie[r] = a.inv[el[r]];
+    if constexpr (MODE == FM_RADD) s[r] = a.add[el[r]];
+  }
+  const int *__restrict__ off = a.t.tile_off;
+  const double *__restrict__ w = a.t.w;
+#pragma unroll 4
+  for (int q = 0; q < a.t.ntpl; ++q) {
+    const double *p = sv + base + off[q];
+    const double wq = (MODE == FM_APPLY || MODE == FM_T) ? w[q] : 1.0;
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+      const double x = p[r * PL];
+      if constexpr (MODE == FM_APPLY) s[r] = s[r] + (wq * ie[r]) * x;
+      else if constexpr (MODE == FM_T) s[r] = s[r] + (wq * si[base + off[q] + r * PL]) * x;
+      else s[r] = s[r] + x;
+    }
+  }
+#pragma unroll 1
+  for (int r = 0; r < RZ; ++r) {
+    if (z0 + r >= nz) break;
+    const int64_t e = gx + (int64_t)nx * (gy + (int64_t)ny * (z0 + r));
+    double v = r ? s[RZ - 1] : s[0];
+    if constexpr (MODE == FM_APPLY) {
+      if (a.copy) a.copy[e] = sv[base + (H * PY + H) * PX + H + r * PL];
+      if constexpr (EPI == FE_VOID) {  // as k_void_pre
+        if (v > 1.0) v = 1.0;
+        a.zt[e] = vecpow1(1.0 + -1 * v, a.sp.vd_penal);
+      }
+      a.out[e] = v;
+      if constexpr (EPI == FE_SIMP) {
+        a.so.y[e] = 1.0;
+        simp_one(e, v, 1.0, a.sp, a.so);
+      }
+    } else if constexpr (MODE == FM_RADD) {
+      v = v * a.scale;
+      const double y = v < 1.0 ? v : 1.0;
+      a.out[e] = y;
+      simp_one(e, a.rho[e], y, a.sp, a.so);
+    } else if constexpr (MODE == FM_RT) {
+      a.out[e] = chain_mid_one(a.src[e], a.y[e], a.rhoq[e], v);
+    } else {
+      a.out[e] = v;
+    }
+  }
 }
 
 // g_e = -dEdz_e * u_e^T (KE u_e), sequential sums without contraction (Compliance.cpp:37-43)
@@ -448,9 +569,53 @@ void filter_rowsum_inv(hipStream_t s, const FilterTemplate &t, double *inv)
   TOFE_LAUNCH_CHECK();
 }
 
+template <int MODE, int EPI>
+static bool filter_tile(hipStream_t s, const FilterArgs &a)
+{
+  const auto go = [&](auto hc) {
+    constexpr int H = decltype(hc)::value;
+    constexpr int TZ = 2 * filter_rz(H, MODE);
+    const dim3 grid((a.t.nx + FTX - 1) / FTX, (a.t.ny + FTY - 1) / FTY, (a.t.nz + TZ - 1) / TZ);
+    if (grid.y > 65535 || grid.z > 65535) return false;
+    k_filter_tile<H, MODE, EPI><<<grid, dim3(FNT), 0, s>>>(a);
+    TOFE_LAUNCH_CHECK();
+    return true;
+  };
+  switch (a.t.tile_h) {
+    case 1: return go(std::integral_constant<int, 1>());
+    case 2: return go(std::integral_constant<int, 2>());
+    case 3: return go(std::integral_constant<int, 3>());
+    case 4: return go(std::integral_constant<int, 4>());
+    case 5: return go(std::integral_constant<int, 5>());
+    default: return false;
+  }
+}
+
+// The tiled kernels serve every filter whose neighbours lie within kFilterTileMax elements
+// (LDS holds the staged box); the ones above walk larger neighbourhoods from global memory.
+int filter_tile_h(const int *off, int n)
+{
+  int h = 1;
+  for (int v = 0; v < 3 * n; ++v) h = std::max(h, std::abs(off[v]));
+  return h <= kFilterTileMax ? h : 0;
+}
+
+void filter_tile_offsets(const int *off, int n, int h, int *out)
+{
+  const int px = FTX + 2 * h, py = FTY + 2 * h;
+  for (int q = 0; q < n; ++q)
+    out[q] = ((off[3 * q + 2] + h) * py + off[3 * q + 1] + h) * px + off[3 * q] + h;
+}
+
 void filter_apply(hipStream_t s, const FilterTemplate &t, const double *inv, const double *x,
                   double *rho)
 {
+  FilterArgs a;
+  a.t = t;
+  a.src = x;
+  a.inv = inv;
+  a.out = rho;
+  if (filter_tile<FM_APPLY, FE_PLAIN>(s, a)) return;
   const int64_t ne = (int64_t)t.nx * t.ny * t.nz;
   k_filter_apply<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(t, inv, x, rho, ne);
   TOFE_LAUNCH_CHECK();
@@ -459,6 +624,12 @@ void filter_apply(hipStream_t s, const FilterTemplate &t, const double *inv, con
 void filter_apply_T(hipStream_t s, const FilterTemplate &t, const double *inv, const double *g,
                     double *gx)
 {
+  FilterArgs a;
+  a.t = t;
+  a.src = g;
+  a.inv = inv;
+  a.out = gx;
+  if (filter_tile<FM_T, FE_PLAIN>(s, a)) return;
   const int64_t ne = (int64_t)t.nx * t.ny * t.nz;
   k_filter_apply_T<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(t, inv, g, gx, ne);
   TOFE_LAUNCH_CHECK();
@@ -485,45 +656,77 @@ static unsigned stride_blocks(int64_t n)
   return nb > 4096 ? 4096 : (nb ? nb : 1);
 }
 
-void void_pre(hipStream_t s, double *rho, int64_t ne, double q, double *zt)
-{
-  k_void_pre<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(rho, ne, q, zt);
-  TOFE_LAUNCH_CHECK();
-}
-
-void rfilter_madd(hipStream_t s, const FilterTemplate &t, const double *REdge, const double *zt,
-                  double inv_vdmin, double *y)
+void design_fields(hipStream_t s, const FilterTemplate &t, const double *inv, const double *x,
+                   double *xcopy, double *rho, const SimpParams &sp, const SimpOut &so)
 {
   const int64_t ne = (int64_t)t.nx * t.ny * t.nz;
-  k_rfilter_madd<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(t, REdge, zt, inv_vdmin, y, ne);
+  FilterArgs a;
+  a.t = t;
+  a.src = x;
+  a.inv = inv;
+  a.out = rho;
+  a.copy = xcopy;
+  a.sp = sp;
+  a.so = so;
+  if (filter_tile<FM_APPLY, FE_SIMP>(s, a)) return;
+  if (xcopy) TOFE_HIP(hipMemcpyAsync(xcopy, x, ne * sizeof(double), hipMemcpyDeviceToDevice, s));
+  filter_apply(s, t, inv, x, rho);
+  k_simp<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(rho, nullptr, ne, sp, so);
   TOFE_LAUNCH_CHECK();
 }
 
-void rfilter_T(hipStream_t s, const FilterTemplate &t, const double *g, double *gx)
+void design_fields_void(hipStream_t s, const FilterTemplate &t, const FilterTemplate &tr,
+                        const double *inv, const double *REdge, const double *x, double *xcopy,
+                        double *rho, double *zt, const SimpParams &sp, const SimpOut &so)
 {
   const int64_t ne = (int64_t)t.nx * t.ny * t.nz;
-  k_rfilter_T<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(t, g, gx, ne);
+  FilterArgs a;
+  a.t = t;
+  a.src = x;
+  a.inv = inv;
+  a.out = rho;
+  a.copy = xcopy;
+  a.zt = zt;
+  a.sp = sp;
+  if (!filter_tile<FM_APPLY, FE_VOID>(s, a)) {
+    if (xcopy) TOFE_HIP(hipMemcpyAsync(xcopy, x, ne * sizeof(double), hipMemcpyDeviceToDevice, s));
+    filter_apply(s, t, inv, x, rho);
+    k_void_pre<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(rho, ne, sp.vd_penal, zt);
+    TOFE_LAUNCH_CHECK();
+  }
+  FilterArgs b;
+  b.t = tr;
+  b.src = zt;
+  b.add = REdge;
+  b.scale = 1 / sp.vd_min;
+  b.rho = rho;
+  b.out = so.y;
+  b.sp = sp;
+  b.so = so;
+  if (filter_tile<FM_RADD, FE_SIMP>(s, b)) return;
+  k_rfilter_madd<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(tr, REdge, zt, b.scale, so.y, ne);
+  TOFE_LAUNCH_CHECK();
+  k_simp<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(rho, so.y, ne, sp, so);
   TOFE_LAUNCH_CHECK();
 }
 
-void simp(hipStream_t s, const double *rho, const double *y, int64_t ne, const SimpParams &sp,
-          double *yout, double *rhoq, double *E, double *dEdz, double *Es, double *dEsdz, float *E32)
+void chain_void(hipStream_t s, const FilterTemplate &tr, const double *dfdE, const double *rho,
+                const double *y, const double *rhoq, double *out, double *t1, double *t2)
 {
-  k_simp<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(rho, y, ne, sp, yout, rhoq, E, dEdz, Es, dEsdz,
-                                                     E32);
+  const int64_t ne = (int64_t)tr.nx * tr.ny * tr.nz;
+  FilterArgs a;
+  a.t = tr;
+  a.src = dfdE;
+  a.rho = rho;
+  a.y = y;
+  a.rhoq = rhoq;
+  a.out = out;
+  if (filter_tile<FM_RT, FE_PLAIN>(s, a)) return;
+  k_mul<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(dfdE, rho, t1, ne);
   TOFE_LAUNCH_CHECK();
-}
-
-void chain_mid(hipStream_t s, const double *dfdE, const double *y, const double *rhoq,
-               const double *RtT, double *out, int64_t ne)
-{
-  k_chain_mid<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(dfdE, y, rhoq, RtT, out, ne);
+  k_rfilter_T<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(tr, t1, t2, ne);
   TOFE_LAUNCH_CHECK();
-}
-
-void mul(hipStream_t s, const double *a, const double *b, double *c, int64_t n)
-{
-  k_mul<<<dim3(stride_blocks(n)), dim3(NT), 0, s>>>(a, b, c, n);
+  k_chain_mid<<<dim3(stride_blocks(ne)), dim3(NT), 0, s>>>(dfdE, y, rhoq, t2, out, ne);
   TOFE_LAUNCH_CHECK();
 }
 

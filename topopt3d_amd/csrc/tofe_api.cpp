@@ -196,7 +196,8 @@ struct tofe_ctx {
   DBuf<float> dKE32;
   DBuf<uint8_t> dfix;
   bool has_fix = false;
-  DBuf<int> dtpl_off;
+  DBuf<int> dtpl_off, dtpl_tile, drtpl_tile;  // entries, and their offsets in a tile's box
+  int tile_h = 0, rtile_h = 0;                // box halo of the tiled filter kernels, 0: not used
   DBuf<double> dtpl_w, filt_inv;
   DBuf<double> x, rho, E, dEdz, Es, dEsdz;
   DBuf<float> E32;
@@ -328,6 +329,8 @@ FilterTemplate rfilter_tpl(const tofe_ctx *c)
   t.nx = c->desc.nx;
   t.ny = c->desc.ny;
   t.nz = c->desc.nz;
+  t.tile_off = c->drtpl_tile.p;
+  t.tile_h = c->rtile_h;
   return t;
 }
 
@@ -340,6 +343,8 @@ FilterTemplate filter_tpl(const tofe_ctx *c)
   t.nx = c->desc.nx;
   t.ny = c->desc.ny;
   t.nz = c->desc.nz;
+  t.tile_off = c->dtpl_tile.p;
+  t.tile_h = c->tile_h;
   return t;
 }
 
@@ -1503,17 +1508,13 @@ int guarded(tofe_ctx *c, const char *name, F &&f, bool settle_first = true)
 void upload_design(tofe_ctx *c, const double *dx)
 {
   const hipStream_t s = c->stream;
-  const FilterTemplate t = filter_tpl(c);
-  if (dx != c->x.p)
-    TOFE_HIP(hipMemcpyAsync(c->x.p, dx, c->ne * sizeof(double), hipMemcpyDeviceToDevice, s));
-  filter_apply(s, t, c->filt_inv.p, c->x.p, c->rho.p);
-  if (c->has_vd) {
-    // rho <- min(rho, 1); y = min(1, (REdge + R (1-rho)^q) / vdMin)
-    void_pre(s, c->rho.p, c->ne, c->sp.vd_penal, c->ebuf3.p);
-    rfilter_madd(s, rfilter_tpl(c), c->REdge.p, c->ebuf3.p, 1 / c->sp.vd_min, c->y.p);
-  }
-  simp(s, c->rho.p, c->has_vd ? c->y.p : nullptr, c->ne, c->sp, c->y.p, c->rhoq.p, c->E.p,
-       c->dEdz.p, c->Es.p, c->dEsdz.p, c->E32.p);
+  double *xcopy = dx != c->x.p ? c->x.p : nullptr;
+  const SimpOut so{c->y.p, c->rhoq.p, c->E.p, c->dEdz.p, c->Es.p, c->dEsdz.p, c->E32.p};
+  if (c->has_vd)
+    design_fields_void(s, filter_tpl(c), rfilter_tpl(c), c->filt_inv.p, c->REdge.p, dx, xcopy, c->rho.p,
+                       c->ebuf3.p, c->sp, so);
+  else
+    design_fields(s, filter_tpl(c), c->filt_inv.p, dx, xcopy, c->rho.p, c->sp, so);
   TOFE_HIP(hipStreamSynchronize(s));
   c->design_set = true;
   c->assembled = false;
@@ -1525,9 +1526,7 @@ void chain_dev(tofe_ctx *c, const double *g, double *out, double *t1, double *t2
 {
   const hipStream_t s = c->stream;
   if (c->has_vd) {
-    mul(s, g, c->rho.p, t1, c->ne);
-    rfilter_T(s, rfilter_tpl(c), t1, t2);
-    chain_mid(s, g, c->y.p, c->rhoq.p, t2, t1, c->ne);
+    chain_void(s, rfilter_tpl(c), g, c->rho.p, c->y.p, c->rhoq.p, t1, t1, t2);
     filter_apply_T(s, filter_tpl(c), c->filt_inv.p, t1, out);
   } else {
     filter_apply_T(s, filter_tpl(c), c->filt_inv.p, g, out);
@@ -1789,6 +1788,18 @@ void h2d(tofe_ctx *c, double *d, const double *h, size_t n)
 {
   TOFE_HIP(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
 }
+// offsets of a filter's entries in the tiled kernels' staged box; returns its halo (0: not used)
+int filter_tile_setup(tofe_ctx *c, const std::vector<int> &off, DBuf<int> &dev)
+{
+  const int n = (int)off.size() / 3, h = filter_tile_h(off.data(), n);
+  if (!h) return 0;
+  std::vector<int> t(n);
+  filter_tile_offsets(off.data(), n, h, t.data());
+  dev.alloc(n);
+  TOFE_HIP(hipMemcpyAsync(dev.p, t.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
+  TOFE_HIP(hipStreamSynchronize(c->stream));  // t is a local
+  return h;
+}
 void d2h(tofe_ctx *c, double *h, const double *d, size_t n)
 {
   TOFE_HIP(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1996,6 +2007,7 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
     TOFE_HIP(hipMemcpyAsync(c->dtpl_off.p, c->tpl_off.data(), c->tpl_off.size() * sizeof(int),
                             hipMemcpyHostToDevice, c->stream));
     h2d(c.get(), c->dtpl_w.p, c->tpl_w.data(), c->tpl_w.size());
+    c->tile_h = filter_tile_setup(c.get(), c->tpl_off, c->dtpl_tile);
     c->filt_inv.alloc(c->ne);
     filter_rowsum_inv(c->stream, filter_tpl(c.get()), c->filt_inv.p);
     c->y.alloc(c->ne);
@@ -2012,6 +2024,7 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       TOFE_HIP(hipMemcpyAsync(c->drtpl_off.p, c->rtpl_off.data(), c->rtpl_off.size() * sizeof(int),
                               hipMemcpyHostToDevice, c->stream));
       h2d(c.get(), c->drtpl_w.p, rw.data(), rw.size());
+      c->rtile_h = filter_tile_setup(c.get(), c->rtpl_off, c->drtpl_tile);
       DBuf<int64_t> cnt;
       cnt.alloc(c->ne);
       filter_count(c->stream, rfilter_tpl(c.get()), cnt.p);

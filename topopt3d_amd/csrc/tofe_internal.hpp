@@ -444,7 +444,15 @@ struct FilterTemplate {
   const double *w = nullptr;   // 1 - dist/R per entry
   int ntpl = 0;
   int nx = 0, ny = 0, nz = 0;
+  // tiled kernels (filter_tile_h > 0): the entries' offsets in a tile's staged box
+  const int *tile_off = nullptr;
+  int tile_h = 0;
 };
+constexpr int kFilterTileMax = 5;
+// Largest neighbour offset of a template if the tiled kernels serve it, else 0; and the n
+// offsets they use.
+int filter_tile_h(const int *off, int n);
+void filter_tile_offsets(const int *off, int n, int h, int *out);
 void filter_rowsum_inv(hipStream_t s, const FilterTemplate &t, double *inv);
 void filter_apply(hipStream_t s, const FilterTemplate &t, const double *inv, const double *x,
                   double *rho);
@@ -458,15 +466,24 @@ struct SimpParams {
   int interp = TOFE_INTERP_SIMP;
   double p0 = 0, p1 = 0;
 };
-void void_pre(hipStream_t s, double *rho, int64_t ne, double q, double *zt);
-void rfilter_madd(hipStream_t s, const FilterTemplate &t, const double *REdge, const double *zt,
-                  double inv_vdmin, double *y);
-void rfilter_T(hipStream_t s, const FilterTemplate &t, const double *g, double *gx);
-void simp(hipStream_t s, const double *rho, const double *y, int64_t ne, const SimpParams &sp,
-          double *yout, double *rhoq, double *E, double *dEdz, double *Es, double *dEsdz, float *E32);
-void chain_mid(hipStream_t s, const double *dfdE, const double *y, const double *rhoq,
-               const double *RtT, double *out, int64_t ne);
-void mul(hipStream_t s, const double *a, const double *b, double *c, int64_t n);
+// Fields of the material interpolation (E32 may be null)
+struct SimpOut {
+  double *y = nullptr, *rhoq = nullptr, *E = nullptr, *dEdz = nullptr, *Es = nullptr, *dEsdz = nullptr;
+  float *E32 = nullptr;
+};
+// MatIntFnc of the plain density filter: rho = P x and the interpolation with y = 1.  xcopy (may
+// be null) receives x.
+void design_fields(hipStream_t s, const FilterTemplate &t, const double *inv, const double *x,
+                   double *xcopy, double *rho, const SimpParams &sp, const SimpOut &so);
+// ... and with a maximum length scale: rho = min(P x, 1), z = (1 - rho)^q in zt, y =
+// min(1, (REdge + R z) / vdMin), then the interpolation.
+void design_fields_void(hipStream_t s, const FilterTemplate &t, const FilterTemplate &tr,
+                        const double *inv, const double *REdge, const double *x, double *xcopy,
+                        double *rho, double *zt, const SimpParams &sp, const SimpOut &so);
+// Middle of the chain rule with a maximum length scale: out = dfdE .* y - rhoq .* (y < 1) .*
+// R^T(dfdE .* rho); t1 and t2 are scratch, and out may be t1 but not dfdE.
+void chain_void(hipStream_t s, const FilterTemplate &tr, const double *dfdE, const double *rho,
+                const double *y, const double *rhoq, double *out, double *t1, double *t2);
 // Element geometry for the stress stiffness: D (6x6), dN_n/dx_a at the Gauss points, det J.
 struct ShapeData {
   double D[36];
