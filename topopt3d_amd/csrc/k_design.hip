@@ -266,9 +266,14 @@ __global__ void k_mul(const double *__restrict__ a, const double *__restrict__ b
 // transpose, which scales by the source's row sum) and its separately rounded operations, in
 // place of three LDS reads, three bounds checks and a gather.  The transpose visits the rows
 // e - off in ascending order; the neighbour list is symmetric with equal weights, so that is
-// the same walk.  Bound: the LDS reads, 8 bytes a term; the 32-wide rows are read without bank
-// conflicts, and z is the axis of the RZ outputs because their offsets are then immediates.
-// H is a template argument for the same reason.
+// the same walk.  Bound: the LDS reads, 8 bytes a term, and the staging loads ahead of them; the
+// 32-wide rows are read without bank conflicts, and z is the axis of the RZ outputs because their
+// offsets are then immediates (H is a template argument for the same reason).  Measured on
+// 144x72x72 elements, us, untiled -> here: R of radius 4.5 (389 entries) with the interpolation 260
+// -> 56, R^T with the chain rule's middle 256 -> 56, P of radius 3.5 (179) 134 -> 34, P^T 160 ->
+// 57; 192x96x96, radius 1.5 (19): P with the interpolation 57 -> 33 (its 149 MB of fields at 4.5
+// TB/s), P^T 45 -> 16.  Reading rows of entries as 16-byte pairs for two outputs measured the same
+// (R^T 54, P 39, P^T 63), as did four planes per thread.
 constexpr int FTX = 32, FTY = 8, FNT = 512;
 enum FiltMode : int { FM_APPLY = 0, FM_T = 1, FM_RADD = 2, FM_RT = 3 };
 // FE_PLAIN: out; FE_SIMP: rho (or y) and the interpolation; FE_VOID: rho and z = (1 - rho)^q
@@ -301,15 +306,33 @@ __global__ __launch_bounds__(FNT) void k_filter_tile(FilterArgs a)
   __shared__ double si[MODE == FM_T ? PL * PZ : 1];
   const int nx = a.t.nx, ny = a.t.ny, nz = a.t.nz;
   const int bx = blockIdx.x * FTX, by = blockIdx.y * FTY, bz = blockIdx.z * (2 * RZ);
-  for (int v = threadIdx.x; v < PL * PZ; v += FNT) {
+  // every load of the box is issued before the first value is used, without a branch (an element
+  // outside the mesh reads element 0): waiting for them one by one cost R^T 6 of 64 us
+  constexpr int NL = (PL * PZ + FNT - 1) / FNT;
+  static_assert(NL <= 32, "one bit per staged element of a thread");
+  double xv[NL], xi[MODE == FM_T || MODE == FM_RT ? NL : 1];
+  unsigned inside = 0;
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    const int v = (int)threadIdx.x + k * FNT;
     const int lz = v / PL, r = v - lz * PL, ly = r / PX, lx = r - ly * PX;
     const int gx = bx - H + lx, gy = by - H + ly, gz = bz - H + lz;
-    const bool in = gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz;
-    const int64_t n = in ? gx + (int64_t)nx * (gy + (int64_t)ny * gz) : 0;
-    double x = in ? a.src[n] : 0.0;
-    if constexpr (MODE == FM_RT) x = in ? x * a.rho[n] : 0.0;
-    sv[v] = x;
-    if constexpr (MODE == FM_T) si[v] = in ? a.inv[n] : 0.0;
+    const bool in = gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz && v < PL * PZ;
+    const int n = in ? gx + nx * (gy + ny * gz) : 0;
+    inside |= (in ? 1u : 0u) << k;
+    xv[k] = a.src[n];
+    if constexpr (MODE == FM_T) xi[k] = a.inv[n];
+    if constexpr (MODE == FM_RT) xi[k] = a.rho[n];
+  }
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    const int v = (int)threadIdx.x + k * FNT;
+    const bool in = (inside >> k) & 1u;
+    if constexpr (MODE == FM_RT) xv[k] = xv[k] * xi[k];
+    if (v < PL * PZ) {
+      sv[v] = in ? xv[k] : 0.0;
+      if constexpr (MODE == FM_T) si[v] = in ? xi[k] : 0.0;
+    }
   }
   __syncthreads();
   const int tx = threadIdx.x % FTX, ty = (threadIdx.x / FTX) % FTY, tz = threadIdx.x / (FTX * FTY);
@@ -328,7 +351,7 @@ __global__ __launch_bounds__(FNT) void k_filter_tile(FilterArgs a)
   }
   const int *__restrict__ off = a.t.tile_off;
   const double *__restrict__ w = a.t.w;
-#pragma unroll 4
+#pragma unroll 8
   for (int q = 0; q < a.t.ntpl; ++q) {
     const double *p = sv + base + off[q];
     const double wq = (MODE == FM_APPLY || MODE == FM_T) ? w[q] : 1.0;
