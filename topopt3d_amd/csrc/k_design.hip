@@ -472,71 +472,6 @@ __device__ inline double mass_q(int a, int b)
   return same == 3 ? 8.0 / 9.0 : same == 2 ? 4.0 / 9.0 : same == 1 ? 2.0 / 9.0 : 1.0 / 9.0;
 }
 
-// y = M x with the consistent mass M = sum_e V_e m0 Q (x) I_3, plus mlump on the diagonal,
-// and the Dirichlet rows and columns of MatZeroRowsColumns(M, fixed, 1e-8): one thread per
-// node gathers its eight elements; V vectors per thread (block row blockIdx.y holds vectors
-// V * blockIdx.y ...).
-template <int V>
-__global__ __launch_bounds__(NT) void k_apply_mc(const double *__restrict__ Ve, double m0,
-                                                 const double *__restrict__ mlump,
-                                                 const uint8_t *__restrict__ fix, int nx, int ny,
-                                                 int nz, const double *__restrict__ x, double *y,
-                                                 int nvec)
-{
-  const int Nx = nx + 1, Ny = ny + 1, Nz = nz + 1;
-  const int64_t nn = (int64_t)Nx * Ny * Nz;
-  const int v0 = blockIdx.y * V, nv = min(V, nvec - v0);
-  x += (int64_t)v0 * 3 * nn;
-  y += (int64_t)v0 * 3 * nn;
-  const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (n >= nn) return;
-  int i, j, k;
-  node_ijk(n, Nx, Ny, i, j, k);
-  double acc[V][3];
-#pragma unroll
-  for (int v = 0; v < V; ++v) acc[v][0] = acc[v][1] = acc[v][2] = 0.0;
-  for (int dz = -1; dz <= 0; ++dz)
-    for (int dy = -1; dy <= 0; ++dy)
-      for (int dx = -1; dx <= 0; ++dx) {
-        const int ex = i + dx, ey = j + dy, ez = k + dz;
-        if (ex < 0 || ex >= nx || ey < 0 || ey >= ny || ez < 0 || ez >= nz) continue;
-        const int kl = lidx(-dx, -dy, -dz);
-        double t[V][3];
-#pragma unroll
-        for (int v = 0; v < V; ++v) t[v][0] = t[v][1] = t[v][2] = 0.0;
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          const int64_t nm = (ex + lnx(m)) + (int64_t)Nx * ((ey + lny(m)) + (int64_t)Ny * (ez + lnz(m)));
-          const double w = mass_q(kl, m);
-          const uint8_t fm = fix ? fix[nm] : 0;
-#pragma unroll
-          for (int v = 0; v < V; ++v) {
-            if (v >= nv) break;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              const double xv = ((fm >> c) & 1) ? 0.0 : x[v * 3 * nn + 3 * nm + c];
-              t[v][c] += w * xv;
-            }
-          }
-        }
-        const double se = Ve[ex + (int64_t)nx * (ey + (int64_t)ny * ez)] * m0;
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) acc[v][c] += se * t[v][c];
-      }
-  const uint8_t fn = fix ? fix[n] : 0;
-#pragma unroll
-  for (int v = 0; v < V; ++v) {
-    if (v >= nv) break;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const int64_t d = v * 3 * nn + 3 * n + c;
-      y[d] = ((fn >> c) & 1) ? 1e-8 * x[d] : acc[v][c] + (mlump ? mlump[3 * n + c] * x[d] : 0.0);
-    }
-  }
-}
-
 __global__ __launch_bounds__(NT) void k_elem_quad(const double *__restrict__ phi,
                                                   const double *__restrict__ KE, int nx, int ny,
                                                   int nz, int64_t ndof, int nvec, double *kq,
@@ -766,19 +701,6 @@ void mass_diag(hipStream_t s, const double *V, int nx, int ny, int nz, double m0
 {
   const int64_t nn = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
   k_mass_diag<<<dim3(blocks_for(nn)), dim3(NT), 0, s>>>(V, nx, ny, nz, m0, mlump, fix, M);
-  TOFE_LAUNCH_CHECK();
-}
-
-void apply_mass_consistent(hipStream_t s, const double *V, double m0, const double *mlump,
-                           const uint8_t *fix, int nx, int ny, int nz, const double *x, double *y,
-                           int nvec)
-{
-  const int64_t nn = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-  if (nvec == 1)
-    k_apply_mc<1><<<dim3(blocks_for(nn)), dim3(NT), 0, s>>>(V, m0, mlump, fix, nx, ny, nz, x, y, 1);
-  else
-    k_apply_mc<4><<<dim3(blocks_for(nn), (nvec + 3) / 4), dim3(NT), 0, s>>>(V, m0, mlump, fix, nx,
-                                                                           ny, nz, x, y, nvec);
   TOFE_LAUNCH_CHECK();
 }
 

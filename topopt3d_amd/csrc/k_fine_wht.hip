@@ -14,6 +14,15 @@
 // layer are its own, its right neighbour's (lane + 1 in the same row of 16 lanes: DPP) and
 // the two of the row above, whose partial sums come through LDS.  Node planes of u are
 // staged in a ring of three LDS planes, loaded into registers one step ahead.
+//
+// The consistent mass (Dynamic.cpp:181-236's element mass as an exact integral) and the stress
+// stiffness (Buckling.cpp:283-414) are sums of element matrices A_e (x) I_3 and take the same march
+// with another middle: in the Walsh-Hadamard basis the mass is diagonal (four distinct values)
+// and the stress matrix, whose rows sum to zero, is a symmetric 7 x 7 block, 28 stored values.
+// A node-centric kernel gathering eight elements of eight nodes each took 1,783 us for M on 16
+// vectors of the 160x80x80 mesh (380 us here) and 812 us for Ks on 10 vectors of 128x64x64 (64
+// values per element read by every group of four vectors; 340 us here, bound by the stress matrices'
+// 117 MB per vector at two wavefronts per SIMD).
 #include "k_common.hpp"
 #include "ke_wht.hpp"
 
@@ -69,6 +78,10 @@ __device__ inline T wplane_load(__amdgpu_buffer_rsrc_t r, unsigned off)
   else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
 
+// what the march applies to an element's values: KE of a box, KE of a cube, the consistent mass,
+// or the element's stress matrix
+enum ElemForm : int { EF_BOX = 0, EF_CUBE = 1, EF_MASS = 2, EF_STRESS = 3 };
+
 // stored value of block entry B_t[i][j] (cubic elements: its group value)
 template <bool CUBE>
 constexpr int wht_slot(int t, int i, int j)
@@ -103,11 +116,48 @@ __device__ inline void element_product(T (&v)[3][8], const T (&kb)[NV], T Ee)
   wht8(v[2]);
 }
 
-// One block of the operator: block `bx` of the launch's `nblocks` (per vector).
-template <typename T, int EPI, bool CUBE>
+// y = Ee m0 (Q (x) I_3) u, in place: Q = 24 (x) [[1/3, 1/6], [1/6, 1/3]] per axis, whose eigenvalues
+// on sums and differences are 1/2 and 1/6.
+template <typename T>
+__device__ inline void mass_product(T (&v)[3][8], T Ee)
+{
+  const T f[4] = {Ee * (T)(3.0 / 8), Ee * (T)(1.0 / 8), Ee * (T)(1.0 / 24), Ee * (T)(1.0 / 72)};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    wht8(v[c]);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) v[c][m] *= f[(m & 1) + ((m >> 1) & 1) + (m >> 2)];
+    wht8(v[c]);
+  }
+}
+
+// y = Ee (H (x) I_3) u, in place, from the 28 values of the stress matrix in this basis.
+template <typename T>
+__device__ inline void stress_product(T (&v)[3][8], const T (&h)[kStressVals], T Ee)
+{
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    wht8(v[c]);
+    T x[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) x[m] = v[c][m];
+    v[c][0] = 0;
+#pragma unroll
+    for (int r = 1; r < 8; ++r) {
+      T acc = 0;
+#pragma unroll
+      for (int m = 1; m < 8; ++m) acc += h[stress_index(r, m)] * x[m];
+      v[c][r] = Ee * acc;
+    }
+    wht8(v[c]);
+  }
+}
+
+// One block of the operator: tile `bid` of the launch's `nblocks` (per vector), vector `vec`.
+template <typename T, int EPI, int FORM>
 __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0, EpiArgs<T> ep,
                                                int tiles_x, int tiles_y, int nblocks, int zlen,
-                                               int blk)
+                                               int bid, int vec)
 {
   // partial sums handed to the row below (lower, upper node): double-buffered in FP32; one
   // buffer and a second barrier per step in FP64, which keeps the block at 33 KB of LDS (four
@@ -119,9 +169,8 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
 
   const int nx = op.nx, ny = op.ny, nz = op.nz;
   const int Nx = nx + 1, Ny = ny + 1, Nz = nz + 1;
-  epi_select_vector(ep, u0, 3 * (int64_t)Nx * Ny * Nz, nblocks);  // vector blockIdx.y
-  const T *__restrict__ u = u0;
-  const int bid = xcd_remap(blk, nblocks);
+  epi_offset(ep, vec, 3 * (int64_t)Nx * Ny * Nz, nblocks);
+  const T *__restrict__ u = u0 + vec * (3 * (int64_t)Nx * Ny * Nz);
   const int txy = tiles_x * tiles_y;
   const int bz = bid / txy;
   const int rem = bid - bz * txy;
@@ -139,10 +188,14 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
   const uint8_t *__restrict__ fix = op.fix;
   const int NxNy = Nx * Ny, nxny = nx * ny;
 
-  constexpr int NV = CUBE ? kWhtCubeVals : kWhtVals;
+  constexpr bool CUBE = FORM == EF_CUBE, KEFORM = FORM == EF_BOX || FORM == EF_CUBE;
+  constexpr int NV = !KEFORM ? 1 : CUBE ? kWhtCubeVals : kWhtVals;
   T kb[NV];
+  if constexpr (KEFORM) {
 #pragma unroll
-  for (int k = 0; k < NV; ++k) kb[k] = op.KE[(CUBE ? kWhtCubeOffset : kWhtOffset) + k];
+    for (int k = 0; k < NV; ++k) kb[k] = op.KE[(CUBE ? kWhtCubeOffset : kWhtOffset) + k];
+  }
+  const int64_t ne = (int64_t)nxny * nz;
 
   // staging map: node slot q of this thread is node t + q * NW of the staged window
   // (x0 - 1 .. x0 + 15) x (y0 - 1 .. y0 + 15), its in-plane index or kNone
@@ -184,7 +237,22 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
     }
   };
   auto load_E = [&](int ez) -> T {
-    return (ez >= 0 && ez < nz && eidx != kNone) ? E[eidx + (int64_t)nxny * ez] : T(0);
+    if (!(ez >= 0 && ez < nz && eidx != kNone)) return T(0);
+    const T e = E[eidx + (int64_t)nxny * ez];
+    return KEFORM ? e : op.escale * e;
+  };
+
+  // stress matrix of this thread's element of layer ez (zero outside the mesh)
+  constexpr int NH = FORM == EF_STRESS ? kStressVals : 1;
+  T h[NH];
+  auto load_H = [&](T (&hv)[NH], int ez) {
+#pragma unroll
+    for (int k = 0; k < NH; ++k) hv[k] = 0;
+    if (ez >= 0 && ez < nz && eidx != kNone) {
+      const T *__restrict__ H = op.H + (eidx + (int64_t)nxny * ez);
+#pragma unroll
+      for (int k = 0; k < NH; ++k) hv[k] = H[k * ne];
+    }
   };
 
   T alo[3], ahi[3];
@@ -201,6 +269,7 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
     load_u(pu, pf, k0);
     store_u(pu, pf, 1);
     Ecur = load_E(k0 - 1);
+    if constexpr (FORM == EF_STRESS) load_H(h, k0 - 1);
   }
   __syncthreads();
   // Step st (element layer ez = k0 - 1 + st) reads node planes ez and ez + 1 from ring slots
@@ -224,6 +293,8 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
     const int64_t n = i + (int64_t)Nx * (j + (int64_t)Ny * ez);
     EpiIn<T, EPI> ein;
     if (emit) epi_load<T, EPI>(ep, u, fix, n, ein);
+    T hn[NH];
+    if constexpr (FORM == EF_STRESS) load_H(hn, more ? ez + 1 : -1);
     T v[3][8];
 #pragma unroll
     for (int l = 0; l < 8; ++l) {
@@ -231,7 +302,9 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
 #pragma unroll
       for (int c = 0; c < 3; ++c) v[c][mof(l)] = su[lnz(l) ? shi : slo][c][nl];
     }
-    element_product<T, CUBE, NV>(v, kb, Ecur);
+    if constexpr (FORM == EF_MASS) mass_product<T>(v, Ecur);
+    else if constexpr (FORM == EF_STRESS) stress_product<T>(v, h, Ecur);
+    else element_product<T, CUBE, NV>(v, kb, Ecur);
     // node (i, j): own element's corner (1, 1) [m = 3 lower, 7 upper] + right element's
     // corner (0, 1) [m = 2, 6]; the row above contributes corners (1, 0) and (0, 0)
     // [m = 1, 5 and 0, 4] of its two elements, summed there and passed through LDS
@@ -253,44 +326,58 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
       ahi[c] = phi[c] + sp[pb][3 + c][tb];
     }
     if (emit) {
-      if (op.spk) {  // spring supports: K + diag(spk) on free DOFs (fixed rows return u below)
+      if (op.spk) {  // spring supports (point masses): + diag(spk) on free DOFs
 #pragma unroll
         for (int c = 0; c < 3; ++c) alo[c] += op.spk[3 * n + c] * ein.u[c];
       }
-      epi_store<T, EPI>(ep, n, ein, alo, dsum, dsum2);
+      if constexpr (KEFORM) {
+        epi_store<T, EPI>(ep, n, ein, alo, dsum, dsum2);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          ep.y[3 * n + c] = ((ein.fm >> c) & 1) ? op.fixval * ein.u[c] : alo[c];
+      }
     }
     Ecur = Enext;
+    if constexpr (FORM == EF_STRESS) {
+#pragma unroll
+      for (int k = 0; k < NH; ++k) h[k] = hn[k];
+    }
   }
   if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2 || EPI == EPI_CHEB_OUT) {
     __syncthreads();
     const double s1 = block_sum<NW>(dsum, sred);
-    if (t == 0) ep.partial[blk] = s1;
+    if (t == 0) ep.partial[bid] = s1;
     if constexpr (EPI == EPI_APPLY_DOT2) {
       __syncthreads();
       const double s2 = block_sum<NW>(dsum2, sred);
-      if (t == 0) ep.partial2[blk] = s2;
+      if (t == 0) ep.partial2[bid] = s2;
     }
   }
 }
 
-template <typename T, int EPI, bool CUBE>
+// Vectors are the launch's second axis.  (Blocks of a tile's vectors next to one another on one XCD,
+// so that E and D^-1 or the stress matrices come from its L2, measured slower: a Chebyshev step on
+// 16 vectors of the 160x80x80 mesh 702 against 670 us, Ks on 10 of 128x64x64 363 against 340 us.)
+template <typename T, int EPI, int FORM>
 __global__ __launch_bounds__(NW) void k_fine_wht(FineOp<T> op, const T *u0, EpiArgs<T> ep,
                                                  int tiles_x, int tiles_y, int nblocks, int zlen)
 {
-  fine_wht_block<T, EPI, CUBE>(op, u0, ep, tiles_x, tiles_y, nblocks, zlen, blockIdx.x);
+  fine_wht_block<T, EPI, FORM>(op, u0, ep, tiles_x, tiles_y, nblocks, zlen,
+                               xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
 }
 
 // The operator of several instances in one grid: entry e of the table owns blocks
 // [b0[e], b0[e + 1]).  (Cubic and general elements take separate launches: one kernel holding
 // both bodies would hold both bodies' LDS arrays.)
-template <typename T, int EPI, bool CUBE>
+template <typename T, int EPI, int FORM>
 __global__ __launch_bounds__(NW) void k_fine_wht_batch(const FineLaunch<T> *__restrict__ tab,
                                                        const int *__restrict__ b0, int n)
 {
   const int e = batch_entry(b0, n, blockIdx.x);
   const FineLaunch<T> L = tab[e];
-  fine_wht_block<T, EPI, CUBE>(L.op, L.u, L.ep, L.tiles_x, L.tiles_y, L.nblocks, L.zlen,
-                               blockIdx.x - b0[e]);
+  fine_wht_block<T, EPI, FORM>(L.op, L.u, L.ep, L.tiles_x, L.tiles_y, L.nblocks, L.zlen,
+                               xcd_remap(blockIdx.x - b0[e], L.nblocks), blockIdx.y);
 }
 
 struct WhtGrid {
@@ -343,27 +430,42 @@ int fine_wht_blocks(const FineOp<T> &op)
   return wht_grid(op).nblocks;
 }
 
-template <typename T, int EPI>
-void launch_wht(hipStream_t s, const FineOp<T> &op, const T *u, const EpiArgs<T> &ep, const WhtGrid &g)
+template <typename T, int EPI, int FORM>
+void launch_form(hipStream_t s, const FineOp<T> &op, const T *u, const EpiArgs<T> &ep)
 {
-  dim3 grid(g.nblocks, ep.nvec), block(NW);
-  if (op.wht_cube)
-    k_fine_wht<T, EPI, true><<<grid, block, 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y, g.nblocks, op.zlen);
-  else
-    k_fine_wht<T, EPI, false><<<grid, block, 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y, g.nblocks, op.zlen);
+  const WhtGrid g = wht_grid(op);
+  k_fine_wht<T, EPI, FORM><<<dim3(g.nblocks, ep.nvec), dim3(NW), 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y,
+                                                                        g.nblocks, op.zlen);
+}
+template <typename T, int EPI>
+void launch_wht(hipStream_t s, const FineOp<T> &op, const T *u, const EpiArgs<T> &ep)
+{
+  if (op.wht_cube) launch_form<T, EPI, EF_CUBE>(s, op, u, ep);
+  else launch_form<T, EPI, EF_BOX>(s, op, u, ep);
+}
+
+void fine_mass(hipStream_t s, const FineOp<double> &op, const double *u, const EpiArgs<double> &ep)
+{
+  launch_form<double, EPI_APPLY, EF_MASS>(s, op, u, ep);
+  TOFE_LAUNCH_CHECK();
+}
+
+void fine_stress(hipStream_t s, const FineOp<double> &op, const double *u, const EpiArgs<double> &ep)
+{
+  launch_form<double, EPI_APPLY, EF_STRESS>(s, op, u, ep);
+  TOFE_LAUNCH_CHECK();
 }
 
 template <typename T>
 void fine_wht(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep)
 {
-  const WhtGrid g = wht_grid(op);
   switch (epi) {
-    case EPI_APPLY: launch_wht<T, EPI_APPLY>(s, op, u, ep, g); break;
-    case EPI_APPLY_DOT: launch_wht<T, EPI_APPLY_DOT>(s, op, u, ep, g); break;
-    case EPI_APPLY_DOT2: launch_wht<T, EPI_APPLY_DOT2>(s, op, u, ep, g); break;
-    case EPI_RESID: launch_wht<T, EPI_RESID>(s, op, u, ep, g); break;
-    case EPI_CHEB: launch_wht<T, EPI_CHEB>(s, op, u, ep, g); break;
-    case EPI_CHEB_OUT: launch_wht<T, EPI_CHEB_OUT>(s, op, u, ep, g); break;
+    case EPI_APPLY: launch_wht<T, EPI_APPLY>(s, op, u, ep); break;
+    case EPI_APPLY_DOT: launch_wht<T, EPI_APPLY_DOT>(s, op, u, ep); break;
+    case EPI_APPLY_DOT2: launch_wht<T, EPI_APPLY_DOT2>(s, op, u, ep); break;
+    case EPI_RESID: launch_wht<T, EPI_RESID>(s, op, u, ep); break;
+    case EPI_CHEB: launch_wht<T, EPI_CHEB>(s, op, u, ep); break;
+    case EPI_CHEB_OUT: launch_wht<T, EPI_CHEB_OUT>(s, op, u, ep); break;
   }
   TOFE_LAUNCH_CHECK();
 }
@@ -382,8 +484,8 @@ void launch_wht_batch(hipStream_t s, bool cube, const FineLaunch<T> *tab, const 
                       int nblocks_total, int nvec)
 {
   dim3 grid(nblocks_total, nvec), block(NW);
-  if (cube) k_fine_wht_batch<T, EPI, true><<<grid, block, 0, s>>>(tab, b0, n);
-  else k_fine_wht_batch<T, EPI, false><<<grid, block, 0, s>>>(tab, b0, n);
+  if (cube) k_fine_wht_batch<T, EPI, EF_CUBE><<<grid, block, 0, s>>>(tab, b0, n);
+  else k_fine_wht_batch<T, EPI, EF_BOX><<<grid, block, 0, s>>>(tab, b0, n);
 }
 
 template <typename T>

@@ -5,11 +5,13 @@
 // ks_e(u) = sum_q W G_q^T S(D B_q u_e) G_q detJ is block diagonal over the three
 // displacement components with the scalar 8x8 matrix
 //   H_e[k][m] = sum_q W detJ grad N_k(q)^T s_q grad N_m(q),   s_q = stress tensor of D B_q u_e,
-// so a state is stored as H_e (64 values per element, [(k*8+m)*nelem + e]) and
-// Ks = sum_e (-Es_e) H_e (x) I_3 is applied node by node.  The adjoint right-hand side uses
+// stored in the Walsh-Hadamard basis of the node coordinates, where the rows that sum to zero
+// leave a symmetric 7x7 block: 28 values per element, [stress_index(s, t) * nelem + e].
+// Ks = sum_e (-Es_e) H_e (x) I_3 is applied by fine_stress.  The adjoint right-hand side uses
 // phi^T ks(e_d) phi = (D B_q e_d) . tau_q summed over q, with tau the Voigt vector of
 // T = sum_i grad phi_i grad phi_i^T (shear entries doubled).
 #include "k_common.hpp"
+#include "ke_wht.hpp"
 
 namespace tofe {
 namespace {
@@ -27,7 +29,27 @@ __device__ inline void element_nodes(int64_t e, int nx, int ny, int64_t (&node)[
     node[l] = (ex + lnx(l)) + (int64_t)Nx * ((ey + lny(l)) + (int64_t)Ny * (ez + lnz(l)));
 }
 
-// H_e of the displacement state U (fixed DOFs taken as given: U is a solution, zero there).
+// coordinate index x + 2y + 4z of element-local node l
+constexpr int node_index(int l) { return lnx(l) + 2 * lny(l) + 4 * lnz(l); }
+
+// unnormalised 8-point Walsh-Hadamard transform of the values at coordinate indices 0..7
+__device__ inline void wht8(double (&v)[8])
+{
+#pragma unroll
+  for (int b = 1; b < 8; b <<= 1)
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+      if (!(m & b)) {
+        const double a = v[m], c = v[m | b];
+        v[m] = a + c;
+        v[m | b] = a - c;
+      }
+}
+
+// H_e of the displacement state U (fixed DOFs taken as given: U is a solution, zero there).  In
+// the Walsh-Hadamard basis the shape gradient of index s has a component along axis a only if s
+// has that bit, so the gradients and the 28 products take about half the terms of the nodal form,
+// and the 28 values are what is written (128x64x64: 80 -> 40 us).
 __global__ __launch_bounds__(NT) void k_stress_h(const double *__restrict__ U, int nx, int ny,
                                                  int nz, ShapeData sd, double *H)
 {
@@ -36,14 +58,16 @@ __global__ __launch_bounds__(NT) void k_stress_h(const double *__restrict__ U, i
   if (e >= ne) return;
   int64_t node[8];
   element_nodes(e, nx, ny, node);
-  double u[8][3];
+  double u[3][8];
 #pragma unroll
   for (int l = 0; l < 8; ++l)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) u[l][c] = U[3 * node[l] + c];
-  double h[36];  // upper triangle k <= m, packed row by row
+    for (int c = 0; c < 3; ++c) u[c][node_index(l)] = U[3 * node[l] + c];
 #pragma unroll
-  for (int v = 0; v < 36; ++v) h[v] = 0.0;
+  for (int c = 0; c < 3; ++c) wht8(u[c]);
+  double h[kStressVals];
+#pragma unroll
+  for (int v = 0; v < kStressVals; ++v) h[v] = 0.0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     // displacement gradient g[c][a] = du_c/dx_a
@@ -54,7 +78,8 @@ __global__ __launch_bounds__(NT) void k_stress_h(const double *__restrict__ U, i
       for (int a = 0; a < 3; ++a) {
         double t = 0.0;
 #pragma unroll
-        for (int l = 0; l < 8; ++l) t += sd.dN[q][a][l] * u[l][c];
+        for (int s = 1; s < 8; ++s)
+          if ((s >> a) & 1) t += sd.dNh[q][a][s] * u[c][s];
         g[c][a] = t;
       }
     const double eps[6] = {g[0][0], g[1][1], g[2][2], g[0][1] + g[1][0], g[1][2] + g[2][1],
@@ -67,92 +92,26 @@ __global__ __launch_bounds__(NT) void k_stress_h(const double *__restrict__ U, i
       for (int b = 0; b < 6; ++b) t += sd.D[a * 6 + b] * eps[b];
       sig[a] = t * sd.detJ[q];  // unit Gauss weight
     }
-    const double s[3][3] = {{sig[0], sig[3], sig[5]}, {sig[3], sig[1], sig[4]}, {sig[5], sig[4], sig[2]}};
+    const double s3[3][3] = {{sig[0], sig[3], sig[5]}, {sig[3], sig[1], sig[4]}, {sig[5], sig[4], sig[2]}};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int s = 1; s < 8; ++s) {
       double t[3];
 #pragma unroll
-      for (int a = 0; a < 3; ++a)
-        t[a] = s[a][0] * sd.dN[q][0][k] + s[a][1] * sd.dN[q][1][k] + s[a][2] * sd.dN[q][2][k];
+      for (int a = 0; a < 3; ++a) {
+        t[a] = 0.0;
 #pragma unroll
-      for (int m = k; m < 8; ++m)
-        h[k * 8 - k * (k - 1) / 2 + (m - k)] +=
-            t[0] * sd.dN[q][0][m] + t[1] * sd.dN[q][1][m] + t[2] * sd.dN[q][2][m];
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k)
-#pragma unroll
-    for (int m = k; m < 8; ++m) {
-      const double v = h[k * 8 - k * (k - 1) / 2 + (m - k)];
-      H[(int64_t)(k * 8 + m) * ne + e] = v;
-      H[(int64_t)(m * 8 + k) * ne + e] = v;
-    }
-}
-
-// y = Ks x with Ks = sum_e (-Es_e) H_e (x) I_3 and the Dirichlet rows and columns of
-// MatZeroRowsColumns(Ks, fixed, 0.0) (Buckling.cpp:28-29): fixed x entries are ignored
-// and fixed rows return 0.  One thread per node; elements in ascending order.
-// V vectors per thread (block row blockIdx.y holds vectors V*blockIdx.y ...), so each H value
-// read serves all of them; every vector's sums run in the same order as for one vector.
-template <int V>
-__global__ __launch_bounds__(NT) void k_apply_ks(const double *__restrict__ H,
-                                                 const double *__restrict__ Es,
-                                                 const uint8_t *__restrict__ fix, int nx, int ny,
-                                                 int nz, const double *__restrict__ x, double *y,
-                                                 int nvec)
-{
-  const int Nx = nx + 1, Ny = ny + 1, Nz = nz + 1;
-  const int64_t nn = (int64_t)Nx * Ny * Nz, ne = (int64_t)nx * ny * nz;
-  const int v0 = blockIdx.y * V, nv = min(V, nvec - v0);
-  x += (int64_t)v0 * 3 * nn;
-  y += (int64_t)v0 * 3 * nn;
-  const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (n >= nn) return;
-  int i, j, k;
-  node_ijk(n, Nx, Ny, i, j, k);
-  double acc[V][3];
-#pragma unroll
-  for (int v = 0; v < V; ++v) acc[v][0] = acc[v][1] = acc[v][2] = 0.0;
-  for (int dz = -1; dz <= 0; ++dz)
-    for (int dy = -1; dy <= 0; ++dy)
-      for (int dx = -1; dx <= 0; ++dx) {
-        const int ex = i + dx, ey = j + dy, ez = k + dz;
-        if (ex < 0 || ex >= nx || ey < 0 || ey >= ny || ez < 0 || ez >= nz) continue;
-        const int64_t e = ex + (int64_t)nx * (ey + (int64_t)ny * ez);
-        const int kl = lidx(-dx, -dy, -dz);
-        int64_t node[8];
-        element_nodes(e, nx, ny, node);
-        double t[V][3];
-#pragma unroll
-        for (int v = 0; v < V; ++v) t[v][0] = t[v][1] = t[v][2] = 0.0;
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          const double hkm = H[(int64_t)(kl * 8 + m) * ne + e];
-          const uint8_t fm = fix ? fix[node[m]] : 0;
-#pragma unroll
-          for (int v = 0; v < V; ++v) {
-            if (v >= nv) break;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              const double xv = ((fm >> c) & 1) ? 0.0 : x[v * 3 * nn + 3 * node[m] + c];
-              t[v][c] += hkm * xv;
-            }
-          }
-        }
-        const double s = -Es[e];
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) acc[v][c] += s * t[v][c];
+        for (int b = 0; b < 3; ++b)
+          if ((s >> b) & 1) t[a] += s3[a][b] * sd.dNh[q][b][s];
       }
-  const uint8_t fn = fix ? fix[n] : 0;
 #pragma unroll
-  for (int v = 0; v < V; ++v) {
-    if (v >= nv) break;
+      for (int m = s; m < 8; ++m)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) y[v * 3 * nn + 3 * n + c] = ((fn >> c) & 1) ? 0.0 : acc[v][c];
+        for (int a = 0; a < 3; ++a)
+          if ((m >> a) & 1) h[stress_index(s, m)] += t[a] * sd.dNh[q][a][m];
+    }
   }
+#pragma unroll
+  for (int k = 0; k < kStressVals; ++k) H[(int64_t)k * ne + e] = h[k];
 }
 
 // q_e = sum_c phi_c^T H_e phi_c for each vector (the unscaled element term of
@@ -168,18 +127,21 @@ __global__ __launch_bounds__(NT) void k_ks_quad(const double *__restrict__ H,
   const double *p = phi + (t / ne) * ndof;
   int64_t node[8];
   element_nodes(e, nx, ny, node);
-  double f[8][3];
+  double f[3][8];
 #pragma unroll
   for (int l = 0; l < 8; ++l)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) f[l][c] = p[3 * node[l] + c];
+    for (int c = 0; c < 3; ++c) f[c][node_index(l)] = p[3 * node[l] + c];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) wht8(f[c]);
   double s = 0.0;
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
+  for (int k = 1; k < 8; ++k)
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const double hkm = H[(int64_t)(k * 8 + m) * ne + e];
-      s += hkm * (f[k][0] * f[m][0] + f[k][1] * f[m][1] + f[k][2] * f[m][2]);
+    for (int m = k; m < 8; ++m) {
+      const double hkm = H[(int64_t)stress_index(k, m) * ne + e];
+      const double d = f[0][k] * f[0][m] + f[1][k] * f[1][m] + f[2][k] * f[2][m];
+      s += (m == k ? hkm : 2 * hkm) * d;
     }
   q[t] = s;
 }
@@ -295,18 +257,6 @@ void stress_h(hipStream_t s, const double *U, int nx, int ny, int nz, const Shap
 {
   const int64_t ne = (int64_t)nx * ny * nz;
   k_stress_h<<<dim3(blocks_for(ne)), dim3(NT), 0, s>>>(U, nx, ny, nz, sd, H);
-  TOFE_LAUNCH_CHECK();
-}
-
-void apply_ks(hipStream_t s, const double *H, const double *Es, const uint8_t *fix, int nx,
-              int ny, int nz, const double *x, double *y, int nvec)
-{
-  const int64_t nn = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-  if (nvec == 1)
-    k_apply_ks<1><<<dim3(blocks_for(nn)), dim3(NT), 0, s>>>(H, Es, fix, nx, ny, nz, x, y, 1);
-  else
-    k_apply_ks<4><<<dim3(blocks_for(nn), (nvec + 3) / 4), dim3(NT), 0, s>>>(H, Es, fix, nx, ny, nz,
-                                                                           x, y, nvec);
   TOFE_LAUNCH_CHECK();
 }
 

@@ -58,4 +58,13 @@ constexpr int wht_index(int t, int i, int j)
   return base + (i == a ? (j == a ? 0 : 1) : 2);
 }
 
+// Position of entry (r, m), 1 <= r, m < 8, among the stored values of an element's stress matrix
+// h_st = (H A H)_st / 64 (symmetric; the rows of A sum to zero, so index 0 vanishes).
+constexpr int kStressVals = 28;
+constexpr int stress_index(int r, int m)
+{
+  const int a = (r < m ? r : m) - 1, b = (r < m ? m : r) - 1;
+  return a * 7 - a * (a - 1) / 2 + (b - a);
+}
+
 }  // namespace tofe

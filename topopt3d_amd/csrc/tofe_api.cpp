@@ -219,7 +219,7 @@ struct tofe_ctx {
   int mass_form = TOFE_MASS_LUMPED;
   double mass_m0 = 0;
   bool has_mass = false, has_mlump = false;
-  // stress state of the buckling analysis: H_e per element (Stability::StressFnc)
+  // stress state of the buckling analysis: H_e per element (Stability::StressFnc), 28 values
   ShapeData shape{};
   DBuf<double> Hs;
   bool has_stress = false;
@@ -1585,14 +1585,37 @@ void solve_dev(tofe_ctx *c, const double *dF, double *dU, int nrhs, double rtol,
 void apply_mass(tofe_ctx *c, const double *X, double *Y, int nrhs)
 {
   if (c->mass_form == TOFE_MASS_CONSISTENT) {
-    for (int i0 = 0; i0 < nrhs; i0 += kMaxBlockVec)
-      apply_mass_consistent(c->stream, c->mV.p, c->mass_m0, c->has_mlump ? c->mlump.p : nullptr,
-                            c->has_fix ? c->dfix.p : nullptr, c->desc.nx, c->desc.ny, c->desc.nz,
-                            X + (size_t)i0 * c->ndof, Y + (size_t)i0 * c->ndof,
-                            std::min(kMaxBlockVec, nrhs - i0));
+    FineOp<double> op = fine_of<double>(c);
+    op.zlen = c->wht_zlen;
+    op.E = c->mV.p;
+    op.escale = c->mass_m0;
+    op.spk = c->has_mlump ? c->mlump.p : nullptr;
+    op.fixval = 1e-8;
+    for (int i0 = 0; i0 < nrhs; i0 += kMaxBlockVec) {
+      EpiArgs<double> ep;
+      ep.y = Y + (size_t)i0 * c->ndof;
+      ep.nvec = std::min(kMaxBlockVec, nrhs - i0);
+      fine_mass(c->stream, op, X + (size_t)i0 * c->ndof, ep);
+    }
   } else {
     diag_mul(c->stream, c->Mdiag.p, X, Y, c->ndof, nrhs);
   }
+}
+
+// Y = Ks X for nv vectors with the stored stress state and the current Es (fixed rows give 0)
+void apply_stress(tofe_ctx *c, const double *X, double *Y, int nv)
+{
+  FineOp<double> op = fine_of<double>(c);
+  op.zlen = c->wht_zlen;
+  op.E = c->Es.p;
+  op.escale = -1;
+  op.H = c->Hs.p;
+  op.spk = nullptr;
+  op.fixval = 0;
+  EpiArgs<double> ep;
+  ep.y = Y;
+  ep.nvec = nv;
+  fine_stress(c->stream, op, X, ep);
 }
 
 // Average ms per launch of nrep back-to-back launches of one level operator kernel on the
@@ -1887,8 +1910,8 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       TOFE_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
       c->fine_tile = fine_tile_choose(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 3);
       c->fine_tile32 = fine_tile_choose(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 6);
-      c->wht_zlen = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 2);
-      c->wht_zlen32 = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 4);
+      c->wht_zlen = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, kWhtHide64);
+      c->wht_zlen32 = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, kWhtHide32);
       if (const char *wz = std::getenv("TOFE_FINE_WHT_Z")) {
         int z64 = 0, z32 = 0;
         if (std::sscanf(wz, "%d:%d", &z64, &z32) != 2 || z64 < 1 || z64 > 64 || z32 < 1 || z32 > 64)
@@ -1924,6 +1947,16 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
     compute_ke(d.E0, d.nu, d.hx, d.hy, d.hz, c->KE);
     dmatrix(d.E0, d.nu, c->shape.D);
     shape_gradients(d.hx, d.hy, d.hz, c->shape.dN, c->shape.detJ);
+    for (int q = 0; q < 8; ++q)
+      for (int a = 0; a < 3; ++a)
+        for (int t = 0; t < 8; ++t) {
+          double v = 0;
+          for (int l = 0; l < 8; ++l) {
+            const int m = ko_coord(l, 0) + 2 * ko_coord(l, 1) + 4 * ko_coord(l, 2);
+            v += (__builtin_popcount(t & m) & 1) ? -c->shape.dN[q][a][l] : c->shape.dN[q][a][l];
+          }
+          c->shape.dNh[q][a][t] = v / 8;
+        }
     // KE, then (cubic elements) the values of its 12 orbits under the symmetries of the
     // cube, used by the fine operator when every entry matches its orbit value up to the
     // rounding of the quadrature.
@@ -2448,7 +2481,7 @@ int tofe_set_stress_dev(tofe_ctx *c, const double *dU)
 {
   return guarded(c, "tofe_set_stress_dev", [&] {
     if (!dU) throw Error(TOFE_ERR_ARG, "null displacement");
-    if (!c->Hs.p) c->Hs.alloc((size_t)64 * c->ne);
+    if (!c->Hs.p) c->Hs.alloc((size_t)kStressVals * c->ne);
     stress_h(c->stream, dU, c->desc.nx, c->desc.ny, c->desc.nz, c->shape, c->Hs.p);
     TOFE_HIP(hipStreamSynchronize(c->stream));
     c->has_stress = true;
@@ -2460,7 +2493,7 @@ int tofe_set_stress(tofe_ctx *c, const double *U)
   return guarded(c, "tofe_set_stress", [&] {
     if (!U) throw Error(TOFE_ERR_ARG, "null displacement");
     h2d(c, c->vp.p, U, c->ndof);
-    if (!c->Hs.p) c->Hs.alloc((size_t)64 * c->ne);
+    if (!c->Hs.p) c->Hs.alloc((size_t)kStressVals * c->ne);
     stress_h(c->stream, c->vp.p, c->desc.nx, c->desc.ny, c->desc.nz, c->shape, c->Hs.p);
     TOFE_HIP(hipStreamSynchronize(c->stream));
     c->has_stress = true;
@@ -2474,9 +2507,8 @@ int tofe_apply_Ks_dev(tofe_ctx *c, const double *dX, double *dY, int nrhs)
     if (!c->design_set) throw Error(TOFE_ERR_STATE, "no design set");
     if (!dX || !dY || nrhs < 1) throw Error(TOFE_ERR_ARG, "bad apply arguments");
     for (int i0 = 0; i0 < nrhs; i0 += kMaxBlockVec)
-      apply_ks(c->stream, c->Hs.p, c->Es.p, c->has_fix ? c->dfix.p : nullptr, c->desc.nx,
-               c->desc.ny, c->desc.nz, dX + (size_t)i0 * c->ndof, dY + (size_t)i0 * c->ndof,
-               std::min(kMaxBlockVec, nrhs - i0));
+      apply_stress(c, dX + (size_t)i0 * c->ndof, dY + (size_t)i0 * c->ndof,
+                   std::min(kMaxBlockVec, nrhs - i0));
     TOFE_HIP(hipStreamSynchronize(c->stream));
   });
 }
@@ -2492,8 +2524,7 @@ int tofe_apply_Ks(tofe_ctx *c, const double *X, double *Y, int nrhs)
       const int nv = std::min(kMaxBlockVec, nrhs - i0);
       const size_t off = (size_t)i0 * c->ndof, len = (size_t)nv * c->ndof;
       h2d(c, c->vp.p, X + off, len);
-      apply_ks(c->stream, c->Hs.p, c->Es.p, c->has_fix ? c->dfix.p : nullptr, c->desc.nx,
-               c->desc.ny, c->desc.nz, c->vp.p, c->vq.p, nv);
+      apply_stress(c, c->vp.p, c->vq.p, nv);
       d2h(c, Y + off, c->vq.p, len);
     }
   });

@@ -77,6 +77,10 @@ struct FineOp {
   bool wht = false;            // KE[592 + k] holds its Walsh-Hadamard blocks: use k_fine_wht
   bool wht_cube = false;       // cubic element: KE[625 + k] holds the 9 cube block values
   const T *spk = nullptr;      // spring stiffness per DOF added to free diagonals (may be null)
+  // fine_mass and fine_stress: element scales escale * E, stress matrices (28 x nelem, fine_stress),
+  // spk the point masses, fixed rows return fixval * u
+  const T *H = nullptr;
+  T escale = 1, fixval = 1;
 };
 
 // Launch shape of the fine operator: one of kFineTiles compiled column tiles and the number of
@@ -89,12 +93,18 @@ struct FineTile {
 };
 FineTile fine_tile_choose(int nx, int ny, int nz, int ncu, int hide);
 // Element-centric fine operator in the Walsh-Hadamard basis of KE (k_fine_wht); hide: blocks per CU
-// that overlap for free (measured: 2 for FP64, 4 for FP32).
+// that overlap for free (measured).
+constexpr int kWhtHide64 = 2, kWhtHide32 = 4;
 int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide);
 template <typename T>
 int fine_wht_blocks(const FineOp<T> &op);
 template <typename T>
 void fine_wht(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep);
+
+// y = sum_e escale E_e A_e (x) I_3 u for ep.nvec vectors in the same march: A_e the consistent element
+// mass Q, or the element's stress matrix from op.H.
+void fine_mass(hipStream_t s, const FineOp<double> &op, const double *u, const EpiArgs<double> &ep);
+void fine_stress(hipStream_t s, const FineOp<double> &op, const double *u, const EpiArgs<double> &ep);
 
 // Stored 27-point block stencil operator of a coarse level.
 // Stencil grids with fewer nodes than this run one thread per DOF instead of one per node
@@ -489,12 +499,13 @@ struct ShapeData {
   double D[36];
   double dN[8][3][8];
   double detJ[8];
+  // (1/8) sum_n h(s, n) dN_n/dx_a with h the Walsh-Hadamard signs over the node coordinates: zero
+  // unless s has the bit of axis a
+  double dNh[8][3][8];
 };
+// H: stress matrices of U in the Walsh-Hadamard basis, H[k * nelem + e] with k = stress_index
 void stress_h(hipStream_t s, const double *U, int nx, int ny, int nz, const ShapeData &sd,
               double *H);
-// y = Ks x for nvec vectors stored one after another (H read once for up to four of them)
-void apply_ks(hipStream_t s, const double *H, const double *Es, const uint8_t *fix, int nx,
-              int ny, int nz, const double *x, double *y, int nvec = 1);
 void ks_quad(hipStream_t s, const double *H, const double *phi, int nx, int ny, int nz,
              int64_t ndof, int nvec, double *q);
 void stab_rhs(hipStream_t s, const double *phi, const double *Es, const uint8_t *fix, int nx,
@@ -508,11 +519,6 @@ void diag_mul(hipStream_t s, const double *d, const double *x, double *y, int64_
 // (consistent mass over m0), per element and vector
 void elem_quad(hipStream_t s, const double *phi, const double *KE, int nx, int ny, int nz,
                int64_t ndof, int nvec, double *kq, double *mq, bool consistent = false);
-// y = M x for nvec vectors with the consistent mass sum_e V_e m0 Q (x) I_3 + diag(mlump) and
-// the Dirichlet rows / columns of MatZeroRowsColumns(M, fixed, 1e-8)
-void apply_mass_consistent(hipStream_t s, const double *V, double m0, const double *mlump,
-                           const uint8_t *fix, int nx, int ny, int nz, const double *x, double *y,
-                           int nvec);
 void sensitivity(hipStream_t s, const double *U, const double *dEdz, const double *KE, int nx,
                  int ny, int nz, double *g);
 
