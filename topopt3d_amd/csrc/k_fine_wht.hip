@@ -399,7 +399,7 @@ WhtGrid wht_grid(const FineOp<T> &op)
 
 }  // namespace
 
-int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide)
+int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide, int nvec)
 {
   // A block lasts a fixed start (the first two planes and the launch itself, about two and a
   // half steps) and zlen + 1 steps, since the chunk's lowest element layer is formed too; with m
@@ -415,7 +415,7 @@ int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide)
   ncu = std::max(ncu, 1);
   for (int zl = 1; zl <= 24; ++zl) {
     const int nb = tiles * ((nz + 1 + zl - 1) / zl);
-    const double cost = (zl + 3.0) * ((nb + ncu - 1) / ncu + hide);
+    const double cost = (zl + 3.0) * (((int64_t)nb * nvec + ncu - 1) / ncu + hide);
     if (cost < best_cost - 1e-9 || (cost < best_cost + 1e-9 && zl > best)) {
       best_cost = cost;
       best = zl;
@@ -431,8 +431,16 @@ int fine_wht_blocks(const FineOp<T> &op)
 }
 
 template <typename T, int EPI, int FORM>
-void launch_form(hipStream_t s, const FineOp<T> &op, const T *u, const EpiArgs<T> &ep)
+void launch_form(hipStream_t s, FineOp<T> op, const T *u, const EpiArgs<T> &ep)
 {
+  // Several vectors fill the CUs with longer chunks, which form fewer extra element layers: up to six
+  // planes (longer ones measured slower: a Chebyshev step on 16 vectors of 160x80x80 670 us at 6, 717
+  // at 14).  The chunk length does not show in the outputs, only in the partial sums of the dot
+  // products, where each vector's stay those of its own launch.
+  if constexpr (EPI != EPI_APPLY_DOT && EPI != EPI_APPLY_DOT2 && EPI != EPI_CHEB_OUT)
+    if (ep.nvec > 1 && op.ncu > 0 && op.zlen < 6)
+      op.zlen = std::min(6, fine_wht_zlen(op.nx, op.ny, op.nz, op.ncu,
+                                          sizeof(T) == 8 ? kWhtHide64 : kWhtHide32, ep.nvec));
   const WhtGrid g = wht_grid(op);
   k_fine_wht<T, EPI, FORM><<<dim3(g.nblocks, ep.nvec), dim3(NW), 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y,
                                                                         g.nblocks, op.zlen);

@@ -290,6 +290,7 @@ struct tofe_ctx {
   std::vector<int> kt_kind;
   bool ke_wht_cube = false;  // ... with the 9-value block structure of a cubic element
   int wht_zlen = 8, wht_zlen32 = 8;  // its z-chunk lengths, FP64 and FP32
+  int ncu = 0;  // compute units (0: the chunk lengths were given)
   int precision = TOFE_PREC_FP64;
   int built_precision = -1;
   tofe_stats stats{};
@@ -370,6 +371,7 @@ FineOp<double> fine_of<double>(tofe_ctx *c)
   f.wht = c->ke_wht;
   f.wht_cube = c->ke_wht_cube;
   if (f.wht) f.zlen = c->wht_zlen;
+  f.ncu = c->ncu;
   f.spk = c->has_springs ? c->spk.p : nullptr;
   return f;
 }
@@ -386,6 +388,7 @@ FineOp<float> fine_of<float>(tofe_ctx *c)
   f.wht = c->ke_wht;
   f.wht_cube = c->ke_wht_cube;
   if (f.wht) f.zlen = c->wht_zlen32;
+  f.ncu = c->ncu;
   f.spk = c->has_springs ? c->spk32.p : nullptr;
   return f;
 }
@@ -1912,10 +1915,12 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       c->fine_tile32 = fine_tile_choose(c->desc.nx, c->desc.ny, c->desc.nz, ncu, 6);
       c->wht_zlen = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, kWhtHide64);
       c->wht_zlen32 = fine_wht_zlen(c->desc.nx, c->desc.ny, c->desc.nz, ncu, kWhtHide32);
+      c->ncu = ncu;
       if (const char *wz = std::getenv("TOFE_FINE_WHT_Z")) {
         int z64 = 0, z32 = 0;
         if (std::sscanf(wz, "%d:%d", &z64, &z32) != 2 || z64 < 1 || z64 > 64 || z32 < 1 || z32 > 64)
           throw Error(TOFE_ERR_ARG, std::string("TOFE_FINE_WHT_Z must be <zlen fp64>:<zlen fp32>, got ") + wz);
+        c->ncu = 0;  // the given lengths hold for every launch
         c->wht_zlen = z64;
         c->wht_zlen32 = z32;
       }

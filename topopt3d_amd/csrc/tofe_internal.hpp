@@ -81,6 +81,7 @@ struct FineOp {
   // spk the point masses, fixed rows return fixval * u
   const T *H = nullptr;
   T escale = 1, fixval = 1;
+  int ncu = 0;  // compute units, for the chunk length of launches over several vectors (0: zlen)
 };
 
 // Launch shape of the fine operator: one of kFineTiles compiled column tiles and the number of
@@ -95,7 +96,7 @@ FineTile fine_tile_choose(int nx, int ny, int nz, int ncu, int hide);
 // Element-centric fine operator in the Walsh-Hadamard basis of KE (k_fine_wht); hide: blocks per CU
 // that overlap for free (measured).
 constexpr int kWhtHide64 = 2, kWhtHide32 = 4;
-int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide);
+int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide, int nvec = 1);
 template <typename T>
 int fine_wht_blocks(const FineOp<T> &op);
 template <typename T>
