@@ -7,6 +7,7 @@
 // stencil is exact, including the Dirichlet identity rows carried up from the fine
 // level and the degenerate last cell of grids with an odd element count.
 #include <cstdlib>
+#include <type_traits>
 
 #include "k_common.hpp"
 
@@ -15,43 +16,26 @@ namespace {
 
 constexpr int NT = 256;
 
-// SPLIT (small grids): one thread per DOF instead of per node, component-major over the
-// blocks (a = blockIdx / node blocks), so a few thousand nodes still fill many waves; each
-// DOF's sum runs in the same order either way.
 // Blocks are remapped so each XCD works on a contiguous range of nodes, whose
 // neighbours' stencil blocks (read again as the transposed lower half) then sit in the
 // same L2.
-template <bool SPLIT>
-__device__ inline void split_index(int64_t nn, int blk, int nb, int64_t &n, int &a0)
-{
-  const int b = xcd_remap(blk, nb);
-  if constexpr (SPLIT) {
-    const int nbn = (int)((nn + NT - 1) / NT);
-    a0 = b / nbn;
-    n = (int64_t)(b - a0 * nbn) * NT + threadIdx.x;
-  } else {
-    a0 = 0;
-    n = (int64_t)b * NT + threadIdx.x;
-  }
-}
+__device__ inline int64_t block_node(int blk, int nb) { return (int64_t)xcd_remap(blk, nb) * NT + threadIdx.x; }
 
-template <typename T, int EPI, bool SPLIT>
+template <typename T, int EPI>
 __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
                                                    EpiArgs<T> ep, int64_t nn)
 {
   __shared__ double sred[NT / 64];
   epi_select_vector(ep, u0, 3 * nn, gridDim.x);  // vector blockIdx.y
   const T *__restrict__ u = u0;
-  int64_t n;
-  int a0;
-  split_index<SPLIT>(nn, blockIdx.x, gridDim.x, n, a0);
+  const int64_t n = block_node(blockIdx.x, gridDim.x);
   const T *__restrict__ S = op.S;
   double dsum = 0, dsum2 = 0;
   if (n < nn) {
     const int Nx = op.Nx, Ny = op.Ny, Nz = op.Nz;
     int i, j, k;
     node_ijk(n, Nx, Ny, i, j, k);
-    constexpr int NA = SPLIT ? 1 : 3;  // components summed by this thread
+    constexpr int NA = 3;
     T acc[NA];
 #pragma unroll
     for (int c = 0; c < NA; ++c) acc[c] = 0;
@@ -66,7 +50,7 @@ __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
       const T u0 = u[3 * m], u1 = u[3 * m + 1], u2 = u[3 * m + 2];
 #pragma unroll
       for (int c = 0; c < NA; ++c) {
-        const int a = SPLIT ? a0 : c;
+        const int a = c;
         T t = acc[c];
         t += S[(int64_t)(o * 9 + a * 3 + 0) * nn + n] * u0;
         t += S[(int64_t)(o * 9 + a * 3 + 1) * nn + n] * u1;
@@ -76,7 +60,7 @@ __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
     }
 #pragma unroll
     for (int c = 0; c < NA; ++c) {
-      const int64_t dof = 3 * n + (SPLIT ? a0 : c);
+      const int64_t dof = 3 * n + c;
       apply_epilogue<T, EPI>(ep, dof, acc[c], u[dof], dsum, dsum2);
     }
   }
@@ -264,28 +248,148 @@ __host__ __device__ inline int64_t su_index(int v, int64_t n)
 #ifndef TOFE_SYM64_G
 #define TOFE_SYM64_G 9
 #endif
+// Inputs of one DOF's epilogue, loaded ahead of the sum that they wait for.
+template <typename T, int EPI>
+struct EpiDof {
+  T u = 0, b = 0, dinv = 0, d = 0;
+};
+template <typename T, int EPI>
+__device__ __forceinline__ void epi_dof_load(const EpiArgs<T> &ep, const T *__restrict__ u, int64_t dof,
+                                             EpiDof<T, EPI> &in)
+{
+  if constexpr (EPI != EPI_APPLY && EPI != EPI_RESID) in.u = u[dof];
+  if constexpr (EPI == EPI_APPLY_DOT2 || EPI == EPI_RESID || EPI == EPI_CHEB) in.b = ep.b[dof];
+  if constexpr (EPI == EPI_CHEB) {
+    in.dinv = ep.dinv[dof];
+    if (ep.c1 != T(0)) in.d = ep.d[dof];
+  }
+}
+template <typename T, int EPI>
+__device__ __forceinline__ void epi_dof_store(const EpiArgs<T> &ep, int64_t dof, const EpiDof<T, EPI> &in,
+                                              T Au, double &dsum, double &dsum2)
+{
+  if constexpr (EPI == EPI_APPLY || EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) ep.y[dof] = Au;
+  if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) dsum += (double)in.u * (double)Au;
+  if constexpr (EPI == EPI_APPLY_DOT2) dsum2 += (double)in.u * (double)in.b;
+  if constexpr (EPI == EPI_RESID) ep.y[dof] = in.b - Au;
+  if constexpr (EPI == EPI_CHEB) {
+    const T r = in.dinv * (in.b - Au);
+    T dn = ep.c2 * r;
+    if (ep.c1 != T(0)) dn = __builtin_elementwise_fma(ep.c2, r, ep.c1 * in.d);  // as apply_epilogue
+    (ep.dout ? ep.dout : ep.d)[dof] = dn;
+    ep.xout[dof] = in.u + dn;
+  }
+}
+
+// Grids below StencilOp::split_nodes: a block holds one component of 64 nodes, and each of its four
+// wavefronts the terms of seven neighbours (the last one six), which the first wavefront adds up
+// in the order of the offsets: the bits are those of a thread that forms all 27.  On a small grid a
+// launch lasts as long as one thread's chain of index work, loads and products, which this cuts by
+// four; on a larger one four times the wavefronts hide the loads.  A Chebyshev step, us, FP32 /
+// FP64: 637 to 4,225 nodes 3.3 / 3.7 (one thread per DOF 6.0 / 7.4), 30,625 nodes 6.6 / 11.5 (one
+// thread per node 7.4 / 12.3), 136,161 nodes 22 / 40 (24 / 43), 232,897 nodes 34.7 / 67 (31.6 / 61):
+// bound there by the stored stencil, read through one wavefront's seven neighbours at a time.
+// V vectors per thread, the first v0.
+constexpr int kGroup = 7;
+template <typename T, int EPI, int V>
+__device__ __forceinline__ void stencil_split_block(const StencilOp<T> &op, const T *u0,
+                                                    const EpiArgs<T> &ep0, int64_t nn, int blk, int nb,
+                                                    int v0)
+{
+  __shared__ T term[V][27 - kGroup][64];  // of neighbours 7..26
+  const int lane = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = xcd_remap(blk, nb), nbn = (int)((nn + 63) >> 6);
+  const int a0 = b / nbn;
+  const int64_t n = (int64_t)(b - a0 * nbn) * 64 + lane, ndof = 3 * nn, dof = 3 * n + a0;
+  const bool live = n < nn;
+  const T *__restrict__ S = op.S;
+  T own[V][kGroup];
+  EpiDof<T, EPI> ein[V];
+  if (live) {
+    if (g == 0) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        EpiArgs<T> ep = ep0;
+        epi_offset(ep, v0 + v, ndof, nb);
+        epi_dof_load<T, EPI>(ep, u0 + (int64_t)(v0 + v) * ndof, dof, ein[v]);
+      }
+    }
+    const int Nx = op.Nx, Ny = op.Ny, Nz = op.Nz;
+    int i, j, k;
+    node_ijk(n, Nx, Ny, i, j, k);
+    const auto group = [&](auto gc) {
+      constexpr int G = decltype(gc)::value, O1 = kGroup * (G + 1) < 27 ? kGroup * (G + 1) : 27;
+#pragma unroll
+      for (int o = kGroup * G; o < O1; ++o) {
+        const int dx = o % 3 - 1, dy = (o / 3) % 3 - 1, dz = o / 9 - 1;
+        // unconditional loads (a missing neighbour reads node n; its term is zero)
+        const bool in = ((unsigned)(i + dx) < (unsigned)Nx) & ((unsigned)(j + dy) < (unsigned)Ny) &
+                        ((unsigned)(k + dz) < (unsigned)Nz);
+        const int64_t m = in ? n + dx + (int64_t)Nx * (dy + (int64_t)Ny * dz) : n;
+        // o >= 13: stored block (n, o); o < 13: stored block (m, 26 - o), transposed
+        const T *B = S + (o >= 13 ? su_index((o - 13) * 9, n) : su_index((13 - o) * 9, m));
+        const int sr = o >= 13 ? 3 : 1, sc = o >= 13 ? 1 : 3;
+        const T b0 = B[(a0 * sr) * 64], b1 = B[(a0 * sr + sc) * 64], b2 = B[(a0 * sr + 2 * sc) * 64];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const T *__restrict__ u = u0 + (int64_t)(v0 + v) * ndof;
+          const T t = row3(b0, b1, b2, u[3 * m], u[3 * m + 1], u[3 * m + 2]);
+          if constexpr (G == 0) own[v][o] = in ? t : T(0);
+          else term[v][o - kGroup][lane] = in ? t : T(0);
+        }
+      }
+    };
+    if (g == 0) group(std::integral_constant<int, 0>());
+    else if (g == 1) group(std::integral_constant<int, 1>());
+    else if (g == 2) group(std::integral_constant<int, 2>());
+    else group(std::integral_constant<int, 3>());
+  }
+  __syncthreads();
+  if (g > 0) return;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    double dsum = 0, dsum2 = 0;
+    EpiArgs<T> ep = ep0;
+    epi_offset(ep, v0 + v, ndof, nb);
+    if (live) {
+      T acc = 0;
+#pragma unroll
+      for (int o = 0; o < kGroup; ++o) acc += own[v][o];
+#pragma unroll
+      for (int o = kGroup; o < 27; ++o) acc += term[v][o - kGroup][lane];
+      epi_dof_store<T, EPI>(ep, dof, ein[v], acc, dsum, dsum2);
+    }
+    if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) {
+      const double t = wave_sum(dsum);
+      if (lane == 0) ep.partial[blk] = t;
+      if constexpr (EPI == EPI_APPLY_DOT2) {
+        const double t2 = wave_sum(dsum2);
+        if (lane == 0) ep.partial2[blk] = t2;
+      }
+    }
+  }
+}
+
 // One block (blk of nb per vector) of the upper-half stencil operator.
-template <typename T, int EPI, bool SPLIT>
+template <typename T, int EPI>
 __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const T *u0,
                                                   EpiArgs<T> ep, int64_t nn, int blk, int nb)
 {
   __shared__ double sred[NT / 64];
   epi_select_vector(ep, u0, 3 * nn, nb);  // vector blockIdx.y
   const T *__restrict__ u = u0;
-  int64_t n;
-  int a0;
-  split_index<SPLIT>(nn, blk, nb, n, a0);
+  const int64_t n = block_node(blk, nb);
   const T *__restrict__ S = op.S;
   double dsum = 0, dsum2 = 0;
   if (n < nn) {
     const int Nx = op.Nx, Ny = op.Ny, Nz = op.Nz;
     int i, j, k;
     node_ijk(n, Nx, Ny, i, j, k);
-    constexpr int NA = SPLIT ? 1 : 3;
+    constexpr int NA = 3;
     T acc[NA];
 #pragma unroll
     for (int c = 0; c < NA; ++c) acc[c] = 0;
-    if constexpr (sizeof(T) == 4 && TOFE_SYM32_G == 27 && !SPLIT) {
+    if constexpr (sizeof(T) == 4 && TOFE_SYM32_G == 27) {
       // FP32: fully unrolled; the compiler issues all 27 neighbours' loads up front (323
       // registers, one wave per SIMD), which measured faster than the rolled form below
 #pragma unroll
@@ -298,7 +402,7 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
         const T u0 = u[3 * m], u1 = u[3 * m + 1], u2 = u[3 * m + 2];
 #pragma unroll
         for (int c = 0; c < NA; ++c) {
-          const int a = SPLIT ? a0 : c;
+          const int a = c;
           T t;
           if (o >= 13) {
             const T *B = S + su_index((o - 13) * 9, n);
@@ -313,7 +417,7 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
     } else {
       // GN neighbours per iteration, the loop kept rolled so that one group's loads are in
       // flight per thread
-      constexpr int GN = sizeof(T) == 4 ? (SPLIT ? 27 : TOFE_SYM32_G) : TOFE_SYM64_G;
+      constexpr int GN = sizeof(T) == 4 ? TOFE_SYM32_G : TOFE_SYM64_G;
 #pragma unroll 1
       for (int g = 0; g < 27 / GN; ++g) {
 #pragma unroll
@@ -336,7 +440,7 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
           const int sr = up ? 3 : 1, sc = up ? 1 : 3;  // strides of (row a, column b)
 #pragma unroll
           for (int c = 0; c < NA; ++c) {
-            const int a = SPLIT ? a0 : c;
+            const int a = c;
             const T t = row3(B[(a * sr + 0 * sc) * 64], B[(a * sr + 1 * sc) * 64],
                              B[(a * sr + 2 * sc) * 64], u0, u1, u2);
             acc[c] = __builtin_fma(w, t, acc[c]);
@@ -346,7 +450,7 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
     }
 #pragma unroll
     for (int c = 0; c < NA; ++c) {
-      const int64_t dof = 3 * n + (SPLIT ? a0 : c);
+      const int64_t dof = 3 * n + c;
       apply_epilogue<T, EPI>(ep, dof, acc[c], u[dof], dsum, dsum2);
     }
   }
@@ -365,26 +469,24 @@ template <typename T, int EPI, bool SPLIT>
 __global__ __launch_bounds__(NT) void k_stencil_op_sym(StencilOp<T> op, const T *u0,
                                                        EpiArgs<T> ep, int64_t nn)
 {
-  stencil_sym_block<T, EPI, SPLIT>(op, u0, ep, nn, blockIdx.x, gridDim.x);
+  if constexpr (SPLIT) stencil_split_block<T, EPI, 1>(op, u0, ep, nn, blockIdx.x, gridDim.x, blockIdx.y);
+  else stencil_sym_block<T, EPI>(op, u0, ep, nn, blockIdx.x, gridDim.x);
 }
 
-// The same operator for V vectors per thread (blockIdx.y numbers groups of V vectors): each
+// The large-grid operator for V vectors per thread (blockIdx.y numbers groups of V vectors): each
 // stored stencil value is read once for the group instead of once per vector.  Per vector,
 // the neighbour terms (row3), their order and the epilogue are those of stencil_sym_block, so
 // every vector's result equals its one-vector launch bit for bit.
-template <typename T, int EPI, bool SPLIT, int V>
+template <typename T, int EPI, int V>
 __device__ __forceinline__ void stencil_sym_block_mv(const StencilOp<T> &op, const T *u0,
                                                      const EpiArgs<T> &ep0, int64_t nn, int blk,
                                                      int nb)
 {
-  __shared__ double sred[NT / 64];
   const int64_t ndof = 3 * nn;
   const int v0 = blockIdx.y * V;
-  int64_t n;
-  int a0;
-  split_index<SPLIT>(nn, blk, nb, n, a0);
+  const int64_t n = block_node(blk, nb);
   const T *__restrict__ S = op.S;
-  constexpr int NA = SPLIT ? 1 : 3;
+  constexpr int NA = 3;
   T acc[V][NA];
 #pragma unroll
   for (int j = 0; j < V; ++j)
@@ -411,7 +513,7 @@ __device__ __forceinline__ void stencil_sym_block_mv(const StencilOp<T> &op, con
       T bv[NA][3];
 #pragma unroll
       for (int c = 0; c < NA; ++c) {
-        const int a = SPLIT ? a0 : c;
+        const int a = c;
 #pragma unroll
         for (int q = 0; q < 3; ++q) bv[c][q] = B[(a * sr + q * sc) * 64];
       }
@@ -433,23 +535,8 @@ __device__ __forceinline__ void stencil_sym_block_mv(const StencilOp<T> &op, con
       const T *__restrict__ u = u0 + (int64_t)(v0 + jv) * ndof;
 #pragma unroll
       for (int c = 0; c < NA; ++c) {
-        const int64_t dof = 3 * n + (SPLIT ? a0 : c);
+        const int64_t dof = 3 * n + c;
         apply_epilogue<T, EPI>(ep, dof, acc[jv][c], u[dof], dsum[jv], dsum2[jv]);
-      }
-    }
-  }
-  if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2 || EPI == EPI_CHEB_OUT) {
-#pragma unroll
-    for (int jv = 0; jv < V; ++jv) {
-      EpiArgs<T> ep = ep0;
-      epi_offset(ep, v0 + jv, ndof, nb);
-      const double t = block_sum<NT>(dsum[jv], sred);
-      if (threadIdx.x == 0) ep.partial[blk] = t;
-      __syncthreads();
-      if constexpr (EPI == EPI_APPLY_DOT2) {
-        const double t2 = block_sum<NT>(dsum2[jv], sred);
-        if (threadIdx.x == 0) ep.partial2[blk] = t2;
-        __syncthreads();
       }
     }
   }
@@ -459,7 +546,10 @@ template <typename T, int EPI, bool SPLIT, int V>
 __global__ __launch_bounds__(NT) void k_stencil_op_sym_mv(StencilOp<T> op, const T *u0,
                                                           EpiArgs<T> ep, int64_t nn)
 {
-  stencil_sym_block_mv<T, EPI, SPLIT, V>(op, u0, ep, nn, blockIdx.x, gridDim.x);
+  if constexpr (SPLIT)
+    stencil_split_block<T, EPI, V>(op, u0, ep, nn, blockIdx.x, gridDim.x, V * blockIdx.y);
+  else
+    stencil_sym_block_mv<T, EPI, V>(op, u0, ep, nn, blockIdx.x, gridDim.x);
 }
 
 template <typename T, int EPI, int V>
@@ -470,13 +560,13 @@ __global__ __launch_bounds__(NT) void k_stencil_op_sym_mv_batch(const StencilLau
   const StencilLaunch<T> L = tab[e];
   const int blk = blockIdx.x - b0[e];
   if (L.nn < L.op.split_nodes)
-    stencil_sym_block_mv<T, EPI, true, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
+    stencil_split_block<T, EPI, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks, V * blockIdx.y);
   else
-    stencil_sym_block_mv<T, EPI, false, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
+    stencil_sym_block_mv<T, EPI, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
 }
 
 // The operator of several instances' levels in one grid: entry e owns blocks
-// [b0[e], b0[e + 1]); grids of either form (one thread per node or per DOF) share the launch.
+// [b0[e], b0[e + 1]); small and large grids share the launch.
 template <typename T, int EPI>
 __global__ __launch_bounds__(NT) void k_stencil_op_sym_batch(const StencilLaunch<T> *__restrict__ tab,
                                                              const int *__restrict__ b0, int n)
@@ -485,9 +575,9 @@ __global__ __launch_bounds__(NT) void k_stencil_op_sym_batch(const StencilLaunch
   const StencilLaunch<T> L = tab[e];
   const int blk = blockIdx.x - b0[e];
   if (L.nn < L.op.split_nodes)
-    stencil_sym_block<T, EPI, true>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
+    stencil_split_block<T, EPI, 1>(L.op, L.u, L.ep, L.nn, blk, L.nblocks, blockIdx.y);
   else
-    stencil_sym_block<T, EPI, false>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
+    stencil_sym_block<T, EPI>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
 }
 
 // FP64 full stencil -> upper half (offsets 13..26) in the node-blocked layout, as To;
@@ -1007,8 +1097,7 @@ template <typename T>
 int stencil_op_blocks(const StencilOp<T> &op)
 {
   const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
-  const int nb = (int)((nn + NT - 1) / NT);
-  return nn < op.split_nodes ? 3 * nb : nb;
+  return nn < op.split_nodes ? 3 * (int)((nn + 63) / 64) : (int)((nn + NT - 1) / NT);
 }
 
 #define TOFE_STENCIL_SWITCH(KERNEL)                                                         \
@@ -1046,7 +1135,15 @@ int stencil_op_blocks(const StencilOp<T> &op)
 template <typename T>
 void stencil_op(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep)
 {
-  TOFE_STENCIL_SWITCH(k_stencil_op);
+  const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
+  const dim3 grid((unsigned)((nn + NT - 1) / NT), ep.nvec), block(NT);
+  switch (epi) {
+    case EPI_APPLY: k_stencil_op<T, EPI_APPLY><<<grid, block, 0, s>>>(op, u, ep, nn); break;
+    case EPI_RESID: k_stencil_op<T, EPI_RESID><<<grid, block, 0, s>>>(op, u, ep, nn); break;
+    case EPI_CHEB: k_stencil_op<T, EPI_CHEB><<<grid, block, 0, s>>>(op, u, ep, nn); break;
+    default: throw Error(TOFE_ERR_ARG, "epilogue not available for the full stencil");
+  }
+  TOFE_LAUNCH_CHECK();
 }
 
 // Vectors per thread of the multi-vector stencil kernels for a launch over nvec vectors of
@@ -1068,9 +1165,13 @@ int stencil_mv_width(int nvec, Epi epi, int64_t nblocks)
 }
 
 template <typename T, int EPI, int V>
-void launch_sym_mv(hipStream_t s, const StencilOp<T> &op, const T *u, const EpiArgs<T> &ep)
+void launch_sym_mv(hipStream_t s, StencilOp<T> op, const T *u, const EpiArgs<T> &ep)
 {
   const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
+  // enough vectors fill the GPU with one thread per node, which reads a stencil value for all three
+  // components' sums at once (V-cycle on 16 vectors of 160x80x80, FP64: 4,566 us per node, 4,874 in
+  // groups; on 4 vectors 1,404 and 1,337)
+  if (nn >= 16384 && (nn + NT - 1) / NT * ep.nvec >= 4 * kMvMinBlocks) op.split_nodes = 0;
   const dim3 grid((unsigned)stencil_op_blocks<T>(op), ep.nvec / V), block(NT);
   if (nn < op.split_nodes) k_stencil_op_sym_mv<T, EPI, true, V><<<grid, block, 0, s>>>(op, u, ep, nn);
   else k_stencil_op_sym_mv<T, EPI, false, V><<<grid, block, 0, s>>>(op, u, ep, nn);

@@ -147,7 +147,8 @@ __device__ inline void apply_epilogue(const EpiArgs<T> &ep, int64_t dof, T Au, T
     ep.y[dof] = ep.b[dof] - Au;
   } else if constexpr (EPI == EPI_CHEB) {
     const T r = ep.dinv[dof] * (ep.b[dof] - Au);
-    const T dn = (ep.c1 == T(0)) ? ep.c2 * r : ep.c1 * ep.d[dof] + ep.c2 * r;
+    // the rounding of the sum is written out: every kernel of a level gives the same bits
+    const T dn = (ep.c1 == T(0)) ? ep.c2 * r : __builtin_elementwise_fma(ep.c2, r, ep.c1 * ep.d[dof]);
     (ep.dout ? ep.dout : ep.d)[dof] = dn;
     ep.xout[dof] = uval + dn;
   } else if constexpr (EPI == EPI_CHEB_OUT) {

@@ -277,7 +277,7 @@ struct tofe_ctx {
   // not been read (coarse_join, coarse_settle).
   bool coarse_unjoined = false, coarse_unchecked = false;
   bool fine_mfma = false;  // TOFE_FINE_MFMA=1: element-centric MFMA fine operator
-  int64_t split_nodes = kStencilSplitNodes;  // TOFE_STENCIL_SPLIT_NODES: one thread per DOF below
+  int64_t split_nodes = kStencilSplitNodes;  // TOFE_STENCIL_SPLIT_NODES: below, four wavefronts per sum
   FineTile fine_tile{0, 8}, fine_tile32{0, 8};  // k_fine_op launch shapes, FP64 and FP32
                                                 // (TOFE_FINE_TILE="<shape>:<zlen>" sets both)
   bool ke_sym = false;  // KE matches the cube-orbit table: fine operator keeps KE in registers
@@ -2155,6 +2155,8 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
       np = std::max(np, level_blocks<double>(c.get(), l));
       np = std::max(np, level_blocks<float>(c.get(), l));
     }
+    for (int l = 1; l < c->L; ++l)  // any threshold between the stencil kernels' two grids
+      np = std::max(np, 3 * (int)((c->grids[l].nn() + 63) / 64));
     if (c->ke_wht && !c->fine_mfma) {  // any z-chunk length tofe_autotune may choose
       FineOp<double> f = fine_of<double>(c.get());
       f.zlen = 1;

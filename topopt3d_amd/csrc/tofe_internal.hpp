@@ -108,16 +108,16 @@ void fine_mass(hipStream_t s, const FineOp<double> &op, const double *u, const E
 void fine_stress(hipStream_t s, const FineOp<double> &op, const double *u, const EpiArgs<double> &ep);
 
 // Stored 27-point block stencil operator of a coarse level.
-// Stencil grids with fewer nodes than this run one thread per DOF instead of one per node
-// (level 2 of the 192x96x96 cantilever, 30k nodes, is faster per node; level 1, 233k, per DOF
-// 44 us against 31 us).  TOFE_STENCIL_SPLIT_NODES overrides it per context.
-constexpr int64_t kStencilSplitNodes = 16384;
+// Stencil grids with fewer nodes than this sum a DOF's neighbours in four wavefronts instead of one
+// thread summing a node's (measured: k_coarse.hip).  TOFE_STENCIL_SPLIT_NODES overrides it per
+// context.
+constexpr int64_t kStencilSplitNodes = 200000;
 
 template <typename T>
 struct StencilOp {
   const T *S = nullptr;        // 243 * nnode
   int Nx = 0, Ny = 0, Nz = 0;  // nodes
-  int64_t split_nodes = kStencilSplitNodes;  // grids below this run one thread per DOF
+  int64_t split_nodes = kStencilSplitNodes;  // grids below this: four wavefronts per sum
 };
 
 constexpr int kRedBlocks = 1024;   // grid of the grid-stride reduction kernels
