@@ -42,7 +42,8 @@ PEAK_FP64_TFLOPS = 78.6
 PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 EPI_NAMES = {0: "apply", 1: "apply+dot", 2: "residual", 3: "Chebyshev step",
-             4: "apply+2 dots", 5: "last Chebyshev step (FP64 out)"}
+             4: "apply+2 dots", 5: "last Chebyshev step (FP64 out)",
+             6: "first two Chebyshev steps"}
 
 
 def log(*a):
@@ -83,11 +84,12 @@ def op_work(lv, level, s, epi):
     """(algorithmic bytes, algorithmic FLOP, stored bytes) of one level-operator launch:
     K-apply s(2N + Ne) and 1152 Ne FLOP (cells of the level), plus the epilogue's vectors --
     Chebyshev step +5sN (the K-apply + s*5N of the reference accounting), residual +sN (b),
-    apply with a second dot +sN (b), last step +3sN and its FP64 output and q (16N).  Stored
+    apply with a second dot +sN (b), last step +3sN and its FP64 output and q (16N), the first two
+    steps from zero +sN (b and D^-1 in, the iterate out, no operand).  Stored
     bytes replace the element scales by what the kernel actually reads as operator: E for the
     matrix-free fine level, the 126-value upper-half stencil per node on coarse levels."""
     N, Ne = lv.N[level], lv.Ne[level]
-    extra = {0: 0, 1: 0, 2: s * N, 3: 5 * s * N, 4: s * N, 5: 3 * s * N + 16 * N}[epi]
+    extra = {0: 0, 1: 0, 2: s * N, 3: 5 * s * N, 4: s * N, 5: 3 * s * N + 16 * N, 6: s * N}[epi]
     alg = s * (2 * N + Ne) + extra
     flops = 1152.0 * Ne
     if level == 0:

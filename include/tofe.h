@@ -325,7 +325,8 @@ typedef struct tofe_kernel_time {
   int level;        /* 0 fine operator, l >= 1 Galerkin stencil of level l */
   int precision;    /* TOFE_PREC_FP64, or TOFE_PREC_MIXED for an FP32 kernel */
   int epilogue;     /* 0 y = Au; 1 with u.Au; 2 residual b - Au; 3 Chebyshev step;
-                       4 with u.Au and u.b; 5 last Chebyshev step with FP64 output */
+                       4 with u.Au and u.b; 5 last Chebyshev step with FP64 output;
+                       6 the first two Chebyshev steps from zero */
   int count;        /* launches timed */
   double total_ms;  /* their summed durations */
 } tofe_kernel_time;

@@ -276,7 +276,7 @@ __device__ __forceinline__ void epi_dof_store(const EpiArgs<T> &ep, int64_t dof,
     const T r = in.dinv * (in.b - Au);
     T dn = ep.c2 * r;
     if (ep.c1 != T(0)) dn = __builtin_elementwise_fma(ep.c2, r, ep.c1 * in.d);  // as apply_epilogue
-    (ep.dout ? ep.dout : ep.d)[dof] = dn;
+    if (ep.keep_d) (ep.dout ? ep.dout : ep.d)[dof] = dn;
     ep.xout[dof] = in.u + dn;
   }
 }
@@ -1232,7 +1232,7 @@ void stencil_sym_batch(hipStream_t s, Epi epi, const StencilLaunch<T> *tab, cons
     case EPI_APPLY_DOT2: launch_sym_batch<T, EPI_APPLY_DOT2>(s, tab, b0, n, nblocks_total, nvec); break;
     case EPI_RESID: launch_sym_batch<T, EPI_RESID>(s, tab, b0, n, nblocks_total, nvec); break;
     case EPI_CHEB: launch_sym_batch<T, EPI_CHEB>(s, tab, b0, n, nblocks_total, nvec); break;
-    case EPI_CHEB_OUT: launch_sym_batch<T, EPI_CHEB_OUT>(s, tab, b0, n, nblocks_total, nvec); break;
+    default: throw Error(TOFE_ERR_ARG, "epilogue not available for stencil levels");
   }
   TOFE_LAUNCH_CHECK();
 }

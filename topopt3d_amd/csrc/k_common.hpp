@@ -149,7 +149,7 @@ __device__ inline void apply_epilogue(const EpiArgs<T> &ep, int64_t dof, T Au, T
     const T r = ep.dinv[dof] * (ep.b[dof] - Au);
     // the rounding of the sum is written out: every kernel of a level gives the same bits
     const T dn = (ep.c1 == T(0)) ? ep.c2 * r : __builtin_elementwise_fma(ep.c2, r, ep.c1 * ep.d[dof]);
-    (ep.dout ? ep.dout : ep.d)[dof] = dn;
+    if (ep.keep_d) (ep.dout ? ep.dout : ep.d)[dof] = dn;
     ep.xout[dof] = uval + dn;
   } else if constexpr (EPI == EPI_CHEB_OUT) {
     const T r = ep.dinv[dof] * (ep.b[dof] - Au);
@@ -180,17 +180,18 @@ __device__ inline void epi_load(const EpiArgs<T> &ep, const T *__restrict__ u, c
   const int64_t d0 = 3 * n;
   in.fm = fix ? fix[n] : 0u;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) in.u[c] = u[d0 + c];
-  if constexpr (EPI == EPI_APPLY_DOT2 || EPI == EPI_RESID || EPI == EPI_CHEB || EPI == EPI_CHEB_OUT) {
+  for (int c = 0; c < 3; ++c) in.u[c] = EPI == EPI_CHEB_FIRST ? T(0) : u[d0 + c];
+  if constexpr (EPI == EPI_APPLY_DOT2 || EPI == EPI_RESID || EPI == EPI_CHEB || EPI == EPI_CHEB_OUT ||
+                EPI == EPI_CHEB_FIRST) {
     const T *__restrict__ b = ep.b;
 #pragma unroll
     for (int c = 0; c < 3; ++c) in.b[c] = b[d0 + c];
   }
-  if constexpr (EPI == EPI_CHEB || EPI == EPI_CHEB_OUT) {
+  if constexpr (EPI == EPI_CHEB || EPI == EPI_CHEB_OUT || EPI == EPI_CHEB_FIRST) {
     const T *__restrict__ dinv = ep.dinv;
 #pragma unroll
     for (int c = 0; c < 3; ++c) in.dinv[c] = dinv[d0 + c];
-    if (ep.c1 != T(0)) {
+    if (EPI != EPI_CHEB_FIRST && ep.c1 != T(0)) {
       const T *__restrict__ d = ep.d;
 #pragma unroll
       for (int c = 0; c < 3; ++c) in.d[c] = d[d0 + c];
@@ -211,7 +212,8 @@ __device__ inline void epi_store(const EpiArgs<T> &ep, int64_t n, const EpiIn<T,
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const int64_t dof = d0 + c;
-    const T uval = in.u[c];
+    // EPI_CHEB_FIRST: the iterate and direction after the first step from zero (as k_cheb_zero)
+    const T uval = EPI == EPI_CHEB_FIRST ? ep.c20 * (in.dinv[c] * in.b[c]) : in.u[c];
     const T Au = ((in.fm >> c) & 1) ? uval : Ku[c];
     if constexpr (EPI == EPI_APPLY) {
       ep.y[dof] = Au;
@@ -224,14 +226,15 @@ __device__ inline void epi_store(const EpiArgs<T> &ep, int64_t n, const EpiIn<T,
       dsum2 += (double)uval * (double)in.b[c];
     } else if constexpr (EPI == EPI_RESID) {
       ep.y[dof] = in.b[c] - Au;
-    } else if constexpr (EPI == EPI_CHEB) {
+    } else if constexpr (EPI == EPI_CHEB || EPI == EPI_CHEB_FIRST) {
       const T r = in.dinv[c] * (in.b[c] - Au);
-      const T dn = (ep.c1 == T(0)) ? ep.c2 * r : ep.c1 * in.d[c] + ep.c2 * r;
-      (ep.dout ? ep.dout : ep.d)[dof] = dn;
+      const T d = EPI == EPI_CHEB_FIRST ? uval : in.d[c];
+      const T dn = (ep.c1 == T(0)) ? ep.c2 * r : __builtin_elementwise_fma(ep.c1, d, ep.c2 * r);
+      if (ep.keep_d) (ep.dout ? ep.dout : ep.d)[dof] = dn;
       ep.xout[dof] = uval + dn;
     } else if constexpr (EPI == EPI_CHEB_OUT) {
       const T r = in.dinv[c] * (in.b[c] - Au);
-      const T dn = (ep.c1 == T(0)) ? ep.c2 * r : ep.c1 * in.d[c] + ep.c2 * r;
+      const T dn = (ep.c1 == T(0)) ? ep.c2 * r : __builtin_elementwise_fma(ep.c1, in.d[c], ep.c2 * r);
       const T xt = uval + dn;
       const double x = (double)xt;
       if (ep.xout64) ep.xout64[dof] = x;

@@ -484,6 +484,7 @@ void fine_op(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const EpiA
     case EPI_RESID: launch_fine<T, EPI_RESID>(s, op, u, ep, g); break;
     case EPI_CHEB: launch_fine<T, EPI_CHEB>(s, op, u, ep, g); break;
     case EPI_CHEB_OUT: launch_fine<T, EPI_CHEB_OUT>(s, op, u, ep, g); break;
+    default: throw Error(TOFE_ERR_ARG, "epilogue not available for this fine operator");
   }
   TOFE_LAUNCH_CHECK();
 }

@@ -243,6 +243,7 @@ void fine_mfma(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const Ep
     case EPI_CHEB_OUT:
       k_fine_mfma<T, EPI_CHEB_OUT><<<grid, block, 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y, g.nblocks);
       break;
+    default: throw Error(TOFE_ERR_ARG, "epilogue not available for this fine operator");
   }
   TOFE_LAUNCH_CHECK();
 }

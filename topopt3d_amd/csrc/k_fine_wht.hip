@@ -208,31 +208,46 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
     const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
     u_node[q] = (nl < WPL && gx >= 0 && gx < Nx && gy >= 0 && gy < Ny) ? unsigned(gx + Nx * gy) : kNone;
   }
-  auto load_u = [&](T (&pu)[NU][3], unsigned (&pf)[NU], int gz) {
+  // EPI_CHEB_FIRST: pu holds b and pd D^-1 of the node, and the staged operand is c20 (D^-1 b)
+  constexpr bool FIRST = EPI == EPI_CHEB_FIRST;
+  constexpr int ND = FIRST ? NU : 1;
+  const T *__restrict__ ub = FIRST ? ep.b : u;
+  auto load_u = [&](T (&pu)[NU][3], T (&pd)[ND][3], unsigned (&pf)[NU], int gz) {
     const bool zin = gz >= 0 && gz < Nz;
     const int64_t z = zin ? gz : 0;
-    const __amdgpu_buffer_rsrc_t ur = wplane_rsrc(u + 3 * NxNy * z, 3 * NxNy * (int)sizeof(T));
+    const __amdgpu_buffer_rsrc_t ur = wplane_rsrc(ub + 3 * NxNy * z, 3 * NxNy * (int)sizeof(T));
+    const __amdgpu_buffer_rsrc_t dr =
+        wplane_rsrc(FIRST ? ep.dinv + 3 * NxNy * z : ub, FIRST ? 3 * NxNy * (int)sizeof(T) : 0);
     const __amdgpu_buffer_rsrc_t fr = wplane_rsrc(fix ? fix + NxNy * z : fix, NxNy);
 #pragma unroll
     for (int q = 0; q < NU; ++q) {
       pu[q][0] = pu[q][1] = pu[q][2] = 0;
+      if constexpr (FIRST) pd[q][0] = pd[q][1] = pd[q][2] = 0;
       pf[q] = 0;
       if (zin && u_node[q] != kNone) {
         const unsigned off = u_node[q] * (3 * sizeof(T));
 #pragma unroll
         for (int c = 0; c < 3; ++c) pu[q][c] = wplane_load<T>(ur, off + c * sizeof(T));
+        if constexpr (FIRST) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) pd[q][c] = wplane_load<T>(dr, off + c * sizeof(T));
+        }
         if (fix) pf[q] = __builtin_amdgcn_raw_buffer_load_b8(fr, u_node[q], 0, 0);
       }
     }
   };
   // the fixed-DOF mask is applied at the store, after the arithmetic that hides the loads
-  auto store_u = [&](const T (&pu)[NU][3], const unsigned (&pf)[NU], int slot) {
+  auto store_u = [&](const T (&pu)[NU][3], const T (&pd)[ND][3], const unsigned (&pf)[NU], int slot) {
 #pragma unroll
     for (int q = 0; q < NU; ++q) {
       const int nl = t + q * NW;
       if (nl < WPL) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) su[slot][c][nl] = ((pf[q] >> c) & 1u) ? T(0) : pu[q][c];
+        for (int c = 0; c < 3; ++c) {
+          T v = pu[q][c];
+          if constexpr (FIRST) v = ep.c20 * (pd[q][c] * v);
+          su[slot][c][nl] = ((pf[q] >> c) & 1u) ? T(0) : v;
+        }
       }
     }
   };
@@ -262,12 +277,12 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
 
   T Ecur;
   {
-    T pu[NU][3];
+    T pu[NU][3], pd[ND][3];
     unsigned pf[NU];
-    load_u(pu, pf, k0 - 1);
-    store_u(pu, pf, 0);
-    load_u(pu, pf, k0);
-    store_u(pu, pf, 1);
+    load_u(pu, pd, pf, k0 - 1);
+    store_u(pu, pd, pf, 0);
+    load_u(pu, pd, pf, k0);
+    store_u(pu, pd, pf, 1);
     Ecur = load_E(k0 - 1);
     if constexpr (FORM == EF_STRESS) load_H(h, k0 - 1);
   }
@@ -281,11 +296,11 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
   for (int ez = k0 - 1; ez < k1; ++ez, ++st) {
     const int slo = st % 3, shi = (st + 1) % 3, pb = NPB == 2 ? (st & 1) : 0;
     const bool more = ez + 1 < k1;
-    T pu[NU][3];
+    T pu[NU][3], pd[ND][3];
     unsigned pf[NU];
     T Enext = 0;
     if (more) {
-      load_u(pu, pf, ez + 2);
+      load_u(pu, pd, pf, ez + 2);
       Enext = load_E(ez + 1);
     }
     // this step's epilogue inputs, loaded ahead of the element arithmetic
@@ -317,7 +332,7 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
       sp[pb][c][t] = v[c][1] + from_next_lane(v[c][0]);
       sp[pb][3 + c][t] = v[c][5] + from_next_lane(v[c][4]);
     }
-    if (more) store_u(pu, pf, (st + 2) % 3);
+    if (more) store_u(pu, pd, pf, (st + 2) % 3);
     __syncthreads();
     const int tb = min(t + WT, NW - 1);  // thread (tx, ty + 1); ty = 15 owns no node
 #pragma unroll
@@ -328,7 +343,10 @@ __device__ __forceinline__ void fine_wht_block(const FineOp<T> &op, const T *u0,
     if (emit) {
       if (op.spk) {  // spring supports (point masses): + diag(spk) on free DOFs
 #pragma unroll
-        for (int c = 0; c < 3; ++c) alo[c] += op.spk[3 * n + c] * ein.u[c];
+        for (int c = 0; c < 3; ++c) {
+          const T uv = FIRST ? ep.c20 * (ein.dinv[c] * ein.b[c]) : ein.u[c];
+          alo[c] += op.spk[3 * n + c] * uv;
+        }
       }
       if constexpr (KEFORM) {
         epi_store<T, EPI>(ep, n, ein, alo, dsum, dsum2);
@@ -474,6 +492,7 @@ void fine_wht(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const Epi
     case EPI_RESID: launch_wht<T, EPI_RESID>(s, op, u, ep); break;
     case EPI_CHEB: launch_wht<T, EPI_CHEB>(s, op, u, ep); break;
     case EPI_CHEB_OUT: launch_wht<T, EPI_CHEB_OUT>(s, op, u, ep); break;
+    case EPI_CHEB_FIRST: launch_wht<T, EPI_CHEB_FIRST>(s, op, u, ep); break;
   }
   TOFE_LAUNCH_CHECK();
 }
@@ -507,6 +526,7 @@ void fine_wht_batch(hipStream_t s, Epi epi, bool cube, const FineLaunch<T> *tab,
     case EPI_RESID: launch_wht_batch<T, EPI_RESID>(s, cube, tab, b0, n, nblocks_total, nvec); break;
     case EPI_CHEB: launch_wht_batch<T, EPI_CHEB>(s, cube, tab, b0, n, nblocks_total, nvec); break;
     case EPI_CHEB_OUT: launch_wht_batch<T, EPI_CHEB_OUT>(s, cube, tab, b0, n, nblocks_total, nvec); break;
+    case EPI_CHEB_FIRST: launch_wht_batch<T, EPI_CHEB_FIRST>(s, cube, tab, b0, n, nblocks_total, nvec); break;
   }
   TOFE_LAUNCH_CHECK();
 }

@@ -409,7 +409,7 @@ __device__ __forceinline__ void fcg_xr_block(double *__restrict__ r, const doubl
     partial += v * nb;
     if (fc.b32) {
       fc.b32 += vo;
-      fc.d += vo;
+      if (fc.d) fc.d += vo;
       if (fc.x) fc.x += vo;
     }
   }
@@ -435,9 +435,11 @@ __device__ __forceinline__ void fcg_xr_block(double *__restrict__ r, const doubl
     if (fc.b32) {  // the V-cycle's first step on the new residual (as k_cheb_zero_from64)
       const float b = (float)ri;
       fc.b32[i] = b;
-      const float v = fc.c2 * (fc.dinv[i] * b);
-      fc.d[i] = v;
-      if (fc.x) fc.x[i] = v;
+      if (fc.d) {
+        const float v = fc.c2 * (fc.dinv[i] * b);
+        fc.d[i] = v;
+        if (fc.x) fc.x[i] = v;
+      }
     }
   }
   const double t = block_sum<NT>(s, sred);

@@ -645,17 +645,25 @@ struct VcycleIO {
   const float *z32 = nullptr;
 };
 
+// Whether the V-cycle's first two fine-level Chebyshev steps run as one launch (EPI_CHEB_FIRST): the
+// first one from zero is then formed where the second one reads it, and no kernel writes it.
+bool first_steps_fused(const tofe_ctx *c)
+{
+  return c->L > 1 && c->desc.nu_pre >= 2 && c->ke_wht && !c->fine_mfma;
+}
+
 // Where the mixed V-cycle's first fine-level Chebyshev step goes (b0, d, the iterate it
 // starts from), for kernels that form that step themselves; x.b32 == nullptr when the
-// V-cycle has no such step.
+// V-cycle has no such step, d == nullptr when only b0 is wanted.
 FirstCheb vcycle_first_step(tofe_ctx *c)
 {
   FirstCheb f;
   const int nu1 = c->desc.nu_pre, nu2 = c->desc.nu_post;
   if (c->built_precision != TOFE_PREC_MIXED || c->L == 1 || nu1 == 0) return f;
+  f.b32 = c->vr32.p;
+  if (first_steps_fused(c)) return f;
   Level<float> &lv = *c->lv32[0];
   const int flips = std::max(nu1 - 1, 0) + nu2;
-  f.b32 = c->vr32.p;
   f.d = lv.d.p;
   // With a second pre-smoothing step, that step reads the iterate from d (the two are equal
   // after the first step from zero), so the first step does not write it.
@@ -670,7 +678,8 @@ FirstCheb vcycle_first_step(tofe_ctx *c)
 FirstCheb64 vcycle_first_step64(tofe_ctx *c)
 {
   FirstCheb64 f;
-  if (c->built_precision != TOFE_PREC_FP64 || c->L == 1 || c->desc.nu_pre < 2) return f;
+  if (c->built_precision != TOFE_PREC_FP64 || c->L == 1 || c->desc.nu_pre < 2 || first_steps_fused(c))
+    return f;
   f.d = c->lv64[0]->d.p;
   f.dinv = c->lv64[0]->dinv.p;
   f.c2 = c->c2[0];
@@ -707,14 +716,17 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
     const double *c1 = &c->c1[(size_t)l * km], *c2 = &c->c2[(size_t)l * km];
     const bool from64 = l == 0 && mixed_io && io->b64;
     const double *b64 = from64 ? io->b64 : nullptr;
-    if (from64 && nu1 == 0)
+    const bool fused = l == 0 && first_steps_fused(c);
+    if (from64 && (nu1 == 0 || (fused && !io->first_done)))
       issue(c, [=](hipStream_t st) { convert<double, T>(st, b64, const_cast<T *>(b0), nd * nvec); });
     if (nu1 > 0) {
       // the first step from x = 0 on levels l >= 1 was formed by the restriction into l
       const T *dinv = lv.dinv.p;
       T *d = lv.d.p;
       const T c20 = (T)c2[0];
-      if constexpr (sizeof(T) == 4) {
+      if (fused) {
+        // formed by the second step
+      } else if constexpr (sizeof(T) == 4) {
         if (from64 && io->first_done) {
           // formed by the kernel that produced b64
         } else if (from64)
@@ -730,14 +742,19 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       // After a first step formed without the iterate (vcycle_first_step), the iterate equals
       // d: the second step reads its operand from d and writes the new d to the iterate's unused
       // buffer (not over d, which other blocks read as operand), and d lives there from then on.
-      bool x_in_d = l == 0 && io && io->first_done && nu1 >= 2 && (sizeof(T) == 8 || from64);
+      bool x_in_d = !fused && l == 0 && io && io->first_done && nu1 >= 2 && (sizeof(T) == 8 || from64);
       T *dc = lv.d.p;
       for (int k = 1; k < nu1; ++k) {
         EpiArgs<T> ep;
         ep.b = b; ep.dinv = lv.dinv.p; ep.d = dc; ep.xout = xo;
         ep.c1 = (T)c1[k]; ep.c2 = (T)c2[k];
         ep.nvec = nvec;
-        if (x_in_d) {
+        ep.keep_d = k + 1 < nu1;  // the sweep after the coarse correction starts anew
+        if (fused && k == 1) {
+          ep.c20 = (T)c2[0];
+          level_apply<T>(c, l, b, EPI_CHEB_FIRST, ep);
+          std::swap(xc, xo);
+        } else if (x_in_d) {
           ep.dout = xc;
           level_apply<T>(c, l, dc, EPI_CHEB, ep);
           T *const freed = dc;
@@ -803,6 +820,7 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       ep.b = b; ep.dinv = lv.dinv.p; ep.d = dcur[l] ? dcur[l] : lv.d.p; ep.xout = xo;
       ep.c1 = (T)(k == 0 ? 0.0 : c1[k]); ep.c2 = (T)c2[k];
       ep.nvec = nvec;
+      ep.keep_d = k + 1 < nu2;
       if (l == 0 && k == nu2 - 1 && mixed_io && io->x64) {
         ep.xout64 = io->want_z32 ? nullptr : io->x64;
         ep.q64 = io->q64; ep.partial = io->partial;

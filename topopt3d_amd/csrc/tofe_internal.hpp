@@ -41,9 +41,11 @@ enum Epi : int {
   EPI_RESID = 2,      // y = b - Au
   EPI_CHEB = 3,       // r = dinv (b - Au); d = c1 d + c2 r; xout = u + d
   EPI_APPLY_DOT2 = 4, // y = Au, partial += u.Au, partial2 += u.b
-  EPI_CHEB_OUT = 5    // last Chebyshev step: x = u + (c1 d + c2 dinv (b - Au)) written in
+  EPI_CHEB_OUT = 5,   // last Chebyshev step: x = u + (c1 d + c2 dinv (b - Au)) written in
                       // FP64 to xout64 (or, with xout64 null, to xout), partial += x.q64 (d is
                       // not updated)
+  EPI_CHEB_FIRST = 6  // the first two Chebyshev steps from x = 0 (fine operator only): u = d =
+                      // c20 (dinv b) is formed from b and dinv wherever it is needed, then EPI_CHEB
 };
 
 template <typename T>
@@ -58,7 +60,8 @@ struct EpiArgs {
   double *partial2 = nullptr;
   double *xout64 = nullptr;
   const double *q64 = nullptr;
-  T c1 = 0, c2 = 0;
+  T c1 = 0, c2 = 0, c20 = 0;
+  bool keep_d = true;  // Chebyshev steps: d is wanted by a further step
   // Vectors per launch: vector v (blockIdx.y) of u, y, b, d, xout, xout64 and q64 starts v
   // level-DOF counts after the first and its partial sums v gridDim.x entries after the
   // first; dinv and the operator are shared by all vectors.
@@ -321,8 +324,8 @@ void record_scalar(hipStream_t s, const double *scal, int slot, double *dst);
 // of r.r; fcg_update_xp forms beta = -sum(zq_part) / scal[PQ], applies the iterate's update
 // x += scal[ALPHA] p of the same step (deferred to where p is read anyway) and p = z + beta p;
 // fcg_update_x applies x += scal[ALPHA] p alone (a step that ends the solve).
-// Optional output of fcg_update_r: the mixed V-cycle's first Chebyshev step on the new
-// residual (b32 = (float) r, d = x = c2 dinv b32), when b32 is set.
+// Optional output of fcg_update_r for the mixed V-cycle, when b32 is set: the residual in FP32 and,
+// with d, the V-cycle's first Chebyshev step d = x = c2 dinv b32 (EPI_CHEB_FIRST forms it itself).
 struct FirstCheb {
   float *b32 = nullptr, *d = nullptr;
   float *x = nullptr;  // null: the iterate is not written (it equals d after the first step)
