@@ -46,15 +46,12 @@ __device__ __forceinline__ void reduce_final_block(const double *__restrict__ pa
     // a frozen right-hand side (converged in a block solve) takes no further steps
     const bool frozen = scal && scal[SL_FROZEN] != 0.0;
     switch (post) {
-      case POST_ALPHA_CG: scal[SL_ALPHA] = frozen ? 0.0 : scal[SL_RZ] / v; break;
-      case POST_BETA_CG:
-        scal[SL_BETA] = frozen ? 0.0 : v / scal[SL_RZ];
-        scal[SL_RZ] = v;
-        break;
+      case POST_RR_CG: scal[SL_RZ] = scal[SL_TMP]; break;
       case POST_ALPHA_FCG: scal[SL_ALPHA] = frozen ? 0.0 : scal[SL_PR] / v; break;
       case POST_BETA_FCG: scal[SL_BETA] = frozen ? 0.0 : -v / scal[SL_PQ]; break;
       case POST_CONV_FCG:
       case POST_CONV_CG:
+        if (post == POST_CONV_CG) scal[SL_RZ] = scal[SL_TMP];
         if (!frozen) {
           scal[SL_ITS] += 1.0;
           const double pq = scal[SL_PQ];
@@ -297,49 +294,6 @@ __global__ void k_fill(T *a, T v, int64_t n)
     a[i] = v;
 }
 
-// r -= alpha q; partial ||r||^2 (the iterate's update x += alpha p follows in k_cg_xp); with
-// fc.d, also the V-cycle's first fine-level Chebyshev step d = c2 D^-1 r (as k_cheb_zero).
-__global__ __launch_bounds__(NT) void k_cg_r(double *__restrict__ r, const double *__restrict__ q,
-                                             int64_t n, const double *__restrict__ scal, int alpha_slot,
-                                             double *partial, FirstCheb64 fc)
-{
-  __shared__ double sred[NT / 64];
-  const int64_t vo = (int64_t)blockIdx.y * n;  // vector blockIdx.y
-  r += vo;
-  q += vo;
-  if (fc.d) fc.d += vo;
-  scal += (int64_t)blockIdx.y * SL_COUNT;
-  partial += (int64_t)blockIdx.y * gridDim.x;
-  const double alpha = scal[alpha_slot];
-  double s = 0;
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    s += ri * ri;
-    if (fc.d) fc.d[i] = fc.c2 * (fc.dinv[i] * ri);
-  }
-  const double t = block_sum<NT>(s, sred);
-  if (threadIdx.x == 0) partial[blockIdx.x] = t;
-}
-
-// x += alpha p (the iterate's update of the step that formed alpha), then p = z + beta p
-__global__ void k_cg_xp(double *__restrict__ p, const double *__restrict__ z, double *__restrict__ x,
-                        int64_t n, const double *__restrict__ scal, int beta_slot, int alpha_slot)
-{
-  const int64_t vo = (int64_t)blockIdx.y * n;  // vector blockIdx.y
-  p += vo;
-  z += vo;
-  x += vo;
-  scal += (int64_t)blockIdx.y * SL_COUNT;
-  const double beta = scal[beta_slot], alpha = scal[alpha_slot];
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
-    const double pi = p[i];
-    // the iterate is touched once per iteration (non-temporal, as in fcg_p_block)
-    __builtin_nontemporal_store(__builtin_nontemporal_load(x + i) + alpha * pi, x + i);
-    p[i] = z[i] + beta * pi;
-  }
-}
-
 // v_i = 0.5 + frac(i * 2654435761 / 2^32): deterministic start vector of the estimate
 template <typename T>
 __global__ void k_power_start(T *v, int64_t n)
@@ -387,6 +341,69 @@ __device__ inline double all_sum(const double *__restrict__ partial, int nparts,
   for (int i = 0; i < NT / 64; ++i) t += smem[i];
   __syncthreads();
   return t;
+}
+
+// CG step without separate reduction launches, first half: alpha = r.z / p.Ap with r.z from
+// scal[TMP] and p.Ap from the operator's partials (block 0 stores p.Ap and alpha in scal); r -=
+// alpha q; partial ||r||^2 (the iterate's update x += alpha p follows in k_cg_xp); with fc.d, also
+// the V-cycle's first fine-level Chebyshev step d = c2 D^-1 r (as k_cheb_zero).
+__global__ __launch_bounds__(NT) void k_cg_r(double *__restrict__ r, const double *__restrict__ q,
+                                             int64_t n, const double *__restrict__ pq_part, int nparts,
+                                             double *scal, double *partial, FirstCheb64 fc)
+{
+  __shared__ double sred[NT / 64];
+  const int64_t vo = (int64_t)blockIdx.y * n;  // vector blockIdx.y
+  r += vo;
+  q += vo;
+  if (fc.d) fc.d += vo;
+  pq_part += (int64_t)blockIdx.y * nparts;
+  scal += (int64_t)blockIdx.y * SL_COUNT;
+  partial += (int64_t)blockIdx.y * gridDim.x;
+  const double pq = all_sum(pq_part, nparts, sred);
+  // a frozen right-hand side (converged in a block solve) takes no further steps
+  const double alpha = scal[SL_FROZEN] != 0.0 ? 0.0 : scal[SL_TMP] / pq;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[SL_PQ] = pq;
+    scal[SL_ALPHA] = alpha;
+  }
+  double s = 0;
+  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
+    const double ri = r[i] - alpha * q[i];
+    r[i] = ri;
+    s += ri * ri;
+    if (fc.d) fc.d[i] = fc.c2 * (fc.dinv[i] * ri);
+  }
+  const double t = block_sum<NT>(s, sred);
+  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
+// Second half: the new r.z from the preconditioner's partials, beta = r.z / scal[RZ] (block 0
+// stores r.z in scal[TMP], which the step's reduction of r.r moved to scal[RZ] before: the other
+// blocks still read the old one there); x += alpha p (the iterate's update of the step that formed
+// alpha), then p = z + beta p.
+__global__ __launch_bounds__(NT) void k_cg_xp(double *__restrict__ p, const double *__restrict__ z,
+                                              double *__restrict__ x, int64_t n,
+                                              const double *__restrict__ rz_part, int nparts, double *scal)
+{
+  __shared__ double sred[NT / 64];
+  const int64_t vo = (int64_t)blockIdx.y * n;  // vector blockIdx.y
+  p += vo;
+  z += vo;
+  x += vo;
+  rz_part += (int64_t)blockIdx.y * nparts;
+  scal += (int64_t)blockIdx.y * SL_COUNT;
+  const double rz = all_sum(rz_part, nparts, sred);
+  const double beta = scal[SL_FROZEN] != 0.0 ? 0.0 : rz / scal[SL_RZ], alpha = scal[SL_ALPHA];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[SL_TMP] = rz;
+    scal[SL_BETA] = beta;
+  }
+  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
+    const double pi = p[i];
+    // the iterate is touched once per iteration (non-temporal, as in fcg_p_block)
+    __builtin_nontemporal_store(__builtin_nontemporal_load(x + i) + alpha * pi, x + i);
+    p[i] = z[i] + beta * pi;
+  }
 }
 
 // Flexible-CG step without separate reduction launches, first half: alpha = p.r / p.Ap
@@ -671,17 +688,16 @@ template void fill<double>(hipStream_t, double *, double, int64_t);
 
 void fill_d(hipStream_t s, double *a, double v, int64_t n) { fill<double>(s, a, v, n); }
 
-void cg_update_r(hipStream_t s, double *r, const double *q, int64_t n, const double *scal,
-                 int alpha_slot, double *partial, int nvec, const FirstCheb64 &fc)
+void cg_update_r(hipStream_t s, double *r, const double *q, int64_t n, const double *pq_part, int nparts,
+                 double *scal, double *partial, int nvec, const FirstCheb64 &fc)
 {
-  k_cg_r<<<dim3(kRedBlocks, nvec), dim3(NT), 0, s>>>(r, q, n, scal, alpha_slot, partial, fc);
+  k_cg_r<<<dim3(kRedBlocks, nvec), dim3(NT), 0, s>>>(r, q, n, pq_part, nparts, scal, partial, fc);
   TOFE_LAUNCH_CHECK();
 }
-
-void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t n, const double *scal,
-                  int beta_slot, int alpha_slot, int nvec)
+void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t n, const double *rz_part,
+                  int nparts, double *scal, int nvec)
 {
-  k_cg_xp<<<dim3(stride_blocks(n), nvec), dim3(NT), 0, s>>>(p, z, x, n, scal, beta_slot, alpha_slot);
+  k_cg_xp<<<dim3(stride_blocks(n), nvec), dim3(NT), 0, s>>>(p, z, x, n, rz_part, nparts, scal);
   TOFE_LAUNCH_CHECK();
 }
 

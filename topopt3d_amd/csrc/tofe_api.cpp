@@ -631,7 +631,8 @@ void coarse_apply(tofe_ctx *c, const T *b, T *x, int nvec = 1)
 
 // FP64 ends of the mixed-precision V-cycle, fused into its first and last fine-level
 // kernels: b64 is converted while the first Chebyshev step is formed, and the last step
-// writes x in FP64 to x64 with the partial sums of x.q64 (one per fine-operator block).
+// writes x in FP64 to x64 with the partial sums of x.q64 (one per fine-operator block).  The FP64
+// V-cycle takes x64 (its x0), q64 and partial likewise.
 struct VcycleIO {
   const double *b64 = nullptr;
   double *x64 = nullptr;
@@ -821,8 +822,8 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       ep.c1 = (T)(k == 0 ? 0.0 : c1[k]); ep.c2 = (T)c2[k];
       ep.nvec = nvec;
       ep.keep_d = k + 1 < nu2;
-      if (l == 0 && k == nu2 - 1 && mixed_io && io->x64) {
-        ep.xout64 = io->want_z32 ? nullptr : io->x64;
+      if (l == 0 && k == nu2 - 1 && io && io->x64) {
+        ep.xout64 = mixed_io && !io->want_z32 ? io->x64 : nullptr;  // FP64: xo is x0 here
         ep.q64 = io->q64; ep.partial = io->partial;
         level_apply<T>(c, l, xc, EPI_CHEB_OUT, ep);
         io->fused_out = true;
@@ -844,7 +845,7 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
   }
 }
 
-// z = M^-1 r.  With q given (flexible CG), also the partial sums of z.q into c->partial;
+// z = M^-1 r.  With q given, also the partial sums of z.q into c->partial;
 // returns how many there are.  With z32 given, a mixed V-cycle whose last step forms z.q may
 // leave z in FP32 instead (*z32 then points to it, else *z32 = null and z holds it).
 int precondition(tofe_ctx *c, const double *r, double *z, const double *q = nullptr,
@@ -871,7 +872,11 @@ int precondition(tofe_ctx *c, const double *r, double *z, const double *q = null
   } else {
     VcycleIO io;
     io.first_done = first_done;  // the CG residual update formed the first fine-level step
-    vcycle<double>(c, r, z, first_done ? &io : nullptr, nvec);
+    if (q && c->L > 1 && !c->fine_mfma) {
+      io.x64 = z; io.q64 = q; io.partial = c->partial.p;
+    }
+    vcycle<double>(c, r, z, &io, nvec);
+    if (io.fused_out) return level_blocks<double>(c, 0);
   }
   if (!q) return 0;
   double *part = c->partial.p;
@@ -978,7 +983,7 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
       c->frozen_dirty = true;
     }
     precondition(c, r, z, nullptr, false, nvec);
-    dot_into(c, r, z, n, SL_RZ, POST_NONE, nvec);
+    dot_into(c, r, z, n, SL_TMP, POST_NONE, nvec);  // CG: becomes scal[RZ] with the step's r.r
     TOFE_HIP(hipMemcpyAsync(p, z, n * nvec * sizeof(double), hipMemcpyDeviceToDevice, s));
   }
   // The next preconditioner application and search direction depend on the device
@@ -998,9 +1003,8 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
       const int nparts = precondition(c, r, z, q, first.b32 != nullptr, nvec, &z32);
       fcg_update_xp(s, p, z, z32, U, n, c->partial.p, nparts, c->scal.p, nvec);
     } else {
-      precondition(c, r, z, nullptr, first64.d != nullptr, nvec);
-      dot_into(c, r, z, n, SL_TMP, POST_BETA_CG, nvec);
-      cg_update_xp(s, p, z, U, n, c->scal.p, SL_BETA, SL_ALPHA, nvec);
+      const int nparts = precondition(c, r, z, r, first64.d != nullptr, nvec);
+      cg_update_xp(s, p, z, U, n, c->partial.p, nparts, c->scal.p, nvec);
     }
     x_pending = false;
   };
@@ -1026,10 +1030,9 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
                    c->hscal_dev);
     } else {
       level_apply<double>(c, 0, p, EPI_APPLY_DOT, ep);
-      reduce_final(s, c->partial.p, nfb, c->scal.p + SL_PQ, POST_ALPHA_CG, c->scal.p, nvec);
-      cg_update_r(s, r, q, n, c->scal.p, SL_ALPHA, c->partial.p, nvec, first64);
+      cg_update_r(s, r, q, n, c->partial.p, nfb, c->scal.p, c->partial3.p, nvec, first64);
       x_pending = true;
-      reduce_final(s, c->partial.p, kRedBlocks, c->scal.p + SL_RR, POST_NONE, c->scal.p, nvec,
+      reduce_final(s, c->partial3.p, kRedBlocks, c->scal.p + SL_RR, POST_RR_CG, c->scal.p, nvec,
                    c->hscal_dev);
     }
     // the reduction has written this iteration's scalars to the mapped host copy: no copy
@@ -1776,14 +1779,12 @@ void iteration_on_device(tofe_ctx *c, double *U, int nvec)
     }
   } else {
     level_apply<double>(c, 0, p, EPI_APPLY_DOT, ep);
-    reduce_into(c, c->partial.p, nfb, c->scal.p + SL_PQ, POST_ALPHA_CG, c->scal.p, nvec);
-    double *scal = c->scal.p, *part = c->partial.p;
+    double *scal = c->scal.p, *part = c->partial.p, *part3 = c->partial3.p;
     const FirstCheb64 first64 = vcycle_first_step64(c);
-    issue(c, [=](hipStream_t st) { cg_update_r(st, r, q, n, scal, SL_ALPHA, part, nvec, first64); });
-    reduce_into(c, c->partial.p, kRedBlocks, c->scal.p + SL_RR, POST_CONV_CG, c->scal.p, nvec);
-    precondition(c, r, z, nullptr, first64.d != nullptr, nvec);
-    dot_into(c, r, z, n, SL_TMP, POST_BETA_CG, nvec);
-    issue(c, [=](hipStream_t st) { cg_update_xp(st, p, z, U, n, scal, SL_BETA, SL_ALPHA, nvec); });
+    issue(c, [=](hipStream_t st) { cg_update_r(st, r, q, n, part, nfb, scal, part3, nvec, first64); });
+    reduce_into(c, c->partial3.p, kRedBlocks, c->scal.p + SL_RR, POST_CONV_CG, c->scal.p, nvec);
+    const int nparts = precondition(c, r, z, r, first64.d != nullptr, nvec);
+    issue(c, [=](hipStream_t st) { cg_update_xp(st, p, z, U, n, part, nparts, scal, nvec); });
   }
 }
 
@@ -1822,7 +1823,7 @@ int start_on_device(tofe_ctx *c, const double *F, double *U, int nvec, double rt
   c->frozen_dirty = true;
   if (live) {
     precondition(c, r, z, nullptr, false, nvec);
-    dot_into(c, r, z, n, SL_RZ, POST_NONE, nvec);
+    dot_into(c, r, z, n, SL_TMP, POST_NONE, nvec);  // CG: becomes scal[RZ] with the step's r.r
     TOFE_HIP(hipMemcpyAsync(p, z, n * nvec * sizeof(double), hipMemcpyDeviceToDevice, s));
   }
   return live;

@@ -309,11 +309,15 @@ void fill_d(hipStream_t s, double *a, double v, int64_t n);
 template <typename T>
 void fill(hipStream_t s, T *a, T v, int64_t n);
 struct FirstCheb64;
-void cg_update_r(hipStream_t s, double *r, const double *q, int64_t n, const double *scal,
-                 int alpha_slot, double *partial, int nvec, const FirstCheb64 &fc);
-// x += scal[alpha_slot] p (the iterate's update, deferred to where p is read), p = z + beta p
-void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t n, const double *scal,
-                  int beta_slot, int alpha_slot, int nvec = 1);
+// CG updates that sum the producers' partials themselves: cg_update_r forms alpha = scal[TMP] /
+// sum(pq_part) (the sum and alpha stored in scal), r -= alpha q, partials of r.r (reduced with
+// POST_RR_CG or POST_CONV_CG, which move scal[TMP] = r.z to scal[RZ]); cg_update_xp forms the new
+// r.z = sum(rz_part) in scal[TMP], beta = r.z / scal[RZ], applies the iterate's update x +=
+// scal[ALPHA] p (deferred to where p is read) and p = z + beta p.
+void cg_update_r(hipStream_t s, double *r, const double *q, int64_t n, const double *pq_part, int nparts,
+                 double *scal, double *partial, int nvec, const FirstCheb64 &fc);
+void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t n, const double *rz_part,
+                  int nparts, double *scal, int nvec = 1);
 template <typename T>
 void power_start(hipStream_t s, T *v, int64_t n);
 template <typename T>
@@ -432,14 +436,13 @@ enum Slot : int {
 // reduce_final post-processing
 enum Post : int {
   POST_NONE = 0,
-  POST_ALPHA_CG = 1,   // scal[ALPHA] = scal[RZ] / v
-  POST_BETA_CG = 2,    // scal[BETA] = v / scal[RZ]; scal[RZ] = v
+  POST_RR_CG = 1,      // v = r.r of a CG step: scal[RZ] = scal[TMP], the step's r.z
   POST_ALPHA_FCG = 3,  // scal[ALPHA] = scal[PR] / v   (v = p.Ap)
   POST_BETA_FCG = 4,   // scal[BETA] = -v / scal[PQ]  (v = z.Ap)
   // v = r.r after a step of a solve whose test runs on the device: unless frozen, count the
   // step in scal[ITS] and freeze with scal[REASON] on convergence (sqrt(v) <= scal[TTOL]:
   // reason scal[CONVCODE]), on p.Ap <= 0 or NaN, on a non-finite residual, or (CG only) on
-  // r.z < 0
+  // r.z < 0 (CG: scal[RZ] = scal[TMP] first)
   POST_CONV_FCG = 5,
   POST_CONV_CG = 6
 };
