@@ -580,22 +580,67 @@ __global__ __launch_bounds__(NT) void k_stencil_op_sym_batch(const StencilLaunch
     stencil_sym_block<T, EPI>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
 }
 
-// FP64 full stencil -> upper half (offsets 13..26) in the node-blocked layout, as To;
-// blockIdx.y is the stored value v (0..125), so no thread divides by nn.
-template <typename To>
-__global__ __launch_bounds__(NT) void k_stencil_upper(const double *__restrict__ S, int64_t nn,
-                                                      To *__restrict__ Su)
+// Start of the estimates of tab's levels: the copies in T of the FP64 inverse diagonal and of
+// the full stencil's upper half (offsets 13..26, in the node-blocked layout), the start vector
+// r, p = D^-1 r and the partials of r.p.
+template <typename T>
+__global__ __launch_bounds__(NT) void k_lz_start(LzTab<T> tab)
 {
-  // One thread per node, all 126 values: a block's four 64-node groups of the node-blocked
-  // layout (32 KB each) are written in order and fill whole lines in the cache, where one value
-  // per block left 256-byte pieces 32 KB apart for other blocks to fill much later; the reads
-  // stay contiguous runs of NT values per stencil plane.
-  const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (n >= nn) return;
-  const double *__restrict__ src = S + (int64_t)(13 * 9) * nn + n;
-  To *__restrict__ dst = Su + su_index(0, n);
-#pragma unroll 9
-  for (int v = 0; v < 126; ++v) dst[(int64_t)v * 64] = (To)src[(int64_t)v * nn];
+  __shared__ double sred[NT / 64];
+  int blk = blockIdx.x, e = 0;
+  for (; blk >= tab.lv[e].nb_start; ++e) blk -= tab.lv[e].nb_start;
+  const LzLevel<T> &L = tab.lv[e];
+  const int ncopy = L.nb_start - L.nb;
+  if (blk < ncopy) {
+    // Nine values (a block of the stencil) of NT nodes: the 14 blocks of a node group follow each
+    // other, so that its lines are written while they are in the cache, and a small level still
+    // has enough threads (all 126 values per thread: 37 us on 637 nodes, 136 on 233,000;
+    // nine: 3.8 and 113, beside the fine level's start).
+    const int64_t nn = L.n / 3, n = (int64_t)(blk / 14) * NT + threadIdx.x;
+    if (n >= nn) return;
+    const int v0 = (blk % 14) * 9;
+    const double *__restrict__ src = L.S64 + (int64_t)(13 * 9 + v0) * nn + n;
+    T *__restrict__ dst = L.Su + su_index(v0, n);
+    double t[9];
+#pragma unroll
+    for (int v = 0; v < 9; ++v) t[v] = src[(int64_t)v * nn];
+#pragma unroll
+    for (int v = 0; v < 9; ++v) dst[(int64_t)v * 64] = (T)t[v];
+    return;
+  }
+  blk -= ncopy;
+  const bool copy = (const void *)L.dinv != (const void *)L.dinv64;
+  double s = 0;
+  for (int64_t i = (int64_t)blk * NT + threadIdx.x; i < L.n; i += (int64_t)L.nb * NT) {
+    const T di = (T)L.dinv64[i];
+    if (copy) L.dinv[i] = di;
+    if (L.r) {
+      const T ri = (T)power_start_value(i), zi = di * ri;
+      L.r[i] = ri;
+      L.p[i] = zi;
+      s += (double)ri * (double)zi;
+    }
+  }
+  if (!L.r) return;
+  const double t = block_sum<NT>(s, sred);
+  if (threadIdx.x == 0) L.part_0[blk] = t;
+}
+
+// q = A p with the partials of p.q on the stencils of tab's levels: the grids of
+// k_stencil_op_sym's split form side by side.
+template <typename T>
+__global__ __launch_bounds__(NT) void k_lz_apply(LzTab<T> tab)
+{
+  int blk = blockIdx.x, e = 0;
+  for (; blk >= tab.lv[e].np; ++e) blk -= tab.lv[e].np;
+  const LzLevel<T> &L = tab.lv[e];
+  StencilOp<T> op;
+  op.S = L.Su;
+  op.Nx = L.Nx; op.Ny = L.Ny; op.Nz = L.Nz;
+  EpiArgs<T> ep;
+  ep.y = L.q;
+  ep.partial = L.part;
+  stencil_split_block<T, EPI_APPLY_DOT, 1>(op, L.p, ep, L.n / 3, blk, L.np, 0);
 }
 
 __global__ void k_stencil_diag(const double *__restrict__ S, int64_t nn, double *diag,
@@ -1248,11 +1293,23 @@ void trigemv_batch(hipStream_t s, bool lower, const TrigemvLaunch<T> *tab, const
   TOFE_LAUNCH_CHECK();
 }
 
-template <typename To>
-void stencil_upper(hipStream_t s, const double *S, int64_t nn, To *Su)
+template <typename T>
+void lz_start(hipStream_t s, const LzTab<T> &tab)
 {
-  if (nn <= 0) return;
-  k_stencil_upper<To><<<dim3((unsigned)((nn + NT - 1) / NT)), dim3(NT), 0, s>>>(S, nn, Su);
+  int nb = 0;
+  for (int e = 0; e < tab.n_start; ++e) nb += tab.lv[e].nb_start;
+  if (nb == 0) return;
+  k_lz_start<T><<<dim3(nb), dim3(NT), 0, s>>>(tab);
+  TOFE_LAUNCH_CHECK();
+}
+
+template <typename T>
+void lz_apply(hipStream_t s, const LzTab<T> &tab)
+{
+  int nb = 0;
+  for (int e = 0; e < tab.n; ++e) nb += tab.lv[e].np;
+  if (nb == 0) return;
+  k_lz_apply<T><<<dim3(nb), dim3(NT), 0, s>>>(tab);
   TOFE_LAUNCH_CHECK();
 }
 
@@ -1338,8 +1395,10 @@ template void trigemv_batch<float>(hipStream_t, bool, const TrigemvLaunch<float>
                                    int, int, int);
 template void trigemv_batch<double>(hipStream_t, bool, const TrigemvLaunch<double> *, const int *,
                                     int, int, int, int);
-template void stencil_upper<float>(hipStream_t, const double *, int64_t, float *);
-template void stencil_upper<double>(hipStream_t, const double *, int64_t, double *);
+template void lz_start<float>(hipStream_t, const LzTab<float> &);
+template void lz_start<double>(hipStream_t, const LzTab<double> &);
+template void lz_apply<float>(hipStream_t, const LzTab<float> &);
+template void lz_apply<double>(hipStream_t, const LzTab<double> &);
 template void stencil_op_sym<double>(hipStream_t, const StencilOp<double> &, const double *, Epi,
                                      const EpiArgs<double> &);
 template void stencil_op_sym<float>(hipStream_t, const StencilOp<float> &, const float *, Epi,

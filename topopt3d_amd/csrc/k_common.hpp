@@ -49,6 +49,13 @@ __device__ inline double wave_sum(double v)
   return v;
 }
 
+// 0.5 + frac(i * 2654435761 / 2^32): deterministic start vector of the eigenvalue estimates
+__device__ inline double power_start_value(int64_t i)
+{
+  const uint32_t h = (uint32_t)((uint64_t)i * 2654435761ull);
+  return 0.5 + (double)h / 4294967296.0;
+}
+
 // Deterministic block sum; the result is valid in thread 0.  smem holds NT/64 doubles.
 template <int NT>
 __device__ inline double block_sum(double v, double *smem)

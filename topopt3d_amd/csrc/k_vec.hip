@@ -294,30 +294,11 @@ __global__ void k_fill(T *a, T v, int64_t n)
     a[i] = v;
 }
 
-// v_i = 0.5 + frac(i * 2654435761 / 2^32): deterministic start vector of the estimate
 template <typename T>
 __global__ void k_power_start(T *v, int64_t n)
 {
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
-    const uint32_t h = (uint32_t)((uint64_t)i * 2654435761ull);
-    v[i] = (T)(0.5 + (double)h / 4294967296.0);
-  }
-}
-
-// z = dinv r, partial r.z (Jacobi-preconditioned CG of the eigenvalue estimate)
-template <typename T>
-__global__ __launch_bounds__(NT) void k_jacobi_dot(const T *__restrict__ r, const T *__restrict__ dinv,
-                                                   T *z, int64_t n, double *partial)
-{
-  __shared__ double sred[NT / 64];
-  double s = 0;
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
-    const T zi = dinv[i] * r[i];
-    z[i] = zi;
-    s += (double)r[i] * (double)zi;
-  }
-  const double t = block_sum<NT>(s, sred);
-  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT)
+    v[i] = (T)power_start_value(i);
 }
 
 __global__ void k_record(const double *scal, int slot, double *dst)
@@ -553,47 +534,57 @@ __global__ __launch_bounds__(NT) void k_fcg_x(double *__restrict__ x, const doub
     x[i] += alpha * p[i];
 }
 
-// Jacobi-CG step of the eigenvalue estimate, first half: alpha = rz_old / p.Ap from the
-// operator's partials; r -= alpha q; partial r.(D^-1 r).  Block 0 records alpha.
+// First half of an estimate's step on the levels of tab: alpha = r.z / p.Ap from the operator's
+// partials; r -= alpha q; partial r.(D^-1 r).  A level's block 0 records alpha.  In the first
+// step r.z is the sum of lz_start's partials, which block 0 stores for k_lz_p.
 template <typename T>
-__global__ __launch_bounds__(NT) void k_lz_r(T *__restrict__ r, const T *__restrict__ q,
-                                             const T *__restrict__ dinv, int64_t n,
-                                             const double *__restrict__ pq_part, int npq,
-                                             const double *__restrict__ scal, int rz_slot,
-                                             double *rec_alpha, double *partial)
+__global__ __launch_bounds__(NT) void k_lz_r(LzTab<T> tab, int k)
 {
   __shared__ double sred[NT / 64];
-  const double alpha = scal[rz_slot] / all_sum(pq_part, npq, sred);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *rec_alpha = alpha;
+  int blk = blockIdx.x, e = 0;
+  for (; blk >= tab.lv[e].nb; ++e) blk -= tab.lv[e].nb;
+  const LzLevel<T> &L = tab.lv[e];
+  const int rz_old = (k & 1) ? SL_RZB : SL_RZA;
+  const double rz = k == 0 ? all_sum(L.part_0, L.nb, sred) : L.scal[rz_old];
+  const double alpha = rz / all_sum(L.part, L.np, sred);
+  if (blk == 0 && threadIdx.x == 0) {
+    L.alpha[k] = alpha;
+    if (k == 0) L.scal[rz_old] = rz;
+  }
   const T a = (T)alpha;
+  T *__restrict__ r = L.r;
+  const T *__restrict__ q = L.q, *__restrict__ dinv = L.dinv;
   double s = 0;
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
+  for (int64_t i = (int64_t)blk * NT + threadIdx.x; i < L.n; i += (int64_t)L.nb * NT) {
     const T ri = r[i] - a * q[i];
     r[i] = ri;
     const T zi = dinv[i] * ri;
     s += (double)ri * (double)zi;
   }
   const double t = block_sum<NT>(s, sred);
-  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+  if (threadIdx.x == 0) L.part_r[blk] = t;
 }
 
-// Second half: rz = sum of the partials, beta = rz / rz_old, p = D^-1 r + beta p.  Block 0
-// records beta and stores rz in the other slot for the next step.
+// Second half: rz = sum of the partials, beta = rz / rz_old, p = D^-1 r + beta p.  A level's
+// block 0 records beta and stores rz in the other slot for the next step.
 template <typename T>
-__global__ __launch_bounds__(NT) void k_lz_p(T *__restrict__ p, const T *__restrict__ r,
-                                             const T *__restrict__ dinv, int64_t n,
-                                             const double *__restrict__ rz_part, int nrz,
-                                             double *scal, int rz_old, int rz_new, double *rec_beta)
+__global__ __launch_bounds__(NT) void k_lz_p(LzTab<T> tab, int k)
 {
   __shared__ double sred[NT / 64];
-  const double rz = all_sum(rz_part, nrz, sred);
-  const double beta = rz / scal[rz_old];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *rec_beta = beta;
-    scal[rz_new] = rz;
+  int blk = blockIdx.x, e = 0;
+  for (; blk >= tab.lv[e].nb; ++e) blk -= tab.lv[e].nb;
+  const LzLevel<T> &L = tab.lv[e];
+  const int rz_old = (k & 1) ? SL_RZB : SL_RZA, rz_new = (k & 1) ? SL_RZA : SL_RZB;
+  const double rz = all_sum(L.part_r, L.nb, sred);
+  const double beta = rz / L.scal[rz_old];
+  if (blk == 0 && threadIdx.x == 0) {
+    L.beta[k] = beta;
+    L.scal[rz_new] = rz;
   }
   const T b = (T)beta;
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
+  T *__restrict__ p = L.p;
+  const T *__restrict__ r = L.r, *__restrict__ dinv = L.dinv;
+  for (int64_t i = (int64_t)blk * NT + threadIdx.x; i < L.n; i += (int64_t)L.nb * NT) {
     const T zi = dinv[i] * r[i];
     p[i] = zi + b * p[i];
   }
@@ -708,13 +699,6 @@ void power_start(hipStream_t s, T *v, int64_t n)
   TOFE_LAUNCH_CHECK();
 }
 
-template <typename T>
-void jacobi_dot(hipStream_t s, const T *r, const T *dinv, T *z, int64_t n, double *partial)
-{
-  k_jacobi_dot<T><<<dim3(kRedBlocks), dim3(NT), 0, s>>>(r, dinv, z, n, partial);
-  TOFE_LAUNCH_CHECK();
-}
-
 void record_scalar(hipStream_t s, const double *scal, int slot, double *dst)
 {
   k_record<<<dim3(1), dim3(64), 0, s>>>(scal, slot, dst);
@@ -782,20 +766,22 @@ void fcg_update_x(hipStream_t s, double *x, const double *p, int64_t n, const do
 }
 
 template <typename T>
-void lanczos_r(hipStream_t s, T *r, const T *q, const T *dinv, int64_t n, const double *pq_part,
-               int npq, const double *scal, int rz_slot, double *rec_alpha, double *partial)
+void lz_r(hipStream_t s, const LzTab<T> &tab, int k)
 {
-  k_lz_r<T><<<dim3(kRedBlocks), dim3(NT), 0, s>>>(r, q, dinv, n, pq_part, npq, scal, rz_slot,
-                                               rec_alpha, partial);
+  int nb = 0;
+  for (int e = 0; e < tab.n; ++e) nb += tab.lv[e].nb;
+  if (nb == 0) return;
+  k_lz_r<T><<<dim3(nb), dim3(NT), 0, s>>>(tab, k);
   TOFE_LAUNCH_CHECK();
 }
 
 template <typename T>
-void lanczos_p(hipStream_t s, T *p, const T *r, const T *dinv, int64_t n, const double *rz_part,
-               double *scal, int rz_old, int rz_new, double *rec_beta)
+void lz_p(hipStream_t s, const LzTab<T> &tab, int k)
 {
-  k_lz_p<T><<<dim3(stride_blocks(n)), dim3(NT), 0, s>>>(p, r, dinv, n, rz_part, kRedBlocks, scal,
-                                                     rz_old, rz_new, rec_beta);
+  int nb = 0;
+  for (int e = 0; e < tab.n; ++e) nb += tab.lv[e].nb;
+  if (nb == 0) return;
+  k_lz_p<T><<<dim3(nb), dim3(NT), 0, s>>>(tab, k);
   TOFE_LAUNCH_CHECK();
 }
 
@@ -810,15 +796,12 @@ void lanczos_p(hipStream_t s, T *p, const T *r, const T *dinv, int64_t n, const 
 
 TOFE_INST_T(double)
 TOFE_INST_T(float)
-#define TOFE_INST_LZ(T)                                                                      \
-  template void power_start<T>(hipStream_t, T *, int64_t);                                  \
-  template void jacobi_dot<T>(hipStream_t, const T *, const T *, T *, int64_t, double *);   \
-  template void lanczos_r<T>(hipStream_t, T *, const T *, const T *, int64_t, const double *, \
-                             int, const double *, int, double *, double *);                 \
-  template void lanczos_p<T>(hipStream_t, T *, const T *, const T *, int64_t, const double *, \
-                             double *, int, int, double *);
+#define TOFE_INST_LZ(T)                                          \
+  template void lz_r<T>(hipStream_t, const LzTab<T> &, int);     \
+  template void lz_p<T>(hipStream_t, const LzTab<T> &, int);
 TOFE_INST_LZ(double)
 TOFE_INST_LZ(float)
+template void power_start<double>(hipStream_t, double *, int64_t);
 template void convert<double, float>(hipStream_t, const double *, float *, int64_t);
 template void convert<float, double>(hipStream_t, const float *, double *, int64_t);
 

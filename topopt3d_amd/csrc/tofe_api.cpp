@@ -171,8 +171,7 @@ struct tofe_ctx {
   // second stream: the coarsest-level factorisation runs beside the Galerkin chain and the
   // Lanczos estimates
   hipStream_t stream2 = nullptr;
-  // third stream: the Lanczos estimates of the coarser smoothed levels run beside the
-  // fine level's
+  // third stream: the Lanczos estimates of the coarse smoothed levels that fill the GPU
   hipStream_t stream3 = nullptr;
   // fourth stream: the fine level's Lanczos estimate.  The third and fourth streams are
   // kept off the first kCoarseCUs compute units, which the latency-bound coarse
@@ -261,8 +260,8 @@ struct tofe_ctx {
   int nvcap = 1;
   bool frozen_dirty = false;  // some SL_FROZEN flag of scal may be set
   DBuf<double> partial, partial2, partial3, scal, eig_ab;
-  DBuf<double> partial_b, partial2_b, scal_b;  // reductions of the third stream
-  DBuf<double> partial_c, partial2_c, scal_c;  // set-up reductions of the main stream
+  DBuf<double> lz_work;          // scalars and partial sums of the levels' Lanczos estimates
+  std::vector<int64_t> lz_off;   // a level's first entry in it
   int npart = 0;
   std::vector<double> lam;
   std::vector<double> c1, c2;  // Chebyshev coefficients, per level * kmax
@@ -1087,58 +1086,119 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
   }
 }
 
-// lambda_max(D^-1 A) of level l from eig_its steps of Jacobi-preconditioned CG: the CG
-// coefficients alpha_k, beta_k (recorded on the device, read back once per assemble)
-// form the Lanczos tridiagonal whose top eigenvalue is the estimate; PETSc's Chebyshev
-// smoother estimates the same quantity (KSPChebyshevEstEigSet 0, 0.1, 0, 1.1).
+// Work of one level's estimate in the level's V-cycle work vectors and c->lz_work.
 template <typename T>
-void lanczos_coefficients(tofe_ctx *c, int l, hipStream_t s, T *r, T *p, T *q, double *part,
-                          double *part2, double *scal)
+LzLevel<T> lz_level(tofe_ctx *c, int l, bool estimate)
 {
   Level<T> &lv = *levels<T>(c)[l];
-  const int64_t nd = lv.g.ndof();
-  const int nb = level_blocks<T>(c, l);
-  const int its = std::min(c->desc.eig_its, kMaxEig);
-  double *alpha = c->eig_ab.p + (size_t)(2 * l) * kMaxEig;
-  double *beta = c->eig_ab.p + (size_t)(2 * l + 1) * kMaxEig;
-  // Three launches per step: the operator with its p.Ap partials, the r update with the
-  // r.z partials, the p update; each consumer sums the producer's partials itself.  The
-  // iterate x of the CG is never needed for the estimate and is not formed.
-  power_start<T>(s, r, nd);
-  jacobi_dot<T>(s, r, lv.dinv.p, p, nd, part);
-  reduce_final(s, part, kRedBlocks, scal + SL_RZA, POST_NONE, scal);
-  for (int k = 0; k < its; ++k) {
-    const int rz_old = (k & 1) ? SL_RZB : SL_RZA, rz_new = (k & 1) ? SL_RZA : SL_RZB;
+  LzLevel<T> e;
+  e.Nx = lv.g.Nx; e.Ny = lv.g.Ny; e.Nz = lv.g.Nz;
+  e.n = lv.g.ndof();
+  e.dinv64 = c->lv64[l]->dinv.p;
+  e.dinv = lv.dinv.p;
+  if (l > 0) {
+    if constexpr (sizeof(T) == 8) {
+      lv.Su.alloc((size_t)126 * ((lv.g.nn() + 63) / 64 * 64));
+      lv.su_ok = true;
+      e.Su = lv.Su.p;
+    } else {
+      e.Su = lv.S.p;
+    }
+    e.S64 = c->lv64[l]->S.p;
+  }
+  e.nb = (int)std::min<int64_t>(kRedBlocks, (e.n + 255) / 256);
+  e.nb_start = (l > 0 ? 14 * (int)((lv.g.nn() + 255) / 256) : 0) + e.nb;
+  if (!estimate) return e;
+  // the fine level's FP64 vectors of the V-cycle are the solver's
+  const bool own = l > 0 || sizeof(T) == 4;
+  if constexpr (sizeof(T) == 8) {
+    e.r = own ? lv.r.p : c->vr.p;
+    e.p = own ? lv.x.p : c->vp.p;
+    e.q = own ? lv.x2.p : c->vq.p;
+  } else {
+    e.r = lv.r.p;
+    e.p = lv.x.p;
+    e.q = lv.x2.p;
+  }
+  e.np = level_blocks<T>(c, l);
+  double *w = c->lz_work.p + c->lz_off[l];
+  e.scal = w;
+  e.part_r = w + SL_COUNT;
+  e.part_0 = e.part_r + kRedBlocks;
+  e.part = e.part_0 + kRedBlocks;
+  e.alpha = c->eig_ab.p + (size_t)(2 * l) * kMaxEig;
+  e.beta = c->eig_ab.p + (size_t)(2 * l + 1) * kMaxEig;
+  return e;
+}
+
+// lambda_max(D^-1 A) of the smoothed levels from eig_its steps of Jacobi-preconditioned CG
+// each: the CG coefficients alpha_k, beta_k (recorded on the device, read back once per
+// assemble) form the Lanczos tridiagonal whose top eigenvalue is the estimate; PETSc's
+// Chebyshev smoother estimates the same quantity (KSPChebyshevEstEigSet 0, 0.1, 0, 1.1).  The
+// iterate x of the CG is never needed for the estimate and is not formed.
+//
+// A step is three launches: the operator with its p.Ap partials, the r update with the r.z
+// partials, the p update; each consumer sums the producer's partials itself.  The estimates
+// are independent: the fine level's runs on the fourth stream, the levels' with the node form of
+// the stencil operator on the third, the others', launched together, on the main stream (on the
+// third, which keeps off the coarse factorisation's compute units, if it is free).  Below
+// some 100,000 nodes a launch takes the host longer than it takes the GPU, so the number of
+// launches sets the time: one chain per level, one chain after the other, against these chains
+// enqueued step by step in turn, set-up in us: 24x12x12 elements (one such level) 426 and 379,
+// 48x24x24 (two) 512 and 394.  A level that fills the GPU has its own launch: 192x96x96 takes
+// 1,905 with a chain per level, 1,946 with all coarse levels in one and 1,842 like this.
+// In the mixed-precision build the estimates run on the FP32 operators of the V-cycle (scalars
+// and recorded coefficients stay FP64), whose copies lz_start makes first; the FP64 build first
+// copies each level's stencil into its upper-half layout there.  ev_lz / ev_lz0 mark the ends of
+// the third and the fourth stream's.
+template <typename T>
+void lanczos_chains(tofe_ctx *c)
+{
+  const int L = c->L;
+  const hipStream_t s3 = c->stream3, s4 = c->stream4;
+  LzTab<T> fine, big, small;
+  std::vector<int> big_level;
+  if (L > 1 || sizeof(T) == 4) fine.lv[fine.n_start++] = lz_level<T>(c, 0, L > 1);
+  for (int l = 1; l + 1 < L; ++l) {
+    LzTab<T> &tab = c->grids[l].nn() < c->split_nodes ? small : big;
+    if (&tab == &big) big_level.push_back(l);
+    tab.lv[tab.n_start++] = lz_level<T>(c, l, true);
+  }
+  const hipStream_t s = big_level.empty() ? s3 : c->stream;
+  fine.n = L > 1 ? 1 : 0;
+  big.n = big.n_start;
+  small.n = small.n_start;
+  if (L > 1) small.lv[small.n_start++] = lz_level<T>(c, L - 1, false);
+  lz_start<T>(s4, fine);
+  lz_start<T>(s3, big);
+  lz_start<T>(s, small);
+  const int its = L > 1 ? std::min(c->desc.eig_its, kMaxEig) : 0;
+  auto apply = [&](int l, const LzLevel<T> &e, hipStream_t st) {
     EpiArgs<T> ep;
-    ep.y = q;
-    ep.partial = part;
-    level_apply<T>(c, l, p, EPI_APPLY_DOT, ep, s);
-    lanczos_r<T>(s, r, q, lv.dinv.p, nd, part, nb, scal, rz_old, alpha + k, part2);
-    lanczos_p<T>(s, p, r, lv.dinv.p, nd, part2, scal, rz_old, rz_new, beta + k);
+    ep.y = e.q;
+    ep.partial = e.part;
+    level_apply_now<T>(c, l, e.p, EPI_APPLY_DOT, ep, st);
+  };
+  for (int k = 0; k < its; ++k) {
+    apply(0, fine.lv[0], s4);
+    for (int e = 0; e < big.n; ++e) apply(big_level[e], big.lv[e], s3);
+    lz_apply<T>(s, small);
+    lz_r<T>(s4, fine, k);
+    lz_r<T>(s3, big, k);
+    lz_r<T>(s, small, k);
+    lz_p<T>(s4, fine, k);
+    lz_p<T>(s3, big, k);
+    lz_p<T>(s, small, k);
   }
 }
 
-// The smoothed levels' estimates are independent: level 1 runs on the third stream, the fine
-// level on the fourth and levels 2.. in order on the main stream, each on its level's V-cycle
-// work vectors and its stream's reduction buffers, once the operators are built on the main
-// stream.  In the mixed-precision build they run on
-// the FP32 operators of the V-cycle (scalars and recorded coefficients stay FP64), whose
-// copies are made on the same streams first; the FP64 build first copies each level's
-// stencil into its upper-half layout there.  ev_lz / ev_lz0 mark their ends.
-// The fine level's estimate on the fourth stream, once the fine diagonal (main stream) is
-// formed: it needs nothing of the Galerkin hierarchy.  ev_lz0 marks its end.
-// after: an event of the main stream recorded once E and the fine diagonal are formed (null:
-// record one now)
-void lanczos_fine_enqueue(tofe_ctx *c, hipEvent_t after = nullptr)
+void lanczos_enqueue(tofe_ctx *c)
 {
   const int L = c->L;
-  const hipStream_t s4 = c->stream4;
   c->eig_ab.alloc((size_t)2 * L * kMaxEig);
-  if (!after) {
-    TOFE_HIP(hipEventRecord(c->ev_ops, c->stream));
-    after = c->ev_ops;
-  }
-  TOFE_HIP(hipStreamWaitEvent(s4, after, 0));
+  TOFE_HIP(hipEventRecord(c->ev_ops, c->stream));
+  TOFE_HIP(hipStreamWaitEvent(c->stream4, c->ev_ops, 0));
+  TOFE_HIP(hipStreamWaitEvent(c->stream3, c->ev_ops, 0));
   if (c->precision == TOFE_PREC_MIXED) {
     if (c->lv32.empty()) {
       for (int l = 0; l < L; ++l) {
@@ -1149,64 +1209,13 @@ void lanczos_fine_enqueue(tofe_ctx *c, hipEvent_t after = nullptr)
       c->vz32.alloc((size_t)c->ndof * c->nvcap);
       TOFE_HIP(hipStreamSynchronize(c->stream));
     }
-    convert<double, float>(s4, c->lv64[0]->dinv.p, c->lv32[0]->dinv.p, c->ndof);
-    convert<double, float>(s4, c->E.p, c->E32.p, c->ne);
-    if (L > 1) {
-      Level<float> &lv = *c->lv32[0];
-      lanczos_coefficients<float>(c, 0, s4, lv.r.p, lv.x.p, lv.x2.p, c->partial.p,
-                                  c->partial2.p, c->scal.p);
-    }
-  } else if (L > 1) {
-    lanczos_coefficients<double>(c, 0, s4, c->vr.p, c->vp.p, c->vq.p, c->partial.p,
-                                 c->partial2.p, c->scal.p);
-  }
-  TOFE_HIP(hipEventRecord(c->ev_lz0, s4));
-}
-
-void lanczos_enqueue(tofe_ctx *c, bool fine_done)
-{
-  const int L = c->L;
-  // level 1 on the third stream, the fine level on the fourth (unless enqueued already),
-  // levels 2.. on the main stream (idle until it joins the others)
-  const hipStream_t s0 = c->stream, s3 = c->stream3, s4 = c->stream4;
-  if (!fine_done) lanczos_fine_enqueue(c);
-  TOFE_HIP(hipEventRecord(c->ev_ops, c->stream));
-  TOFE_HIP(hipStreamWaitEvent(s3, c->ev_ops, 0));
-  (void)s4;
-  if (c->precision == TOFE_PREC_MIXED) {
-    for (int l = 1; l < L; ++l) {
-      const hipStream_t sl = l == 1 ? s3 : s0;
-      convert<double, float>(sl, c->lv64[l]->dinv.p, c->lv32[l]->dinv.p, c->grids[l].ndof());
-      stencil_upper<float>(sl, c->lv64[l]->S.p, c->grids[l].nn(), c->lv32[l]->S.p);
-    }
-    for (int l = 1; l + 1 < L; ++l) {
-      Level<float> &lv = *c->lv32[l];
-      if (l == 1)
-        lanczos_coefficients<float>(c, l, s3, lv.r.p, lv.x.p, lv.x2.p, c->partial_b.p,
-                                    c->partial2_b.p, c->scal_b.p);
-      else
-        lanczos_coefficients<float>(c, l, s0, lv.r.p, lv.x.p, lv.x2.p, c->partial_c.p,
-                                    c->partial2_c.p, c->scal_c.p);
-    }
+    convert<double, float>(c->stream4, c->E.p, c->E32.p, c->ne);
+    lanczos_chains<float>(c);
   } else {
-    // FP64: upper-half copies of the level stencils for the Lanczos steps and the solve
-    for (int l = 1; l < L; ++l) {
-      Level<double> &lv = *c->lv64[l];
-      lv.Su.alloc((size_t)126 * ((lv.g.nn() + 63) / 64 * 64));
-      stencil_upper<double>(l == 1 ? s3 : s0, lv.S.p, lv.g.nn(), lv.Su.p);
-      lv.su_ok = true;
-    }
-    for (int l = 1; l + 1 < L; ++l) {
-      Level<double> &lv = *c->lv64[l];
-      if (l == 1)
-        lanczos_coefficients<double>(c, l, s3, lv.r.p, lv.x.p, lv.x2.p, c->partial_b.p,
-                                     c->partial2_b.p, c->scal_b.p);
-      else
-        lanczos_coefficients<double>(c, l, s0, lv.r.p, lv.x.p, lv.x2.p, c->partial_c.p,
-                                     c->partial2_c.p, c->scal_c.p);
-    }
+    lanczos_chains<double>(c);
   }
-  TOFE_HIP(hipEventRecord(c->ev_lz, s3));
+  TOFE_HIP(hipEventRecord(c->ev_lz0, c->stream4));
+  TOFE_HIP(hipEventRecord(c->ev_lz, c->stream3));
 }
 
 void lanczos_lambdas(tofe_ctx *c)
@@ -1477,15 +1486,13 @@ void assemble(tofe_ctx *c)
     TOFE_HIP(hipEventRecord(c->ev_inv, c->stream2));
     c->coarse_unjoined = c->coarse_unchecked = true;
   }
-  // The fine level's Lanczos estimate needs E and the fine diagonal only, but the fourth stream
-  // starts it after the Galerkin chain: the chain feeds the other estimates, and the estimate's
-  // bandwidth-bound kernels beside it slow it down (measured: 0.07 ms more set-up per call on the
-  // 192x96x96 cantilever when started with the chain).
-  lanczos_fine_enqueue(c);
   // Four streams from here: the coarsest level's factorisation on the second, the Lanczos
-  // estimates of level 1 on the third, of the fine level on the fourth (enqueued above) and of
-  // levels 2.. on the main stream, which then joins the other three.
-  lanczos_enqueue(c, true);
+  // estimates of large coarse levels on the third, of the fine level on the fourth and of the other
+  // levels on the main stream, which then joins the third and the fourth.  The fine level's needs E and the fine diagonal only, but it starts after
+  // the Galerkin chain: the chain feeds the other estimates, and the estimate's bandwidth-bound
+  // kernels beside it slow it down (measured: 0.07 ms more set-up per call on the 192x96x96
+  // cantilever when started with the chain).
+  lanczos_enqueue(c);
   TOFE_HIP(hipStreamWaitEvent(s, c->ev_lz, 0));
   TOFE_HIP(hipStreamWaitEvent(s, c->ev_lz0, 0));
   lanczos_lambdas(c);
@@ -2187,14 +2194,13 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
     c->partial3.alloc(np);
     c->scal.alloc(SL_COUNT);
     c->scal.zero(c->stream);
-    c->partial_b.alloc(np);
-    c->partial2_b.alloc(np);
-    c->scal_b.alloc(SL_COUNT);
-    c->scal_b.zero(c->stream);
-    c->partial_c.alloc(np);
-    c->partial2_c.alloc(np);
-    c->scal_c.alloc(SL_COUNT);
-    c->scal_c.zero(c->stream);
+    int64_t lz = 0;
+    for (int l = 0; l < c->L; ++l) {  // SL_COUNT scalars, then lz_r's, lz_start's and the operator's
+      c->lz_off.push_back(lz);
+      lz += SL_COUNT + 2 * kRedBlocks + np;
+    }
+    c->lz_work.alloc(lz);
+    c->lz_work.zero(c->stream);
     TOFE_HIP(hipStreamSynchronize(c->stream));
     c->stats.levels = c->L;
     c->stats.coarse_size = c->grids[c->L - 1].ndof();

@@ -187,13 +187,10 @@ template <typename T>
 void stencil_op(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep);
 // Coarse stencil of P^T A P, restricted axis by axis through the scratch fields T1 and T2
 // (sizes from galerkin_scratch: values in T1, and in T2 through n2).
-// Stencil operator from the upper half of a symmetric stencil (126 values per node) and
-// the FP64 full -> FP32 upper-half conversion.
+// Stencil operator from the upper half of a symmetric stencil (126 values per node; lz_start
+// forms it from the full FP64 stencil).
 template <typename T>
 void stencil_op_sym(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep);
-// FP64 full stencil -> its upper half (offsets 13..26) in k_stencil_op_sym's layout
-template <typename To>
-void stencil_upper(hipStream_t s, const double *S, int64_t nn, To *Su);
 void galerkin(hipStream_t s, const double *Sf, int Nfx, int Nfy, int Nfz, double *Sc, double *T1,
               double *T2);
 int64_t galerkin_scratch(int Nfx, int Nfy, int Nfz, int64_t *n2);
@@ -320,8 +317,6 @@ void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t 
                   int nparts, double *scal, int nvec = 1);
 template <typename T>
 void power_start(hipStream_t s, T *v, int64_t n);
-template <typename T>
-void jacobi_dot(hipStream_t s, const T *r, const T *dinv, T *z, int64_t n, double *partial);
 void record_scalar(hipStream_t s, const double *scal, int slot, double *dst);
 // Flexible-CG updates that sum the producers' partials themselves: fcg_update_r forms
 // alpha = sum(pr_part) / sum(pq_part) (stored with both sums in scal), r -= alpha q, partials
@@ -416,16 +411,44 @@ void restrict_batch(hipStream_t s, const RestrictLaunch<T> *tab, const int *b0, 
 template <typename T>
 void prolong_batch(hipStream_t s, const ProlongLaunch<T> *tab, const int *b0, int n,
                    int nblocks_total, int nvec);
-// Fused Jacobi-CG steps of the eigenvalue estimate (no separate reduction launches):
-// lanczos_r: alpha = scal[rz_slot] / sum(pq_part[0..npq)), recorded; r -= alpha q; partials
-// of r.(D^-1 r).  lanczos_p: beta = sum(rz_part) / scal[rz_old], recorded; scal[rz_new] =
-// the sum; p = D^-1 r + beta p.
+// Jacobi-CG steps of the eigenvalue estimates, one launch for the levels of a table (passed by
+// value in the kernel's arguments).
+constexpr int kLzLevels = 14;  // at most 16 levels, without the fine and the coarsest one
 template <typename T>
-void lanczos_r(hipStream_t s, T *r, const T *q, const T *dinv, int64_t n, const double *pq_part,
-               int npq, const double *scal, int rz_slot, double *rec_alpha, double *partial);
+struct LzLevel {
+  int Nx = 0, Ny = 0, Nz = 0;      // nodes
+  int64_t n = 0;                   // DOFs
+  const double *S64 = nullptr;     // full FP64 stencil (null: no copy to form)
+  T *Su = nullptr;                 // its upper half
+  const double *dinv64 = nullptr;
+  T *dinv = nullptr;               // dinv64 or its copy in T, which lz_start forms
+  T *r = nullptr, *p = nullptr, *q = nullptr;  // r null: copies only, no estimate
+  double *part = nullptr;          // p.Ap partials of the operator, np of them
+  double *part_r = nullptr;        // r.z partials of lz_r, nb of them
+  double *part_0 = nullptr;        // r.z partials of lz_start, nb of them
+  double *scal = nullptr, *alpha = nullptr, *beta = nullptr;
+  int np = 0, nb = 0;
+  int nb_start = 0;                // blocks of lz_start: the stencil's copy, then nb
+};
 template <typename T>
-void lanczos_p(hipStream_t s, T *p, const T *r, const T *dinv, int64_t n, const double *rz_part,
-               double *scal, int rz_old, int rz_new, double *rec_beta);
+struct LzTab {
+  int n = 0;          // entries with an estimate, first in lv
+  int n_start = 0;    // entries of lz_start
+  LzLevel<T> lv[kLzLevels + 1];
+};
+// Copies in T (inverse diagonal, upper-half stencil), r = the start vector, p = D^-1 r and the
+// partials of r.p.
+template <typename T>
+void lz_start(hipStream_t s, const LzTab<T> &tab);
+// q = A p and the partials of p.q on the levels' stencils
+template <typename T>
+void lz_apply(hipStream_t s, const LzTab<T> &tab);
+// alpha = r.z / sum(part), recorded; r -= alpha q; partials of r.(D^-1 r)
+template <typename T>
+void lz_r(hipStream_t s, const LzTab<T> &tab, int k);
+// beta = sum(part_r) / r.z, recorded; p = D^-1 r + beta p; the sum is the next step's r.z
+template <typename T>
+void lz_p(hipStream_t s, const LzTab<T> &tab, int k);
 
 // device scalar slots (ctx->scal)
 enum Slot : int {
