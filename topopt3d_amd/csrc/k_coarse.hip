@@ -1307,7 +1307,7 @@ template <typename T>
 void lz_apply(hipStream_t s, const LzTab<T> &tab)
 {
   int nb = 0;
-  for (int e = 0; e < tab.n; ++e) nb += tab.lv[e].np;
+  for (int e = 0; e < tab.n_apply; ++e) nb += tab.lv[e].np;
   if (nb == 0) return;
   k_lz_apply<T><<<dim3(nb), dim3(NT), 0, s>>>(tab);
   TOFE_LAUNCH_CHECK();

@@ -171,7 +171,7 @@ struct tofe_ctx {
   // second stream: the coarsest-level factorisation runs beside the Galerkin chain and the
   // Lanczos estimates
   hipStream_t stream2 = nullptr;
-  // third stream: the Lanczos estimates of the coarse smoothed levels that fill the GPU
+  // third stream: the Lanczos estimates of the coarse smoothed levels
   hipStream_t stream3 = nullptr;
   // fourth stream: the fine level's Lanczos estimate.  The third and fourth streams are
   // kept off the first kCoarseCUs compute units, which the latency-bound coarse
@@ -1139,14 +1139,13 @@ LzLevel<T> lz_level(tofe_ctx *c, int l, bool estimate)
 //
 // A step is three launches: the operator with its p.Ap partials, the r update with the r.z
 // partials, the p update; each consumer sums the producer's partials itself.  The estimates
-// are independent: the fine level's runs on the fourth stream, the levels' with the node form of
-// the stencil operator on the third, the others', launched together, on the main stream (on the
-// third, which keeps off the coarse factorisation's compute units, if it is free).  Below
-// some 100,000 nodes a launch takes the host longer than it takes the GPU, so the number of
-// launches sets the time: one chain per level, one chain after the other, against these chains
-// enqueued step by step in turn, set-up in us: 24x12x12 elements (one such level) 426 and 379,
-// 48x24x24 (two) 512 and 394.  A level that fills the GPU has its own launch: 192x96x96 takes
-// 1,905 with a chain per level, 1,946 with all coarse levels in one and 1,842 like this.
+// are independent: the fine level's runs on the fourth stream, the coarse levels' on the third,
+// where they share the launches.  Below some 100,000 nodes a launch takes the host longer than it
+// takes the GPU, so the number of launches sets the time: one chain per level, one chain after the
+// other, against these two enqueued step by step in turn, set-up in us: 24x12x12 elements (one such
+// level) 426 and 379, 48x24x24 (two) 512 and 394.  Only the operator of a level that the stencil's
+// node form takes has a launch of its own (192x96x96: 1,895; in the split form with the others,
+// 1,946).
 // In the mixed-precision build the estimates run on the FP32 operators of the V-cycle (scalars
 // and recorded coefficients stay FP64), whose copies lz_start makes first; the FP64 build first
 // copies each level's stencil into its upper-half layout there.  ev_lz / ev_lz0 mark the ends of
@@ -1156,39 +1155,35 @@ void lanczos_chains(tofe_ctx *c)
 {
   const int L = c->L;
   const hipStream_t s3 = c->stream3, s4 = c->stream4;
-  LzTab<T> fine, big, small;
-  std::vector<int> big_level;
+  LzTab<T> fine, coarse;
   if (L > 1 || sizeof(T) == 4) fine.lv[fine.n_start++] = lz_level<T>(c, 0, L > 1);
-  for (int l = 1; l + 1 < L; ++l) {
-    LzTab<T> &tab = c->grids[l].nn() < c->split_nodes ? small : big;
-    if (&tab == &big) big_level.push_back(l);
-    tab.lv[tab.n_start++] = lz_level<T>(c, l, true);
-  }
-  const hipStream_t s = big_level.empty() ? s3 : c->stream;
   fine.n = L > 1 ? 1 : 0;
-  big.n = big.n_start;
-  small.n = small.n_start;
-  if (L > 1) small.lv[small.n_start++] = lz_level<T>(c, L - 1, false);
+  std::vector<int> level;  // of the coarse table's entries: those of lz_apply first
+  for (const bool split : {true, false}) {
+    for (int l = 1; l + 1 < L; ++l)
+      if ((c->grids[l].nn() < c->split_nodes) == split) level.push_back(l);
+    if (split) coarse.n_apply = (int)level.size();
+  }
+  for (int l : level) coarse.lv[coarse.n++] = lz_level<T>(c, l, true);
+  coarse.n_start = coarse.n;
+  if (L > 1) coarse.lv[coarse.n_start++] = lz_level<T>(c, L - 1, false);
   lz_start<T>(s4, fine);
-  lz_start<T>(s3, big);
-  lz_start<T>(s, small);
+  lz_start<T>(s3, coarse);
   const int its = L > 1 ? std::min(c->desc.eig_its, kMaxEig) : 0;
-  auto apply = [&](int l, const LzLevel<T> &e, hipStream_t st) {
+  auto apply = [&](int l, const LzLevel<T> &e, hipStream_t s) {
     EpiArgs<T> ep;
     ep.y = e.q;
     ep.partial = e.part;
-    level_apply_now<T>(c, l, e.p, EPI_APPLY_DOT, ep, st);
+    level_apply_now<T>(c, l, e.p, EPI_APPLY_DOT, ep, s);
   };
   for (int k = 0; k < its; ++k) {
     apply(0, fine.lv[0], s4);
-    for (int e = 0; e < big.n; ++e) apply(big_level[e], big.lv[e], s3);
-    lz_apply<T>(s, small);
+    for (int e = coarse.n_apply; e < coarse.n; ++e) apply(level[e], coarse.lv[e], s3);
+    lz_apply<T>(s3, coarse);
     lz_r<T>(s4, fine, k);
-    lz_r<T>(s3, big, k);
-    lz_r<T>(s, small, k);
+    lz_r<T>(s3, coarse, k);
     lz_p<T>(s4, fine, k);
-    lz_p<T>(s3, big, k);
-    lz_p<T>(s, small, k);
+    lz_p<T>(s3, coarse, k);
   }
 }
 
@@ -1196,9 +1191,14 @@ void lanczos_enqueue(tofe_ctx *c)
 {
   const int L = c->L;
   c->eig_ab.alloc((size_t)2 * L * kMaxEig);
+  // The host waits for the operators, and in assemble for the estimates, where the streams could
+  // wait for each other's events: hardware queues that share a pipe are served in turn, and one
+  // whose head is such a wait gives the pipe back only at the end of its time slice, 1 ms.  Whether
+  // two of a context's queues share one depends on the streams that the process made before.  Set-up
+  // of a context made beside others, us: 192x96x96 3,015 with the streams' waits, 1,921 with the
+  // host's, 96x48x48 1,465 and 650, 80x40x40 1,322 and 475; alone in its process no difference.
   TOFE_HIP(hipEventRecord(c->ev_ops, c->stream));
-  TOFE_HIP(hipStreamWaitEvent(c->stream4, c->ev_ops, 0));
-  TOFE_HIP(hipStreamWaitEvent(c->stream3, c->ev_ops, 0));
+  TOFE_HIP(hipEventSynchronize(c->ev_ops));
   if (c->precision == TOFE_PREC_MIXED) {
     if (c->lv32.empty()) {
       for (int l = 0; l < L; ++l) {
@@ -1486,15 +1486,14 @@ void assemble(tofe_ctx *c)
     TOFE_HIP(hipEventRecord(c->ev_inv, c->stream2));
     c->coarse_unjoined = c->coarse_unchecked = true;
   }
-  // Four streams from here: the coarsest level's factorisation on the second, the Lanczos
-  // estimates of large coarse levels on the third, of the fine level on the fourth and of the other
-  // levels on the main stream, which then joins the third and the fourth.  The fine level's needs E and the fine diagonal only, but it starts after
-  // the Galerkin chain: the chain feeds the other estimates, and the estimate's bandwidth-bound
-  // kernels beside it slow it down (measured: 0.07 ms more set-up per call on the 192x96x96
-  // cantilever when started with the chain).
+  // Three streams from here: the coarsest level's factorisation on the second, the Lanczos
+  // estimates of the coarse levels on the third, of the fine level on the fourth.  The fine level's
+  // needs E and the fine diagonal only, but it starts after the Galerkin chain: the chain feeds the
+  // other estimates, and the estimate's bandwidth-bound kernels beside it slow it down (measured:
+  // 0.07 ms more set-up per call on the 192x96x96 cantilever when started with the chain).
   lanczos_enqueue(c);
-  TOFE_HIP(hipStreamWaitEvent(s, c->ev_lz, 0));
-  TOFE_HIP(hipStreamWaitEvent(s, c->ev_lz0, 0));
+  TOFE_HIP(hipEventSynchronize(c->ev_lz));
+  TOFE_HIP(hipEventSynchronize(c->ev_lz0));
   lanczos_lambdas(c);
   chebyshev_coefficients(c);
   // the factorisation (flagged where it was enqueued, so that a call after a failure here

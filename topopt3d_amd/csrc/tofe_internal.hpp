@@ -433,6 +433,7 @@ struct LzLevel {
 template <typename T>
 struct LzTab {
   int n = 0;          // entries with an estimate, first in lv
+  int n_apply = 0;    // of these, entries of lz_apply, first in lv
   int n_start = 0;    // entries of lz_start
   LzLevel<T> lv[kLzLevels + 1];
 };
