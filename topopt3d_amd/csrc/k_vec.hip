@@ -147,8 +147,12 @@ __global__ void k_cheb_zero_from64(const double *__restrict__ b64, float *__rest
 // loads; the sums run in the same ascending order as a skip-based loop and the zero terms
 // leave them unchanged.
 
-// b_c(I) = sum over fine nodes i within one fine step of 2I of w(i,I) r_f(i)  (P^T r)
-template <typename T>
+// b_c(I) = sum over fine nodes i within one fine step of 2I of w(i,I) r_f(i)  (P^T r) for NQ
+// components per thread.  A coarse level's launch is a chain of latencies: a thread per DOF has its
+// 27 loads in flight at once (637 nodes, FP64: 6.6 us per node, 3.4 per DOF; 12,800 nodes x 4
+// vectors, FP32: 6.5 and 6.1).  A grid that fills the GPU is bound by the number of loads either
+// way and shares a node's indices and weights (233,000 nodes, FP32: 11.2 and 14.0).
+template <typename T, int NQ>
 __device__ __forceinline__ void restrict_block(const T *__restrict__ rf, int Nfx, int Nfy, int Nfz,
                                                T *__restrict__ bc, int Ncx, int Ncy, int Ncz,
                                                FirstStep<T> fs, int blk)
@@ -163,62 +167,78 @@ __device__ __forceinline__ void restrict_block(const T *__restrict__ rf, int Nfx
       fs.x += v * 3 * ncn;
     }
   }
-  const int64_t I = (int64_t)blk * NT + threadIdx.x;
-  if (I >= ncn) return;
+  const int64_t t = ((int64_t)blk * NT + threadIdx.x) * NQ;
+  if (t >= 3 * ncn) return;
+  const unsigned I = (unsigned)t / 3u;
   int Ix, Iy, Iz;
   node_ijk(I, Ncx, Ncy, Ix, Iy, Iz);
-  int ix[3], iy[3], iz[3];
-  double wx[3], wy[3], wz[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int fx = 2 * Ix - 1 + d, fy = 2 * Iy - 1 + d, fz = 2 * Iz - 1 + d;
-    const bool okx = fx >= 0 && fx < Nfx, oky = fy >= 0 && fy < Nfy, okz = fz >= 0 && fz < Nfz;
-    ix[d] = okx ? fx : 2 * Ix;
-    iy[d] = oky ? fy : 2 * Iy;
-    iz[d] = okz ? fz : 2 * Iz;
-    wx[d] = okx ? w1d(fx, Ix, Nfx) : 0.0;
-    wy[d] = oky ? w1d(fy, Iy, Nfy) : 0.0;
-    wz[d] = okz ? w1d(fz, Iz, Nfz) : 0.0;
-  }
-  double acc[3] = {0, 0, 0};
+  rf += (int64_t)((unsigned)t - 3u * I);
+  // partners 2I - 1, 2I and 2I + 1 of each axis; the weight of 2I is one
+  const int fx = 2 * Ix, fy = 2 * Iy, fz = 2 * Iz;
+  const bool xl = fx > 0, xr = fx + 1 < Nfx, yl = fy > 0, yr = fy + 1 < Nfy, zl = fz > 0, zr = fz + 1 < Nfz;
+  const int iy[3] = {yl ? fy - 1 : fy, fy, yr ? fy + 1 : fy};
+  const int iz[3] = {zl ? fz - 1 : fz, fz, zr ? fz + 1 : fz};
+  const int dl = xl ? -3 : 0, dr = xr ? 3 : 0;
+  T v[27][NQ];
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
-    for (int b = 0; b < 3; ++b)
+    for (int b = 0; b < 3; ++b) {
+      const unsigned f = ((unsigned)iz[c] * (unsigned)Nfy + (unsigned)iy[b]) * (unsigned)Nfx + (unsigned)fx;
+      const T *m = rf + 3 * (int64_t)f;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const double w = wx[a] * wy[b] * wz[c];
-        const int64_t f = ix[a] + (int64_t)Nfx * (iy[b] + (int64_t)Nfy * iz[c]);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) acc[q] += w * (double)rf[3 * f + q];
+      for (int q = 0; q < NQ; ++q) {
+        v[9 * c + 3 * b][q] = m[dl + q];
+        v[9 * c + 3 * b + 1][q] = m[q];
+        v[9 * c + 3 * b + 2][q] = m[dr + q];
       }
+    }
+  if (NQ == 1) __builtin_amdgcn_sched_barrier(0);  // every load before the first sum
+  const double wl = xl ? w1d(fx - 1, Ix, Nfx) : 0.0, wr = xr ? w1d(fx + 1, Ix, Nfx) : 0.0;
+  const double wy[3] = {yl ? w1d(fy - 1, Iy, Nfy) : 0.0, 1.0, yr ? w1d(fy + 1, Iy, Nfy) : 0.0};
+  const double wz[3] = {zl ? w1d(fz - 1, Iz, Nfz) : 0.0, 1.0, zr ? w1d(fz + 1, Iz, Nfz) : 0.0};
+  double acc[NQ] = {};  // the weights are powers of two: their products are exact in any order
 #pragma unroll
-  for (int q = 0; q < 3; ++q) bc[3 * I + q] = (T)acc[q];
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      const double w = wy[b] * wz[c];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        acc[q] += w * wl * (double)v[9 * c + 3 * b][q];
+        acc[q] += w * (double)v[9 * c + 3 * b + 1][q];
+        acc[q] += w * wr * (double)v[9 * c + 3 * b + 2][q];
+      }
+    }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) bc[t + q] = (T)acc[q];
   if (fs.d) {  // the coarse level's first Chebyshev step from x = 0 (as k_cheb_zero)
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const T v = fs.c2 * (fs.dinv[3 * I + q] * (T)acc[q]);
-      fs.d[3 * I + q] = v;
-      fs.x[3 * I + q] = v;
+    for (int q = 0; q < NQ; ++q) {
+      const T x = fs.c2 * (fs.dinv[t + q] * (T)acc[q]);
+      fs.d[t + q] = x;
+      fs.x[t + q] = x;
     }
   }
 }
 
-template <typename T>
+template <typename T, int NQ>
 __global__ __launch_bounds__(NT) void k_restrict(const T *__restrict__ rf, int Nfx, int Nfy,
                                                  int Nfz, T *__restrict__ bc, int Ncx, int Ncy,
                                                  int Ncz, FirstStep<T> fs)
 {
-  restrict_block<T>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, blockIdx.x);
+  restrict_block<T, NQ>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, blockIdx.x);
 }
 
+// a thread per DOF, whatever the entries' grids: 1.2 us less per launch on 12 instances' levels of
+// up to 4,000 nodes, 0.3 more on their 39,000
 template <typename T>
 __global__ __launch_bounds__(NT) void k_restrict_batch(const RestrictLaunch<T> *__restrict__ tab,
                                                        const int *__restrict__ b0, int n)
 {
   const int e = batch_entry(b0, n, blockIdx.x);
   const RestrictLaunch<T> L = tab[e];
-  restrict_block<T>(L.rf, L.Nfx, L.Nfy, L.Nfz, L.bc, L.Ncx, L.Ncy, L.Ncz, L.fs, blockIdx.x - b0[e]);
+  restrict_block<T, 1>(L.rf, L.Nfx, L.Nfy, L.Nfz, L.bc, L.Ncx, L.Ncy, L.Ncz, L.fs, blockIdx.x - b0[e]);
 }
 
 // x_f(i) += sum over coarse parents J of w(i,J) x_c(J)  (P x_c)
@@ -641,13 +661,19 @@ void cheb_zero_from64(hipStream_t s, const double *b64, float *b32, const float 
   TOFE_LAUNCH_CHECK();
 }
 
+// coarse nodes x vectors from which the restriction takes a thread per node: 72,000 take 6.5 us per
+// node and 6.1 per DOF, 78,000 7.0 and 7.3
+constexpr int64_t kRestrictNode = 75000;
+
 template <typename T>
 void restrict_op(hipStream_t s, const T *rf, int Nfx, int Nfy, int Nfz, T *bc, int Ncx, int Ncy,
                  int Ncz, const FirstStep<T> &fs, int nvec)
 {
   const int64_t ncn = (int64_t)Ncx * Ncy * Ncz;
-  k_restrict<T><<<dim3((unsigned)((ncn + NT - 1) / NT), nvec), dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc,
-                                                                           Ncx, Ncy, Ncz, fs);
+  const bool node = ncn * nvec >= kRestrictNode;
+  const dim3 grid((unsigned)(((node ? 1 : 3) * ncn + NT - 1) / NT), nvec);
+  if (node) k_restrict<T, 3><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs);
+  else k_restrict<T, 1><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs);
   TOFE_LAUNCH_CHECK();
 }
 

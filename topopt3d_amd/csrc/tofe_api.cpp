@@ -789,7 +789,7 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       d.rf = lv.r.p; d.Nfx = gf.Nx; d.Nfy = gf.Ny; d.Nfz = gf.Nz;
       d.bc = LV[l + 1]->b.p; d.Ncx = gc.Nx; d.Ncy = gc.Ny; d.Ncz = gc.Nz;
       d.fs = fs;
-      d.nblocks = (int)((gc.nn() + 255) / 256);
+      d.nblocks = (int)((gc.ndof() + 255) / 256);
       rec_push(c, batch_key(BK_RESTRICT, sizeof(T) == 4), d, d.nblocks);
     } else {
       restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec);
