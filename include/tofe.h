@@ -245,6 +245,14 @@ int tofe_stability_terms(tofe_ctx *ctx, const double *phi, int nvec, double *pks
 int tofe_element_bilinear(tofe_ctx *ctx, const double *A, int nvec, const double *B,
                           double *out);
 
+/* Eigenvalue sensitivities dmu_j/dx of the nev buckling modes (mu, K-normalised rows of phi) in
+ * the displacement state U of tofe_set_stress: the terms above, the adjoint solves (rtol, maxit; its
+ * and reason as in tofe_solve_dev, may be NULL) and Chain_Filter (Buckling.cpp:130-262) without
+ * leaving the device.  d_dmudx (nev * nelem) is left alone if a solve fails.  mu is host memory. */
+int tofe_buckling_sensitivity_dev(tofe_ctx *ctx, const double *d_U, const double *mu,
+                                  const double *d_phi, int nev, double rtol, int maxit,
+                                  double *d_dmudx, int *its, int *reason);
+
 /* Z = M^-1 R, one multigrid V-cycle; PCApply of the KUF preconditioner
  * (LOPGMRES.cpp:125). */
 int tofe_pc_apply(tofe_ctx *ctx, const double *R, double *Z, int nrhs);

@@ -46,7 +46,8 @@ EXPORTS = (
     "tofe_apply_M_dev", "tofe_element_quadratic", "tofe_petsc_vec_write", "tofe_petsc_vec_read",
     "tofe_petsc_aij_write", "tofe_petsc_aij_read", "tofe_mesh_out", "tofe_print_vals",
     "tofe_set_stress", "tofe_set_stress_dev", "tofe_apply_Ks", "tofe_apply_Ks_dev",
-    "tofe_stability_terms", "tofe_element_bilinear", "tofe_compliance_noalloc",
+    "tofe_stability_terms", "tofe_element_bilinear", "tofe_buckling_sensitivity_dev",
+    "tofe_compliance_noalloc",
     "tofe_set_mass_form", "tofe_autotune", "tofe_batch_create", "tofe_batch_destroy",
     "tofe_batch_last_error", "tofe_batch_solve_dev", "tofe_batch_get_stats", "tofe_set_springs",
 )
@@ -156,6 +157,8 @@ def lib():
         "tofe_apply_Ks_dev": ([vp, vp, vp, C.c_int], C.c_int),
         "tofe_stability_terms": ([vp, dp, C.c_int, dp, dp], C.c_int),
         "tofe_element_bilinear": ([vp, dp, C.c_int, dp, dp], C.c_int),
+        "tofe_buckling_sensitivity_dev": ([vp, vp, dp, vp, C.c_int, C.c_double, C.c_int, vp, ip, ip],
+                                          C.c_int),
         "tofe_set_mass_form": ([vp, C.c_int], C.c_int),
         "tofe_set_springs": ([vp, dp], C.c_int),
         "tofe_autotune": ([vp, C.c_int, ip, i64p], C.c_int),
@@ -439,6 +442,15 @@ class Context:
         r = np.empty((nvec, self.ndof)) if rhs else None
         self._check(lib().tofe_stability_terms(self.h, _dp(phi), nvec, _dp(q), _dp(r)))
         return q, r
+
+    def buckling_sensitivity_dev(self, U_ptr, mu, phi_ptr, g_ptr, rtol=1e-10, maxit=2000):
+        """dmu_j/dx of the modes (mu, phi) into g (nev, nelem); U, phi and g in device memory."""
+        mu = _f64(mu)
+        its, reason = C.c_int(), C.c_int()
+        self._check(lib().tofe_buckling_sensitivity_dev(
+            self.h, C.c_void_p(U_ptr), _dp(mu), C.c_void_p(phi_ptr), mu.size, rtol, maxit,
+            C.c_void_p(g_ptr), C.byref(its), C.byref(reason)))
+        return its.value, reason.value
 
     def element_bilinear(self, A, B):
         A, B = _f64(A), _f64(B)

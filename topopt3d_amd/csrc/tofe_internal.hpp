@@ -539,8 +539,12 @@ void stress_h(hipStream_t s, const double *U, int nx, int ny, int nz, const Shap
               double *H);
 void ks_quad(hipStream_t s, const double *H, const double *phi, int nx, int ny, int nz,
              int64_t ndof, int nvec, double *q);
-void stab_rhs(hipStream_t s, const double *phi, const double *Es, const uint8_t *fix, int nx,
+void stab_rhs(hipStream_t s, const double *phi, int nvec, const double *Es, const uint8_t *fix, int nx,
               int ny, int nz, const ShapeData &sd, double *r);
+// element gradients of nvec buckling eigenvalues mu (host values), before the filter
+void buckling_grad(hipStream_t s, const double *H, const double *phi, const double *V, const double *U,
+                   const double *KE, const double *dEdz, const double *dEsdz, const double *mu, int nvec,
+                   int nx, int ny, int nz, int64_t ndof, double *g);
 void elem_bilinear(hipStream_t s, const double *A, const double *B, const double *KE, int nx,
                    int ny, int nz, int64_t ndof, int nvec, double *out);
 void mass_diag(hipStream_t s, const double *V, int nx, int ny, int nz, double m0,

@@ -192,21 +192,17 @@ def buckling_sensitivities(ctx, U, mu, phi, rtol=1e-10, maxit=2000):
     tensor; U the displacement, a CUDA tensor): (nev, nelem) array, Buckling.cpp:130-262
     per eigenvalue, filter chain rule included."""
     torch = _torch()
-    phi_h = phi.cpu().numpy()
-    U_h = U.cpu().numpy()
-    nev = phi_h.shape[0]
-    pksp, rhs = ctx.stability_terms(phi_h)
-    pkp, _ = ctx.element_quadratic(phi_h, mass=False)
-    rhs_d = torch.from_numpy(np.ascontiguousarray(rhs)).to(U.device)
-    V = torch.zeros_like(rhs_d)
-    its, reason = ctx.solve_dev(rhs_d.data_ptr(), V.data_ptr(), nrhs=nev, rtol=rtol, maxit=maxit)
+    nev = phi.shape[0]
+    phi = phi.to(U.device, torch.float64).contiguous()
+    U = U.to(torch.float64).contiguous()
+    if phi.numel() != nev * ctx.ndof or U.numel() < ctx.ndof:
+        raise ValueError(f"expected {ctx.ndof} values per mode and displacement, got modes "
+                         f"{tuple(phi.shape)} and displacement {tuple(U.shape)}")
+    g = torch.empty((nev, ctx.nelem), dtype=torch.float64, device=U.device)
+    torch.cuda.current_stream(U.device).synchronize()  # phi and U are formed
+    _, reason = ctx.buckling_sensitivity_dev(U.data_ptr(), [float(mu[j]) for j in range(nev)],
+                                             phi.data_ptr(), g.data_ptr(), rtol=rtol, maxit=maxit)
     if reason < 0:
         raise RuntimeError(f"adjoint solves did not converge (reason {reason})")
-    vku = ctx.element_bilinear(V.cpu().numpy(), U_h)
-    dEdz = ctx.field(_lib.FIELD_DEDZ)
-    dEsdz = ctx.field(_lib.FIELD_DESDZ)
-    g = np.empty((nev, ctx.nelem))
-    for j in range(nev):
-        gj = -dEsdz * pksp[j] - mu[j] * dEdz * pkp[j] + dEdz * vku[j]
-        g[j] = ctx.chain_filter(None, gj)[1]
-    return g
+    out = torch.empty(g.shape, dtype=g.dtype, pin_memory=True)
+    return out.copy_(g).numpy()
