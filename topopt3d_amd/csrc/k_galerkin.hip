@@ -66,74 +66,126 @@ __device__ inline int elem_form(int ex, int nel, int Nf)
 // Per direction the candidate elements are ex = 2 I - 2 + d, d = 0..3 (window start
 // I - 1 + d / 2); both nodes lie in the window for d = 0..3 (D = 0), 2..3 (D = +1) or
 // 0..1 (D = -1), so positions, local node indices and the interpolation form of a regular
-// element are compile-time constants and its Q^T KE Q block comes through uniform
-// (scalar) loads.  Elements with a Dirichlet DOF (their own masked matrix) and the last
+// element follow from the window position alone and its Q^T KE Q block is the same for
+// every node.  Elements with a Dirichlet DOF (their own masked matrix) and the last
 // element of a grid with an even node count (single-parent form) add their own blocks.
 template <int O>
 __device__ inline void galerkin_block(const double *__restrict__ E, const int *__restrict__ emap,
                                       const double *__restrict__ KEC,
-                                      const double *__restrict__ KCm, const int (&Ic)[3],
-                                      const int (&nel)[3], const int (&Nf)[3], double (&acc)[9])
+                                      const double *__restrict__ KCm,
+                                      const uint8_t *__restrict__ fix, const int (&Ic)[3],
+                                      const int (&nel)[3], const int (&Nf)[3], double *sK, bool live,
+                                      double (&acc)[9])
 {
   constexpr int DX = O % 3 - 1, DY = (O / 3) % 3 - 1, DZ = O / 9 - 1;
   constexpr int X0 = DX > 0 ? 2 : 0, X1 = DX < 0 ? 2 : 4;
   constexpr int Y0 = DY > 0 ? 2 : 0, Y1 = DY < 0 ? 2 : 4;
   constexpr int Z0 = DZ > 0 ? 2 : 0, Z1 = DZ < 0 ? 2 : 4;
-  // Every element of the window is visited without a branch, so its loads are issued with
-  // the others: an element outside the grid (clamped load, weight 0) or of a special form adds
-  // w = 0 times its regular block, which leaves the sum unchanged, so the sum runs over the same
-  // elements in the same order as with those skipped.  A special element then adds its own
-  // block right away (a branch taken only near Dirichlet faces and at the last element of an
-  // axis with an even node count).
+  // Row after row of elements along x, the next row's map entries and moduli under way while one is
+  // summed.  Every element of a row is visited without a branch: one outside the grid (clamped
+  // load, weight 0) or of a special form adds 0 times its regular block, which leaves the sum
+  // unchanged, so the sum runs over the same elements in the same order as with those skipped.  A
+  // special element then adds its own block right away (a branch taken only near Dirichlet faces
+  // and at the last element of an axis with an even node count).  The regular blocks of the window
+  // come from LDS: through scalar loads, whose cache the table of 124 KB overflows, each row
+  // waited for the L2.  With the fixed-DOF masks below read at once instead of in up to 27 dependent
+  // steps, us: 637 coarse nodes 47.5 -> 32.7, 30,000 62 -> 40, 233,000 291 -> 227 (the chain of
+  // special elements' loads beside the Dirichlet faces remains; issuing them per row for all lanes:
+  // 40, 58 and 327, at 228 registers).
+  constexpr int NX = X1 - X0, NY = Y1 - Y0, NR = NY * (Z1 - Z0);
+  for (int v = threadIdx.x; v < NR * NX * 9; v += NT) {
+    const int pos = v / 9, q = v - 9 * pos;
+    const int dx = X0 + pos % NX, dy = Y0 + (pos / NX) % NY, dz = Z0 + pos / (NX * NY);
+    const int li = lidx(1 - (dx >> 1), 1 - (dy >> 1), 1 - (dz >> 1));
+    const int lj = lidx(1 - (dx >> 1) + DX, 1 - (dy >> 1) + DY, 1 - (dz >> 1) + DZ);
+    const int F = (dx & 1) + 3 * (dy & 1) + 9 * (dz & 1);
+    sK[v] = KEC[F * 576 + (3 * li + q / 3) * 24 + 3 * lj + q % 3];
+  }
+  __syncthreads();
+  if (!live) return;
+  int mn[NX];
+  double En[NX];
+  auto fetch = [&](int row) {
+    const int ez = 2 * Ic[2] - 2 + Z0 + row / NY, ey = 2 * Ic[1] - 2 + Y0 + row % NY;
+    const bool rin = ez >= 0 && ez < nel[2] && ey >= 0 && ey < nel[1];
 #pragma unroll
-  for (int dz = Z0; dz < Z1; ++dz) {
-    const int ez = 2 * Ic[2] - 2 + dz;
-    const bool zin = ez >= 0 && ez < nel[2];
+    for (int x = 0; x < NX; ++x) {
+      const int ex = 2 * Ic[0] - 2 + X0 + x;
+      const bool in = rin && ex >= 0 && ex < nel[0];
+      const int64_t e = in ? ex + (int64_t)nel[0] * (ey + (int64_t)nel[1] * ez) : 0;
+      const int m = emap[e];
+      En[x] = E[e];
+      mn[x] = in ? m : -2;
+    }
+  };
+  fetch(0);
+#pragma unroll 1
+  for (int row = 0; row < NR; ++row) {
+    const int dz = Z0 + row / NY, dy = Y0 + row % NY;
+    const int ez = 2 * Ic[2] - 2 + dz, ey = 2 * Ic[1] - 2 + dy;
+    // single-parent form: even position (even ex) that is the last element of a grid with an even
+    // node count
+    const bool sy = !(dy & 1) && (Nf[1] & 1) == 0 && ey == Nf[1] - 2;
+    const bool sz = !(dz & 1) && (Nf[2] & 1) == 0 && ez == Nf[2] - 2;
+    int m[NX];
+    double Ee[NX];
 #pragma unroll
-    for (int dy = Y0; dy < Y1; ++dy) {
-      const int ey = 2 * Ic[1] - 2 + dy;
-      const bool yin = ey >= 0 && ey < nel[1];
+    for (int x = 0; x < NX; ++x) {
+      m[x] = mn[x];
+      Ee[x] = En[x];
+    }
+    if (row + 1 < NR) fetch(row + 1);
 #pragma unroll
-      for (int dx = X0; dx < X1; ++dx) {
-        const int ex = 2 * Ic[0] - 2 + dx;
-        const bool in = zin && yin && ex >= 0 && ex < nel[0];
+    for (int x = 0; x < NX; ++x) {
+      const int dx = X0 + x;
+      const bool sx = !(dx & 1) && (Nf[0] & 1) == 0 && 2 * Ic[0] - 2 + dx == Nf[0] - 2;
+      const bool special = m[x] >= 0 || (m[x] == -1 && (sx || sy || sz));
+      const double w = (m[x] == -1 && !special) ? Ee[x] : 0.0;
+      const double *K = sK + (row * NX + x) * 9;
+#pragma unroll
+      for (int q = 0; q < 9; ++q) acc[q] = __builtin_fma(w, K[q], acc[q]);
+      if (special) {
         const int li = lidx(1 - (dx >> 1), 1 - (dy >> 1), 1 - (dz >> 1));
         const int lj = lidx(1 - (dx >> 1) + DX, 1 - (dy >> 1) + DY, 1 - (dz >> 1) + DZ);
-        const int64_t e = in ? ex + (int64_t)nel[0] * (ey + (int64_t)nel[1] * ez) : 0;
-        const int m = in ? emap[e] : -1;
-        const double Ee = E[e];
-        // single-parent form: even position (even ex) that is the last element of a grid
-        // with an even node count
-        const bool sx = !(dx & 1) && (Nf[0] & 1) == 0 && ex == Nf[0] - 2;
-        const bool sy = !(dy & 1) && (Nf[1] & 1) == 0 && ey == Nf[1] - 2;
-        const bool sz = !(dz & 1) && (Nf[2] & 1) == 0 && ez == Nf[2] - 2;
-        const bool special = in && (m >= 0 || sx || sy || sz);
-        const double w = (in && !special) ? Ee : 0.0;
-        const int F = (dx & 1) + 3 * (dy & 1) + 9 * (dz & 1);
-        const double *K = KEC + F * 576 + 3 * li * 24 + 3 * lj;
+        const int Fs = (sx ? 2 : (dx & 1)) + 3 * (sy ? 2 : (dy & 1)) + 9 * (sz ? 2 : (dz & 1));
+        // a masked element's block holds its E
+        const double *Ks = (m[x] < 0 ? KEC + Fs * 576 : KCm + (int64_t)m[x] * 576) + 3 * li * 24 + 3 * lj;
+        const double ws = m[x] < 0 ? Ee[x] : 1.0;
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-          for (int b = 0; b < 3; ++b) acc[a * 3 + b] = __builtin_fma(w, K[a * 24 + b], acc[a * 3 + b]);
-        if (special) {
-          if (m < 0) {
-            const int Fs = (sx ? 2 : (dx & 1)) + 3 * (sy ? 2 : (dy & 1)) + 9 * (sz ? 2 : (dz & 1));
-            const double *Ks = KEC + (int64_t)Fs * 576 + 3 * li * 24 + 3 * lj;
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-              for (int b = 0; b < 3; ++b) acc[a * 3 + b] = __builtin_fma(Ee, Ks[a * 24 + b], acc[a * 3 + b]);
-          } else {
-            const double *Km = KCm + (int64_t)m * 576 + 3 * li * 24 + 3 * lj;
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-              for (int b = 0; b < 3; ++b) acc[a * 3 + b] += Km[a * 24 + b];
-          }
-        }
+        for (int q = 0; q < 9; ++q) acc[q] = __builtin_fma(ws, Ks[(q / 3) * 24 + q % 3], acc[q]);
       }
     }
   }
+  // P^T M P: unit diagonal of the fixed fine DOFs that both nodes interpolate to, per axis
+  // 2 I - 1 .. 2 I + 1 (D = 0) or the one between the two nodes (and, at the end of an even grid,
+  // none: the weight is zero)
+  if (!fix) return;
+  constexpr int FX = DX ? 1 : 3, FY = DY ? 1 : 3, FZ = DZ ? 1 : 3;
+  uint8_t fm[FX * FY * FZ];
+  double wf[FX * FY * FZ];
+#pragma unroll
+  for (int z = 0; z < FZ; ++z)
+#pragma unroll
+    for (int y = 0; y < FY; ++y)
+#pragma unroll
+      for (int x = 0; x < FX; ++x) {
+        const int i[3] = {2 * Ic[0] + (DX ? DX : x - 1), 2 * Ic[1] + (DY ? DY : y - 1), 2 * Ic[2] + (DZ ? DZ : z - 1)};
+        const int Dd[3] = {DX, DY, DZ};
+        bool in = true;
+        double wt = 1.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          in = in && i[d] >= 0 && i[d] < Nf[d];
+          wt *= w1d(i[d], Ic[d], Nf[d]) * w1d(i[d], Ic[d] + Dd[d], Nf[d]);
+        }
+        const int q = x + FX * (y + FY * z);
+        fm[q] = fix[in ? i[0] + (int64_t)Nf[0] * (i[1] + (int64_t)Nf[1] * i[2]) : 0];
+        wf[q] = in ? wt : 0.0;
+      }
+#pragma unroll
+  for (int q = 0; q < FX * FY * FZ; ++q)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) acc[a * 4] += ((fm[q] >> a) & 1) ? wf[q] : 0.0;
 }
 
 // One thread per (coarse node I, coarse offset o >= 13); the transposed block goes to
@@ -172,66 +224,39 @@ __global__ __launch_bounds__(NT) void k_galerkin_fine(const double *__restrict__
   const int Nc[3] = {(Nf[0] + 1) / 2, (Nf[1] + 1) / 2, (Nf[2] + 1) / 2};
   const int64_t ncn = (int64_t)Nc[0] * Nc[1] * Nc[2];
   // grid: x over the coarse nodes, y over the 14 upper offsets
+  __shared__ double sK[576];
   const int64_t I = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (I >= ncn) return;
+  bool live = I < ncn;
   const int o = 13 + (int)blockIdx.y;
   const int D[3] = {o % 3 - 1, (o / 3) % 3 - 1, o / 9 - 1};
   int Ic[3];
-  node_ijk(I, Nc[0], Nc[1], Ic[0], Ic[1], Ic[2]);
+  node_ijk(live ? I : 0, Nc[0], Nc[1], Ic[0], Ic[1], Ic[2]);
   int Jc[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     Jc[d] = Ic[d] + D[d];
-    if (Jc[d] < 0 || Jc[d] >= Nc[d]) return;
+    if (Jc[d] < 0 || Jc[d] >= Nc[d]) live = false;  // no such neighbour
   }
   double acc[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) acc[q] = 0.0;
   switch (o) {
-    case 13: galerkin_block<13>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 14: galerkin_block<14>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 15: galerkin_block<15>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 16: galerkin_block<16>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 17: galerkin_block<17>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 18: galerkin_block<18>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 19: galerkin_block<19>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 20: galerkin_block<20>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 21: galerkin_block<21>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 22: galerkin_block<22>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 23: galerkin_block<23>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 24: galerkin_block<24>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    case 25: galerkin_block<25>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
-    default: galerkin_block<26>(E, emap, KEC, KCm, Ic, nel, Nf, acc); break;
+    case 13: galerkin_block<13>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 14: galerkin_block<14>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 15: galerkin_block<15>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 16: galerkin_block<16>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 17: galerkin_block<17>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 18: galerkin_block<18>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 19: galerkin_block<19>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 20: galerkin_block<20>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 21: galerkin_block<21>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 22: galerkin_block<22>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 23: galerkin_block<23>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 24: galerkin_block<24>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    case 25: galerkin_block<25>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
+    default: galerkin_block<26>(E, emap, KEC, KCm, fix, Ic, nel, Nf, sK, live, acc); break;
   }
-  // P^T M P: unit diagonal of the fixed fine DOFs
-  if (fix) {
-    int il[3][3], cn[3];
-    double wl[3][3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      int c = 0;
-      for (int i = 2 * Ic[d] - 1; i <= 2 * Ic[d] + 1; ++i) {
-        if (i < 0 || i >= Nf[d]) continue;
-        const double w = w1d(i, Ic[d], Nf[d]) * w1d(i, Jc[d], Nf[d]);
-        if (w == 0.0) continue;
-        il[d][c] = i;
-        wl[d][c] = w;
-        ++c;
-      }
-      cn[d] = c;
-    }
-    for (int cz = 0; cz < cn[2]; ++cz)
-      for (int cy = 0; cy < cn[1]; ++cy)
-        for (int cx = 0; cx < cn[0]; ++cx) {
-          const int64_t n = il[0][cx] + (int64_t)Nf[0] * (il[1][cy] + (int64_t)Nf[1] * il[2][cz]);
-          const uint8_t fm = fix[n];
-          if (!fm) continue;
-          const double w = wl[0][cx] * wl[1][cy] * wl[2][cz];
-#pragma unroll
-          for (int a = 0; a < 3; ++a)
-            if ((fm >> a) & 1) acc[a * 4] += w;
-        }
-  }
+  if (!live) return;
 #pragma unroll
   for (int q = 0; q < 9; ++q) Sc[(int64_t)(o * 9 + q) * ncn + I] = acc[q];
   if (o != 13) {
