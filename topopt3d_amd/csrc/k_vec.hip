@@ -225,8 +225,12 @@ __device__ __forceinline__ void restrict_block(const T *__restrict__ rf, int Nfx
 template <typename T, int NQ>
 __global__ __launch_bounds__(NT) void k_restrict(const T *__restrict__ rf, int Nfx, int Nfy,
                                                  int Nfz, T *__restrict__ bc, int Ncx, int Ncy,
-                                                 int Ncz, FirstStep<T> fs)
+                                                 int Ncz, FirstStep<T> fs, ReduceTail tail)
 {
+  if (tail.partial && blockIdx.x == gridDim.x - 1) {
+    reduce_final_block(tail.partial, tail.nparts, tail.out, tail.post, tail.scal, tail.mirror);
+    return;
+  }
   restrict_block<T, NQ>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, blockIdx.x);
 }
 
@@ -667,13 +671,14 @@ constexpr int64_t kRestrictNode = 75000;
 
 template <typename T>
 void restrict_op(hipStream_t s, const T *rf, int Nfx, int Nfy, int Nfz, T *bc, int Ncx, int Ncy,
-                 int Ncz, const FirstStep<T> &fs, int nvec)
+                 int Ncz, const FirstStep<T> &fs, int nvec,
+                 const ReduceTail &tail)
 {
   const int64_t ncn = (int64_t)Ncx * Ncy * Ncz;
   const bool node = ncn * nvec >= kRestrictNode;
-  const dim3 grid((unsigned)(((node ? 1 : 3) * ncn + NT - 1) / NT), nvec);
-  if (node) k_restrict<T, 3><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs);
-  else k_restrict<T, 1><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs);
+  const dim3 grid((unsigned)(((node ? 1 : 3) * ncn + NT - 1) / NT + (tail.partial ? 1 : 0)), nvec);
+  if (node) k_restrict<T, 3><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
+  else k_restrict<T, 1><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
   TOFE_LAUNCH_CHECK();
 }
 
@@ -815,7 +820,7 @@ void lz_p(hipStream_t s, const LzTab<T> &tab, int k)
   template void dot_partial<T>(hipStream_t, const T *, const T *, int64_t, double *, int);  \
   template void cheb_zero<T>(hipStream_t, const T *, const T *, T, T *, T *, int64_t, int); \
   template void restrict_op<T>(hipStream_t, const T *, int, int, int, T *, int, int, int,        \
-                               const FirstStep<T> &, int);                                    \
+                               const FirstStep<T> &, int, const ReduceTail &);                \
   template void prolong_add<T>(hipStream_t, const T *, int, int, int, T *, int, int, int, int); \
   template void restrict_batch<T>(hipStream_t, const RestrictLaunch<T> *, const int *, int, int, int); \
   template void prolong_batch<T>(hipStream_t, const ProlongLaunch<T> *, const int *, int, int, int); \

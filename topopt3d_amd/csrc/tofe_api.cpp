@@ -268,6 +268,7 @@ struct tofe_ctx {
 
   DBuf<double> vr, vz, vp, vq, vF, vU;
   DBuf<float> vr32, vz32;
+  ReduceTail tail;  // of a solve: goes with the next restriction
   DBuf<double> ebuf, ebuf2;
   DBuf<double> sens_r, sens_v;  // buckling sensitivities: adjoint right-hand sides and solutions
 
@@ -793,7 +794,10 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       d.nblocks = (int)((gc.ndof() + 255) / 256);
       rec_push(c, batch_key(BK_RESTRICT, sizeof(T) == 4), d, d.nblocks);
     } else {
-      restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec);
+      restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec,
+                     c->tail);
+      if (c->tail.partial) TOFE_HIP(hipEventRecord(c->ev_scal, s));  // the solve's scalars are on the host
+      c->tail = ReduceTail();
     }
     cur[l] = xc;
     oth[l] = xo;
@@ -948,6 +952,7 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
   double *h = hv.data();
   auto H = [&](int v, int slot) { return h[(size_t)v * SL_COUNT + slot]; };
 
+  c->tail = ReduceTail();
   if (c->frozen_dirty) {
     set_frozen(s, c->scal.p, nvec, 0ull);
     c->frozen_dirty = false;
@@ -1025,23 +1030,30 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
       level_apply<double>(c, 0, p, EPI_APPLY_DOT2, ep);
       fcg_update_r(s, r, q, n, c->partial.p, c->partial2.p, nfb, c->scal.p, c->partial3.p, first,
                    nvec);
-      x_pending = true;
-      reduce_final(s, c->partial3.p, kRedBlocks, c->scal.p + SL_RR, POST_NONE, c->scal.p, nvec,
-                   c->hscal_dev);
     } else {
       level_apply<double>(c, 0, p, EPI_APPLY_DOT, ep);
       cg_update_r(s, r, q, n, c->partial.p, nfb, c->scal.p, c->partial3.p, nvec, first64);
-      x_pending = true;
-      reduce_final(s, c->partial3.p, kRedBlocks, c->scal.p + SL_RR, POST_RR_CG, c->scal.p, nvec,
-                   c->hscal_dev);
     }
-    // the reduction has written this iteration's scalars to the mapped host copy: no copy
-    // launch between it and the next direction's kernels
-    TOFE_HIP(hipEventRecord(c->ev_scal, s));
+    x_pending = true;
     bool ahead = k + 1 < maxit;
     for (int v = 0; v < nvec && ahead; ++v)
       if (!reason[v] && !(rn_prev[v] * std::min(rate[v], 1.0) > 3 * ttol[v])) ahead = false;
-    if (ahead) next_direction();
+    // r.r, which no kernel before the next step waits for, and this iteration's scalars to the mapped
+    // host copy: with the next direction's first restriction if that is queued before the host reads
+    // them, else now.  (Step of 48x24x24 elements with a launch of its own 114.0 us, this way 111.7;
+    // 87x45x39 mixed 151.6 and 150.1, 192x96x96 mixed 538 and 536.)  No copy launch between it and the
+    // next direction's kernels.
+    ReduceTail rr;
+    rr.partial = c->partial3.p; rr.nparts = kRedBlocks; rr.post = flex ? POST_NONE : POST_RR_CG;
+    rr.out = c->scal.p + SL_RR; rr.scal = c->scal.p; rr.mirror = c->hscal_dev;
+    if (ahead && c->L > 1) {
+      c->tail = rr;
+      next_direction();
+    } else {
+      reduce_final(s, rr.partial, rr.nparts, rr.out, rr.post, rr.scal, nvec, rr.mirror);
+      TOFE_HIP(hipEventRecord(c->ev_scal, s));
+      if (ahead) next_direction();
+    }
     scal_wait(c, h, nvec);
     ++k;
     unsigned long long newly = 0;

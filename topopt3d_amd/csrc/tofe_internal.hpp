@@ -293,9 +293,17 @@ struct FirstStep {
   T c2 = 0;
   T *d = nullptr, *x = nullptr;
 };
+// A reduce_final that rides on another kernel's launch, as one block more per vector (partial null:
+// none).
+struct ReduceTail {
+  const double *partial = nullptr;
+  int nparts = 0, post = 0;
+  double *out = nullptr, *scal = nullptr, *mirror = nullptr;
+};
 template <typename T>
 void restrict_op(hipStream_t s, const T *rf, int Nfx, int Nfy, int Nfz, T *bc, int Ncx, int Ncy,
-                 int Ncz, const FirstStep<T> &fs = FirstStep<T>(), int nvec = 1);
+                 int Ncz, const FirstStep<T> &fs = FirstStep<T>(), int nvec = 1,
+                 const ReduceTail &tail = ReduceTail());
 template <typename T>
 void prolong_add(hipStream_t s, const T *xc, int Ncx, int Ncy, int Ncz, T *xf, int Nfx, int Nfy,
                  int Nfz, int nvec = 1);
