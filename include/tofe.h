@@ -344,9 +344,9 @@ int tofe_time_kernels(tofe_ctx *ctx, int start, tofe_kernel_time *out, int max_k
 /* Launch shapes from measurement (no reference counterpart: PETSc has no such knob): for
  * the precision of the last assemble, times the fine operator's Chebyshev step over
  * candidate z-chunk lengths and every coarse level's stencil kernel one thread per node
- * and one per DOF (nrep launches each), keeps the fastest chunk length and the node-count
- * threshold below which levels run per DOF that minimises their summed time.  Outputs
- * (may be NULL): the chunk length and the threshold. */
+ * and split over four wavefronts (nrep launches each), keeps the fastest chunk length and
+ * the node-count threshold below which levels run split that minimises their summed time.
+ * Outputs (may be NULL): the chunk length and the threshold. */
 int tofe_autotune(tofe_ctx *ctx, int nrep, int *fine_zlen, int64_t *split_nodes);
 
 /* ---- batches of independent instances ---------------------------------------------

@@ -1703,7 +1703,7 @@ double time_level_op(tofe_ctx *c, int level, bool f32, Epi epi, int nrep)
 
 // Launch shapes of the current precision's operators from measurement: the fine operator's
 // z-chunk length (element-centric form) over candidate lengths, and the node-count
-// threshold below which a stencil level runs one thread per DOF, chosen to minimise the
+// threshold below which a stencil level runs in the split form, chosen to minimise the
 // summed Chebyshev-step time of the coarse levels.  The chosen shapes stay in the context.
 void autotune(tofe_ctx *c, int nrep, int *zlen_out, int64_t *split_out)
 {
