@@ -270,7 +270,9 @@ __global__ __launch_bounds__(NT) void k_galerkin_fine(const double *__restrict__
 
 // Jacobi diagonal of the fine K with Dirichlet rows: sum over the node's elements in
 // ascending order of the rounded products E_e KE_ii (the assembly order of
-// FEAnalysis.cpp:448-464), 1 on fixed DOFs, and diag <= 0 -> 1 (476-484).
+// FEAnalysis.cpp:448-464), 1 on fixed DOFs, and diag <= 0 -> 1 (476-484).  A thread per node, its
+// eight moduli loaded once and at once: per DOF, element by element, the loads set the time (1.8M
+// nodes 58 -> 36 us, 4,200 nodes 4.8 -> 4.1).
 __global__ void k_fine_diag(const double *__restrict__ E, const double *__restrict__ KE,
                             const uint8_t *__restrict__ fix, int nx, int ny, int nz,
                             double *diag, double *dinv, const double *__restrict__ spk)
@@ -278,29 +280,35 @@ __global__ void k_fine_diag(const double *__restrict__ E, const double *__restri
 #pragma clang fp contract(off)
   const int Nx = nx + 1, Ny = ny + 1, Nz = nz + 1;
   const int64_t nn = (int64_t)Nx * Ny * Nz;
-  const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (t >= 3 * nn) return;
-  const int64_t n = t / 3;
-  const int a = (int)(t - 3 * n);
+  const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
+  if (n >= nn) return;
   int i, j, k;
   node_ijk(n, Nx, Ny, i, j, k);
-  double s = 0.0;
-  for (int ez = k - 1; ez <= k; ++ez) {
-    if (ez < 0 || ez >= nz) continue;
-    for (int ey = j - 1; ey <= j; ++ey) {
-      if (ey < 0 || ey >= ny) continue;
-      for (int ex = i - 1; ex <= i; ++ex) {
-        if (ex < 0 || ex >= nx) continue;
-        const int l = lidx(i - ex, j - ey, k - ez);
-        s = s + E[ex + (int64_t)nx * (ey + (int64_t)ny * ez)] * KE[(3 * l + a) * 25];
-      }
-    }
+  // the (up to eight) elements' moduli at once: an element outside the grid reads element 0
+  double Ee[8];
+  bool in[8];
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    const int ex = i - 1 + (m & 1), ey = j - 1 + ((m >> 1) & 1), ez = k - 1 + (m >> 2);
+    in[m] = ex >= 0 && ex < nx && ey >= 0 && ey < ny && ez >= 0 && ez < nz;
+    Ee[m] = E[in[m] ? ex + (int64_t)nx * (ey + (int64_t)ny * ez) : 0];
   }
-  if (spk) s = s + spk[t];  // MatDiagonalSet(K, spKVec, ADD_VALUES), FEAnalysis.cpp:471
-  if (fix && ((fix[n] >> a) & 1)) s = 1.0;
-  if (!(s > 0)) s = 1.0;
-  diag[t] = s;
-  dinv[t] = 1.0 / s;
+  const uint8_t fm = fix ? fix[n] : 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    double s = 0.0;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int l = lidx(1 - (m & 1), 1 - ((m >> 1) & 1), 1 - (m >> 2));
+      const double v = s + Ee[m] * KE[(3 * l + a) * 25];
+      s = in[m] ? v : s;
+    }
+    if (spk) s = s + spk[3 * n + a];  // MatDiagonalSet(K, spKVec, ADD_VALUES), FEAnalysis.cpp:471
+    if ((fm >> a) & 1) s = 1.0;
+    if (!(s > 0)) s = 1.0;
+    diag[3 * n + a] = s;
+    dinv[3 * n + a] = 1.0 / s;
+  }
 }
 
 // Sc(I, I + o) += sum over fine nodes f shared by the supports of I and I + o of
@@ -380,8 +388,8 @@ void fine_diag(hipStream_t s, const double *E, const double *KE, const uint8_t *
                int nz, double *diag, double *dinv, const double *spk)
 {
   const int64_t nn = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-  k_fine_diag<<<dim3((unsigned)((3 * nn + NT - 1) / NT)), dim3(NT), 0, s>>>(E, KE, fix, nx, ny, nz,
-                                                                          diag, dinv, spk);
+  k_fine_diag<<<dim3((unsigned)((nn + NT - 1) / NT)), dim3(NT), 0, s>>>(E, KE, fix, nx, ny, nz, diag, dinv,
+                                                                        spk);
   TOFE_LAUNCH_CHECK();
 }
 
