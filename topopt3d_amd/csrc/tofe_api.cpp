@@ -2612,7 +2612,7 @@ int tofe_buckling_sensitivity_dev(tofe_ctx *c, const double *dU, const double *m
     const size_t nd = (size_t)c->ndof * nev, ne = (size_t)c->ne * nev;
     // kept with the context; the gradients before the filter take the right-hand sides' place.  With
     // the element terms, right-hand sides and solutions passing through host arrays half of a call was
-    // copies, allocations and host sums (64x32x32, 6 modes: 10.7 ms, of which the GPU worked 5.2; 3.7).
+    // copies, allocations and host sums (64x32x32, 6 modes: 10.7 ms, of which the GPU worked 5.2; 3.8).
     if (c->sens_r.n < std::max(nd, ne)) c->sens_r.alloc(std::max(nd, ne));
     if (c->sens_v.n < nd) c->sens_v.alloc(nd);
     const tofe_desc &d = c->desc;

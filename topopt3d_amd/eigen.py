@@ -204,5 +204,4 @@ def buckling_sensitivities(ctx, U, mu, phi, rtol=1e-10, maxit=2000):
                                              phi.data_ptr(), g.data_ptr(), rtol=rtol, maxit=maxit)
     if reason < 0:
         raise RuntimeError(f"adjoint solves did not converge (reason {reason})")
-    out = torch.empty(g.shape, dtype=g.dtype, pin_memory=True)
-    return out.copy_(g).numpy()
+    return g.cpu().numpy()
