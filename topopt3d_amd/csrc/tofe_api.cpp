@@ -827,15 +827,19 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       ep.nvec = nvec;
       ep.keep_d = k + 1 < nu2;
       if (l == 0 && k == nu2 - 1 && io && io->x64) {
-        ep.xout64 = mixed_io && !io->want_z32 ? io->x64 : nullptr;  // FP64: xo is x0 here
+        ep.xout64 = mixed_io && !io->want_z32 ? io->x64 : nullptr;
         ep.q64 = io->q64; ep.partial = io->partial;
         level_apply<T>(c, l, xc, EPI_CHEB_OUT, ep);
         io->fused_out = true;
-        if constexpr (sizeof(T) == 4)
+        if constexpr (sizeof(T) == 4) {
           if (io->want_z32) io->z32 = xo;
-        return;
+          return;
+        }
+        // FP64: xo is x0, or (odd nu_pre + nu_post with x_in_d, whose direction took a buffer's
+        // place) another buffer, which the copy below then takes there
+      } else {
+        level_apply<T>(c, l, xc, EPI_CHEB, ep);
       }
-      level_apply<T>(c, l, xc, EPI_CHEB, ep);
       std::swap(xc, xo);
     }
     cur[l] = xc;
