@@ -268,7 +268,6 @@ struct tofe_ctx {
 
   DBuf<double> vr, vz, vp, vq, vF, vU;
   DBuf<float> vr32, vz32;
-  ReduceTail tail;  // of a solve: goes with the next restriction
   DBuf<double> ebuf, ebuf2;
   DBuf<double> sens_r, sens_v;  // buckling sensitivities: adjoint right-hand sides and solutions
 
@@ -645,6 +644,7 @@ struct VcycleIO {
   // then writes it to the level's free FP32 buffer, returned in z32, instead of x64
   bool want_z32 = false;
   const float *z32 = nullptr;
+  ReduceTail tail;  // goes with the fine level's restriction; the context's ev_scal marks its end
 };
 
 // Whether the V-cycle's first two fine-level Chebyshev steps run as one launch (EPI_CHEB_FIRST): the
@@ -794,10 +794,9 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       d.nblocks = (int)((gc.ndof() + 255) / 256);
       rec_push(c, batch_key(BK_RESTRICT, sizeof(T) == 4), d, d.nblocks);
     } else {
-      restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec,
-                     c->tail);
-      if (c->tail.partial) TOFE_HIP(hipEventRecord(c->ev_scal, s));  // the solve's scalars are on the host
-      c->tail = ReduceTail();
+      const ReduceTail tail = l == 0 && io ? io->tail : ReduceTail();
+      restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec, tail);
+      if (tail.partial) TOFE_HIP(hipEventRecord(c->ev_scal, s));  // the solve's scalars are on the host
     }
     cur[l] = xc;
     oth[l] = xo;
@@ -855,9 +854,11 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
 
 // z = M^-1 r.  With q given, also the partial sums of z.q into c->partial;
 // returns how many there are.  With z32 given, a mixed V-cycle whose last step forms z.q may
-// leave z in FP32 instead (*z32 then points to it, else *z32 = null and z holds it).
+// leave z in FP32 instead (*z32 then points to it, else *z32 = null and z holds it).  tail: a
+// reduction for the V-cycle's first restriction to carry (more than one level).
 int precondition(tofe_ctx *c, const double *r, double *z, const double *q = nullptr,
-                 bool first_done = false, int nvec = 1, const float **z32 = nullptr)
+                 bool first_done = false, int nvec = 1, const float **z32 = nullptr,
+                 const ReduceTail &tail = ReduceTail())
 {
   const hipStream_t s = c->stream;
   if (z32) *z32 = nullptr;
@@ -865,6 +866,7 @@ int precondition(tofe_ctx *c, const double *r, double *z, const double *q = null
     VcycleIO io;
     io.b64 = r;
     io.first_done = first_done;
+    io.tail = tail;
     if (q && c->L > 1 && !c->fine_mfma) {
       io.x64 = z; io.q64 = q; io.partial = c->partial.p;
       io.want_z32 = z32 != nullptr;
@@ -880,6 +882,7 @@ int precondition(tofe_ctx *c, const double *r, double *z, const double *q = null
   } else {
     VcycleIO io;
     io.first_done = first_done;  // the CG residual update formed the first fine-level step
+    io.tail = tail;
     if (q && c->L > 1 && !c->fine_mfma) {
       io.x64 = z; io.q64 = q; io.partial = c->partial.p;
     }
@@ -956,7 +959,6 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
   double *h = hv.data();
   auto H = [&](int v, int slot) { return h[(size_t)v * SL_COUNT + slot]; };
 
-  c->tail = ReduceTail();
   if (c->frozen_dirty) {
     set_frozen(s, c->scal.p, nvec, 0ull);
     c->frozen_dirty = false;
@@ -1006,13 +1008,13 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
   // CG and flexible CG apply the iterate's update x += alpha p in the next search-direction
   // kernel, which reads p anyway; x_pending marks a step whose update is still owed
   bool x_pending = false;
-  auto next_direction = [&] {
+  auto next_direction = [&](const ReduceTail &tail = ReduceTail()) {
     if (flex) {
       const float *z32 = nullptr;
-      const int nparts = precondition(c, r, z, q, first.b32 != nullptr, nvec, &z32);
+      const int nparts = precondition(c, r, z, q, first.b32 != nullptr, nvec, &z32, tail);
       fcg_update_xp(s, p, z, z32, U, n, c->partial.p, nparts, c->scal.p, nvec);
     } else {
-      const int nparts = precondition(c, r, z, r, first64.d != nullptr, nvec);
+      const int nparts = precondition(c, r, z, r, first64.d != nullptr, nvec, nullptr, tail);
       cg_update_xp(s, p, z, U, n, c->partial.p, nparts, c->scal.p, nvec);
     }
     x_pending = false;
@@ -1051,8 +1053,7 @@ void solve_block(tofe_ctx *c, const double *F, double *U, int nvec, double rtol,
     rr.partial = c->partial3.p; rr.nparts = kRedBlocks; rr.post = flex ? POST_NONE : POST_RR_CG;
     rr.out = c->scal.p + SL_RR; rr.scal = c->scal.p; rr.mirror = c->hscal_dev;
     if (ahead && c->L > 1) {
-      c->tail = rr;
-      next_direction();
+      next_direction(rr);
     } else {
       reduce_final(s, rr.partial, rr.nparts, rr.out, rr.post, rr.scal, nvec, rr.mirror);
       TOFE_HIP(hipEventRecord(c->ev_scal, s));
