@@ -248,7 +248,9 @@ int tofe_element_bilinear(tofe_ctx *ctx, const double *A, int nvec, const double
 /* Eigenvalue sensitivities dmu_j/dx of the nev buckling modes (mu, K-normalised rows of phi) in
  * the displacement state U of tofe_set_stress: the terms above, the adjoint solves (rtol, maxit; its
  * and reason as in tofe_solve_dev, may be NULL) and Chain_Filter (Buckling.cpp:130-262) without
- * leaving the device.  d_dmudx (nev * nelem) is left alone if a solve fails.  mu is host memory. */
+ * leaving the device.  If a solve fails d_dmudx (nev * nelem) is left alone and reason is negative;
+ * without reason the call returns TOFE_ERR_NUMERIC.  mu is host memory.  The context keeps the
+ * right-hand sides and solutions, 2 * nev * max(ndof, nelem) doubles at most, until tofe_destroy. */
 int tofe_buckling_sensitivity_dev(tofe_ctx *ctx, const double *d_U, const double *mu,
                                   const double *d_phi, int nev, double rtol, int maxit,
                                   double *d_dmudx, int *its, int *reason);

@@ -2627,7 +2627,10 @@ int tofe_buckling_sensitivity_dev(tofe_ctx *c, const double *dU, const double *m
     int rs = 0;
     solve_dev(c, c->sens_r.p, c->sens_v.p, nev, rtol, maxit, its, &rs);
     if (reason) *reason = rs;
-    if (rs < 0) return;
+    if (rs < 0) {
+      if (!reason) throw Error(TOFE_ERR_NUMERIC, "adjoint solve failed, reason " + std::to_string(rs));
+      return;
+    }
     buckling_grad(c->stream, c->Hs.p, dphi, c->sens_v.p, dU, c->dKE.p, c->dEdz.p, c->dEsdz.p, mu, nev, d.nx,
                   d.ny, d.nz, c->ndof, c->sens_r.p);
     for (int j = 0; j < nev; ++j)
