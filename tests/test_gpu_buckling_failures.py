@@ -43,3 +43,24 @@ def test_failed_adjoint_solve_is_reported(tofe):
     rc = L.tofe_buckling_sensitivity_dev(*args, 2000, C.c_void_p(g.data_ptr()), None, None)
     assert rc == tofe.TOFE_OK and not (g == -7.0).any()
     ctx.close()
+
+
+def test_more_vectors_than_a_grid_axis_holds(tofe):
+    """70,001 vectors of a mesh of two elements: the adjoint right-hand sides of the first and the last
+    ones are those of a call of their own, bit for bit."""
+    print("case 70,001 vectors", flush=True)
+    nel, nvec = (2, 1, 1), 70001
+    fixed = np.zeros(36, np.uint8)
+    fixed[[0, 1, 2, 9, 10, 11]] = 1
+    ctx = tofe.Context(nel, rmin=1.0, mg_levels=1, fixed_dof=fixed)
+    ctx.set_design(np.array([0.3, 0.8]))
+    phi = np.random.default_rng(5).standard_normal((nvec, ctx.ndof))
+    U = np.random.default_rng(6).standard_normal(ctx.ndof)
+    ctx.set_stress(U)
+    q, r = ctx.stability_terms(phi)
+    for j in (0, 1, 65534, 65535, 65536, nvec - 1):
+        qj, rj = ctx.stability_terms(phi[j])
+        np.testing.assert_array_equal(r[j], rj[0])
+        np.testing.assert_array_equal(q[j], qj[0])
+        assert np.abs(rj).max() > 0
+    ctx.close()

@@ -17,6 +17,7 @@ namespace tofe {
 namespace {
 
 constexpr int NT = 256;
+constexpr int kGridY = 65535;  // vectors of one launch: a grid's second axis ends at 65,536 blocks
 
 struct BucklingMu {  // eigenvalues of one launch
   static constexpr int kMax = 32;
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(NT) void k_buckling_grad(const double *__restrict__
 // Adjoint right-hand side of eigenvector blockIdx.y (Buckling.cpp:150-191):
 // r_d = sum_{e holding d} Es_e sum_q (D B_q e_d) . tau_q(phi_e), fixed rows zero.
 // One thread per node; the node's elements in ascending order, each recomputing tau.  All vectors
-// in one launch: a vector alone leaves a wavefront per SIMD (6 of 71,000 nodes: 312 -> 164 us).
+// in one launch (up to kGridY): a vector alone leaves a wavefront per SIMD (6 of 71,000 nodes: 312 -> 164 us).
 __global__ __launch_bounds__(NT) void k_stab_rhs(const double *__restrict__ phi,
                                                  const double *__restrict__ Es,
                                                  const uint8_t *__restrict__ fix, int nx, int ny,
@@ -335,8 +336,12 @@ void stab_rhs(hipStream_t s, const double *phi, int nvec, const double *Es, cons
               int ny, int nz, const ShapeData &sd, double *r)
 {
   const int64_t nn = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-  k_stab_rhs<<<dim3(blocks_for(nn), nvec), dim3(NT), 0, s>>>(phi, Es, fix, nx, ny, nz, sd, r);
-  TOFE_LAUNCH_CHECK();
+  for (int j0 = 0; j0 < nvec; j0 += kGridY) {
+    const int nv = std::min(nvec - j0, kGridY);
+    k_stab_rhs<<<dim3(blocks_for(nn), nv), dim3(NT), 0, s>>>(phi + j0 * 3 * nn, Es, fix, nx, ny, nz, sd,
+                                                            r + j0 * 3 * nn);
+    TOFE_LAUNCH_CHECK();
+  }
 }
 
 void buckling_grad(hipStream_t s, const double *H, const double *phi, const double *V, const double *U,
