@@ -448,17 +448,25 @@ int fine_wht_blocks(const FineOp<T> &op)
   return wht_grid(op).nblocks;
 }
 
+// Several vectors, or the instances of a batch, fill the CUs with longer chunks, which form fewer
+// extra element layers: up to six planes (longer ones measured slower: a Chebyshev step on 16 vectors of
+// 160x80x80 670 us at 6, 717 at 14; a merged solve of 32 instances of 16 to 96 elements along x,
+// ms: with their own lengths 57.5 for four load cases each and 35.3 for one, this way 54.1 and
+// 34.4).  The chunk length does not show in the outputs, only in the
+// partial sums of the dot products, where each vector's stay those of its own launch.
+template <typename T>
+int fine_wht_shared_zlen(const FineOp<T> &op, Epi epi, int nvec)
+{
+  const bool sums = epi == EPI_APPLY_DOT || epi == EPI_APPLY_DOT2 || epi == EPI_CHEB_OUT;
+  if (sums || nvec <= 1 || op.ncu <= 0 || op.zlen >= 6) return op.zlen;
+  return std::min(6, fine_wht_zlen(op.nx, op.ny, op.nz, op.ncu, sizeof(T) == 8 ? kWhtHide64 : kWhtHide32,
+                                   nvec));
+}
+
 template <typename T, int EPI, int FORM>
 void launch_form(hipStream_t s, FineOp<T> op, const T *u, const EpiArgs<T> &ep)
 {
-  // Several vectors fill the CUs with longer chunks, which form fewer extra element layers: up to six
-  // planes (longer ones measured slower: a Chebyshev step on 16 vectors of 160x80x80 670 us at 6, 717
-  // at 14).  The chunk length does not show in the outputs, only in the partial sums of the dot
-  // products, where each vector's stay those of its own launch.
-  if constexpr (EPI != EPI_APPLY_DOT && EPI != EPI_APPLY_DOT2 && EPI != EPI_CHEB_OUT)
-    if (ep.nvec > 1 && op.ncu > 0 && op.zlen < 6)
-      op.zlen = std::min(6, fine_wht_zlen(op.nx, op.ny, op.nz, op.ncu,
-                                          sizeof(T) == 8 ? kWhtHide64 : kWhtHide32, ep.nvec));
+  op.zlen = fine_wht_shared_zlen(op, (Epi)EPI, ep.nvec);
   const WhtGrid g = wht_grid(op);
   k_fine_wht<T, EPI, FORM><<<dim3(g.nblocks, ep.nvec), dim3(NW), 0, s>>>(op, u, ep, g.tiles_x, g.tiles_y,
                                                                         g.nblocks, op.zlen);
@@ -537,6 +545,8 @@ template void fine_wht_batch<double>(hipStream_t, Epi, bool, const FineLaunch<do
                                      int, int, int);
 template void fine_wht_batch<float>(hipStream_t, Epi, bool, const FineLaunch<float> *, const int *,
                                     int, int, int);
+template int fine_wht_shared_zlen<double>(const FineOp<double> &, Epi, int);
+template int fine_wht_shared_zlen<float>(const FineOp<float> &, Epi, int);
 template int fine_wht_blocks<double>(const FineOp<double> &);
 template int fine_wht_blocks<float>(const FineOp<float> &);
 template void fine_wht<double>(hipStream_t, const FineOp<double> &, const double *, Epi, const EpiArgs<double> &);

@@ -156,6 +156,9 @@ struct RecOp {
 };
 struct Recorder {
   std::vector<RecOp> ops;
+  // the unfinished instances' nodes over this instance's: how many such instances the launches hold
+  double share = 1;
+  int vectors(int nvec) const { return (int)std::min(nvec * share, 1e6); }
 };
 
 }  // namespace
@@ -442,8 +445,9 @@ void level_record(tofe_ctx *c, int l, const T *u, Epi epi, const EpiArgs<T> &ep)
 {
   constexpr bool f32 = sizeof(T) == 4;
   if (l == 0) {
-    const FineOp<T> f = fine_of<T>(c);
+    FineOp<T> f = fine_of<T>(c);
     if (f.wht && !c->fine_mfma) {
+      f.zlen = fine_wht_shared_zlen<T>(f, epi, c->rec->vectors(ep.nvec));
       FineLaunch<T> d;
       d.op = f;
       d.u = u;
@@ -3142,8 +3146,12 @@ struct BatchProgram {
     batched = single = recorded = 0;
     const size_t n = ctx.size();
     std::vector<Recorder> rec(n);
+    double nodes = 0;
+    for (size_t i = 0; i < n; ++i)
+      if (live[i]) nodes += (double)ctx[i]->nn;
     for (size_t i = 0; i < n; ++i) {
       if (!live[i]) continue;
+      rec[i].share = nodes / (double)ctx[i]->nn;
       struct Stop {
         tofe_ctx *c;
         ~Stop() { c->rec = nullptr; }

@@ -102,6 +102,9 @@ constexpr int kWhtHide64 = 2, kWhtHide32 = 4;
 int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide, int nvec = 1);
 template <typename T>
 int fine_wht_blocks(const FineOp<T> &op);
+// chunk length of a launch that serves nvec vectors of this mesh, or as many nodes of several meshes
+template <typename T>
+int fine_wht_shared_zlen(const FineOp<T> &op, Epi epi, int nvec);
 template <typename T>
 void fine_wht(hipStream_t s, const FineOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep);
 
