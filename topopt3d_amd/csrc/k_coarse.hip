@@ -552,6 +552,11 @@ __global__ __launch_bounds__(NT) void k_stencil_op_sym_mv(StencilOp<T> op, const
     stencil_sym_block_mv<T, EPI, V>(op, u0, ep, nn, blockIdx.x, gridDim.x);
 }
 
+// The operator of several instances' levels in one grid, V vectors per thread: entry e owns blocks
+// [b0[e], b0[e + 1]); small and large grids share the launch.  One vector takes the rolled node form
+// too: the unrolled one of single launches, in one kernel with the split form, held that to its own
+// 323 registers and one wavefront per SIMD (32 instances of 16 to 96 elements along x, one load case,
+// mixed: 34.4 -> 22.4 ms a solve, at 58 registers; groups of nine neighbours at 104: 23.2).
 template <typename T, int EPI, int V>
 __global__ __launch_bounds__(NT) void k_stencil_op_sym_mv_batch(const StencilLaunch<T> *__restrict__ tab,
                                                                 const int *__restrict__ b0, int n)
@@ -563,21 +568,6 @@ __global__ __launch_bounds__(NT) void k_stencil_op_sym_mv_batch(const StencilLau
     stencil_split_block<T, EPI, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks, V * blockIdx.y);
   else
     stencil_sym_block_mv<T, EPI, V>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
-}
-
-// The operator of several instances' levels in one grid: entry e owns blocks
-// [b0[e], b0[e + 1]); small and large grids share the launch.
-template <typename T, int EPI>
-__global__ __launch_bounds__(NT) void k_stencil_op_sym_batch(const StencilLaunch<T> *__restrict__ tab,
-                                                             const int *__restrict__ b0, int n)
-{
-  const int e = batch_entry(b0, n, blockIdx.x);
-  const StencilLaunch<T> L = tab[e];
-  const int blk = blockIdx.x - b0[e];
-  if (L.nn < L.op.split_nodes)
-    stencil_split_block<T, EPI, 1>(L.op, L.u, L.ep, L.nn, blk, L.nblocks, blockIdx.y);
-  else
-    stencil_sym_block<T, EPI>(L.op, L.u, L.ep, L.nn, blk, L.nblocks);
 }
 
 // Start of the estimates of tab's levels: the copies in T of the FP64 inverse diagonal and of
@@ -1244,20 +1234,14 @@ void stencil_op_sym(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, 
 }
 
 template <typename T, int EPI>
-void launch_sym_batch(hipStream_t s, const StencilLaunch<T> *tab, const int *b0, int n,
-                      int nblocks_total, int nvec)
-{
-  k_stencil_op_sym_batch<T, EPI><<<dim3(nblocks_total, nvec), dim3(NT), 0, s>>>(tab, b0, n);
-}
-
-template <typename T, int EPI>
 void launch_sym_mv_batch(hipStream_t s, const StencilLaunch<T> *tab, const int *b0, int n,
                          int nblocks_total, int nvec, int V)
 {
   const dim3 grid(nblocks_total, nvec / V), block(NT);
   if (V == 4) k_stencil_op_sym_mv_batch<T, EPI, 4><<<grid, block, 0, s>>>(tab, b0, n);
   else if (V == 3) k_stencil_op_sym_mv_batch<T, EPI, 3><<<grid, block, 0, s>>>(tab, b0, n);
-  else k_stencil_op_sym_mv_batch<T, EPI, 2><<<grid, block, 0, s>>>(tab, b0, n);
+  else if (V == 2) k_stencil_op_sym_mv_batch<T, EPI, 2><<<grid, block, 0, s>>>(tab, b0, n);
+  else k_stencil_op_sym_mv_batch<T, EPI, 1><<<grid, block, 0, s>>>(tab, b0, n);
 }
 
 template <typename T>
@@ -1265,20 +1249,9 @@ void stencil_sym_batch(hipStream_t s, Epi epi, const StencilLaunch<T> *tab, cons
                        int nblocks_total, int nvec)
 {
   const int V = stencil_mv_width(nvec, epi, nblocks_total);
-  if (V > 1) {
-    if (epi == EPI_CHEB) launch_sym_mv_batch<T, EPI_CHEB>(s, tab, b0, n, nblocks_total, nvec, V);
-    else launch_sym_mv_batch<T, EPI_RESID>(s, tab, b0, n, nblocks_total, nvec, V);
-    TOFE_LAUNCH_CHECK();
-    return;
-  }
-  switch (epi) {
-    case EPI_APPLY: launch_sym_batch<T, EPI_APPLY>(s, tab, b0, n, nblocks_total, nvec); break;
-    case EPI_APPLY_DOT: launch_sym_batch<T, EPI_APPLY_DOT>(s, tab, b0, n, nblocks_total, nvec); break;
-    case EPI_APPLY_DOT2: launch_sym_batch<T, EPI_APPLY_DOT2>(s, tab, b0, n, nblocks_total, nvec); break;
-    case EPI_RESID: launch_sym_batch<T, EPI_RESID>(s, tab, b0, n, nblocks_total, nvec); break;
-    case EPI_CHEB: launch_sym_batch<T, EPI_CHEB>(s, tab, b0, n, nblocks_total, nvec); break;
-    default: throw Error(TOFE_ERR_ARG, "epilogue not available for stencil levels");
-  }
+  if (epi == EPI_CHEB) launch_sym_mv_batch<T, EPI_CHEB>(s, tab, b0, n, nblocks_total, nvec, V);
+  else if (epi == EPI_RESID) launch_sym_mv_batch<T, EPI_RESID>(s, tab, b0, n, nblocks_total, nvec, V);
+  else throw Error(TOFE_ERR_ARG, "epilogue not available for a batch's stencil levels");
   TOFE_LAUNCH_CHECK();
 }
 
