@@ -1,0 +1,36 @@
+"""V-cycles on several vectors on either side of the rules that give such launches another stencil
+form, and with the threshold between the forms given: every vector keeps its single launch's bits."""
+import pytest
+
+from topopt3d_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+
+# level 1 holds 70,785 nodes, 277 blocks of nodes a vector: 8 vectors stay below the bound of 2,400, 9
+# reach it without filling the GPU with three vectors per thread, 10, 12 and 16 take the node form with two,
+# three and four vectors per thread
+@pytest.mark.parametrize("split", [None, "0", "1000000"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_block_vcycle_forms(tofe, monkeypatch, precision, split):
+    import torch
+
+    print(f"case block forms precision={precision} split={split}", flush=True)
+    nel = (128, 64, 64)
+    pb = configs.cantilever(nel, seed=5, lo=0.05, hi=1.0)
+    if split is not None:
+        monkeypatch.setenv("TOFE_STENCIL_SPLIT_NODES", split)
+    c = tofe.Context(nel, fixed_dof=pb.fixed_dof, precision=precision)
+    c.set_design(pb.x)
+    c.assemble()
+    R = torch.randn((16, pb.ndof), dtype=torch.float64, generator=torch.Generator().manual_seed(2)).cuda()
+    R[:, torch.from_numpy(pb.fixed_dof.astype(bool)).cuda()] = 0
+    Z1, Z = torch.empty_like(R), torch.empty_like(R)
+    for j in range(16):
+        c.pc_apply_dev(R[j].data_ptr(), Z1[j].data_ptr(), 1)
+    assert torch.isfinite(Z1).all() and Z1.abs().max() > 0
+    for nv in (8, 9, 10, 12, 16):
+        Z.zero_()
+        c.pc_apply_dev(R.data_ptr(), Z.data_ptr(), nv)
+        assert torch.equal(Z[:nv], Z1[:nv]), nv
+    c.close()

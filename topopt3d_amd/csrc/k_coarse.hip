@@ -1199,14 +1199,31 @@ int stencil_mv_width(int nvec, Epi epi, int64_t nblocks)
   return 1;
 }
 
-template <typename T, int EPI, int V>
-void launch_sym_mv(hipStream_t s, StencilOp<T> op, const T *u, const EpiArgs<T> &ep)
+// Enough vectors fill the GPU with one thread per node, which reads a stencil value for all three
+// components' sums at once.  V-cycles, level 1 per node over split (time ratio, FP64 / FP32), by
+// nodes / 256 x vectors: up to 2,000 1.10 to 1.16 / 1.07 to 1.15; 2,128 (136,161 nodes) 1.00 / 1.03;
+// 2,216 (70,785) 1.02 / 1.04; 2,256 (47,937) 1.00 / 0.98; 3,008 (47,937) 1.00 / 0.99; 3,192 (136,161)
+// 0.91 / 0.95; 4,432 (70,785) 0.91 / 0.95; 8,512 (136,161) 0.87 / 0.93.  Merged batches follow the
+// rule with what the launch holds (12 and 32 instances of 16 to 96 elements along x, four load
+// cases, ms a solve: split 29.6 and 54.1, this way 28.5 and 51.7; per node from 4,096 nodes on 28.5 and
+// 50.7, FP64 45.3 for 12 against 42.6).  With one vector per thread, where a value serves one vector
+// only, the split form stayed the faster one (12.2 and 13.1).
+constexpr int64_t kNodeFormNodes = 16384, kNodeFormBlocks = 2400;
+template <typename T>
+int64_t stencil_shared_split(const StencilOp<T> &op, Epi epi, int nvec, double share)
 {
   const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
-  // enough vectors fill the GPU with one thread per node, which reads a stencil value for all three
-  // components' sums at once (V-cycle on 16 vectors of 160x80x80, FP64: 4,566 us per node, 4,874 in
-  // groups; on 4 vectors 1,404 and 1,337)
-  if (nn >= 16384 && (nn + NT - 1) / NT * ep.nvec >= 4 * kMvMinBlocks) op.split_nodes = 0;
+  const double nb = (double)((nn + NT - 1) / NT) * share;
+  if (op.split_given || nn < kNodeFormNodes || nb * nvec < kNodeFormBlocks ||
+      stencil_mv_width(nvec, epi, (int64_t)nb) == 1)
+    return op.split_nodes;
+  return 0;
+}
+
+template <typename T, int EPI, int V>
+void launch_sym_mv(hipStream_t s, const StencilOp<T> &op, const T *u, const EpiArgs<T> &ep)
+{
+  const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
   const dim3 grid((unsigned)stencil_op_blocks<T>(op), ep.nvec / V), block(NT);
   if (nn < op.split_nodes) k_stencil_op_sym_mv<T, EPI, true, V><<<grid, block, 0, s>>>(op, u, ep, nn);
   else k_stencil_op_sym_mv<T, EPI, false, V><<<grid, block, 0, s>>>(op, u, ep, nn);
@@ -1221,8 +1238,10 @@ void launch_sym_mv(hipStream_t s, const StencilOp<T> &op, const T *u, const EpiA
 }
 
 template <typename T>
-void stencil_op_sym(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep)
+void stencil_op_sym(hipStream_t s, const StencilOp<T> &op0, const T *u, Epi epi, const EpiArgs<T> &ep)
 {
+  StencilOp<T> op = op0;
+  op.split_nodes = stencil_shared_split(op, epi, ep.nvec, 1.0);
   const int V = stencil_mv_width(ep.nvec, epi, stencil_op_blocks<T>(op));
   if (V > 1) {
     if (epi == EPI_CHEB) launch_sym_mv<T, EPI_CHEB>(s, op, u, ep, V);
@@ -1372,6 +1391,8 @@ template void lz_start<float>(hipStream_t, const LzTab<float> &);
 template void lz_start<double>(hipStream_t, const LzTab<double> &);
 template void lz_apply<float>(hipStream_t, const LzTab<float> &);
 template void lz_apply<double>(hipStream_t, const LzTab<double> &);
+template int64_t stencil_shared_split<double>(const StencilOp<double> &, Epi, int, double);
+template int64_t stencil_shared_split<float>(const StencilOp<float> &, Epi, int, double);
 template void stencil_op_sym<double>(hipStream_t, const StencilOp<double> &, const double *, Epi,
                                      const EpiArgs<double> &);
 template void stencil_op_sym<float>(hipStream_t, const StencilOp<float> &, const float *, Epi,

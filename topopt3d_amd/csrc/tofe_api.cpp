@@ -281,6 +281,7 @@ struct tofe_ctx {
   bool coarse_unjoined = false, coarse_unchecked = false;
   bool fine_mfma = false;  // TOFE_FINE_MFMA=1: element-centric MFMA fine operator
   int64_t split_nodes = kStencilSplitNodes;  // TOFE_STENCIL_SPLIT_NODES: below, four wavefronts per sum
+  bool split_given = false;                  // by the variable: then it holds for every launch
   FineTile fine_tile{0, 8}, fine_tile32{0, 8};  // k_fine_op launch shapes, FP64 and FP32
                                                 // (TOFE_FINE_TILE="<shape>:<zlen>" sets both)
   bool ke_sym = false;  // KE matches the cube-orbit table: fine operator keeps KE in registers
@@ -464,6 +465,8 @@ void level_record(tofe_ctx *c, int l, const T *u, Epi epi, const EpiArgs<T> &ep)
       d.op.S = f32 ? lv.S.p : lv.Su.p;
       d.op.Nx = lv.g.Nx; d.op.Ny = lv.g.Ny; d.op.Nz = lv.g.Nz;
       d.op.split_nodes = c->split_nodes;
+      d.op.split_given = c->split_given;
+      d.op.split_nodes = stencil_shared_split<T>(d.op, epi, ep.nvec, c->rec->share);
       d.u = u;
       d.ep = ep;
       d.nn = lv.g.nn();
@@ -502,6 +505,7 @@ void level_apply_now(tofe_ctx *c, int l, const T *u, Epi epi, const EpiArgs<T> &
     op.S = lv.S.p;
     op.Nx = lv.g.Nx; op.Ny = lv.g.Ny; op.Nz = lv.g.Nz;
     op.split_nodes = c->split_nodes;
+    op.split_given = c->split_given;
     const bool timed = kernel_timer_begin(c, s, l, sizeof(T) == 4, epi);
     // FP32 levels keep the upper half of the (exactly symmetric) Galerkin stencil; FP64 levels
     // read their upper-half copy once the FP64 set-up has formed it (half the stencil traffic)
@@ -1739,7 +1743,7 @@ void autotune(tofe_ctx *c, int nrep, int *zlen_out, int64_t *split_out)
   for (int l = 1; l < c->L; ++l) {
     c->split_nodes = 0;  // every grid one thread per node
     t_node[l] = time_level_op(c, l, f32, EPI_CHEB, nrep);
-    c->split_nodes = INT64_MAX;  // every grid one thread per DOF
+    c->split_nodes = INT64_MAX;  // every grid in the split form
     t_dof[l] = time_level_op(c, l, f32, EPI_CHEB, nrep);
   }
   int64_t best_split = keep_split;
@@ -1921,7 +1925,10 @@ int tofe_create(const tofe_desc *desc, tofe_ctx **out)
   try {
     TOFE_HIP(hipGetDevice(&c->device));
     if (const char *fm = std::getenv("TOFE_FINE_MFMA")) c->fine_mfma = fm[0] == '1';
-    if (const char *sn = std::getenv("TOFE_STENCIL_SPLIT_NODES")) c->split_nodes = std::atoll(sn);
+    if (const char *sn = std::getenv("TOFE_STENCIL_SPLIT_NODES")) {
+      c->split_nodes = std::atoll(sn);
+      c->split_given = true;
+    }
     // level count: floor(log2(min nel)) unless given (RecMesh.cpp:552-554), truncated
     // once a coarse grid has <= 10 DOFs (Interpolation.cpp:70-71)
     int L = d.mg_levels;

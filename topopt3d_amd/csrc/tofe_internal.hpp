@@ -115,8 +115,9 @@ void fine_stress(hipStream_t s, const FineOp<double> &op, const double *u, const
 
 // Stored 27-point block stencil operator of a coarse level.
 // Stencil grids with fewer nodes than this sum a DOF's neighbours in four wavefronts instead of one
-// thread summing a node's (measured: k_coarse.hip).  TOFE_STENCIL_SPLIT_NODES overrides it per
-// context.
+// thread summing a node's (measured: k_coarse.hip).  TOFE_STENCIL_SPLIT_NODES overrides it for every
+// launch of a context; by default launches that hold several vectors or instances may run larger grids
+// per node (stencil_shared_split).
 constexpr int64_t kStencilSplitNodes = 200000;
 
 template <typename T>
@@ -124,6 +125,7 @@ struct StencilOp {
   const T *S = nullptr;        // 243 * nnode
   int Nx = 0, Ny = 0, Nz = 0;  // nodes
   int64_t split_nodes = kStencilSplitNodes;  // grids below this: four wavefronts per sum
+  bool split_given = false;                  // split_nodes holds for every launch
 };
 
 constexpr int kRedBlocks = 1024;   // grid of the grid-stride reduction kernels
@@ -194,6 +196,9 @@ void stencil_op(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, cons
 // forms it from the full FP64 stencil).
 template <typename T>
 void stencil_op_sym(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep);
+// split_nodes of a launch over nvec vectors that holds `share` times this grid's nodes
+template <typename T>
+int64_t stencil_shared_split(const StencilOp<T> &op, Epi epi, int nvec, double share);
 void galerkin(hipStream_t s, const double *Sf, int Nfx, int Nfy, int Nfz, double *Sc, double *T1,
               double *T2);
 int64_t galerkin_scratch(int Nfx, int Nfy, int Nfz, int64_t *n2);
