@@ -149,9 +149,9 @@ __global__ void k_cheb_zero_from64(const double *__restrict__ b64, float *__rest
 
 // b_c(I) = sum over fine nodes i within one fine step of 2I of w(i,I) r_f(i)  (P^T r) for NQ
 // components per thread.  A coarse level's launch is a chain of latencies: a thread per DOF has its
-// 27 loads in flight at once (637 nodes, FP64: 6.6 us per node, 3.4 per DOF; 12,800 nodes x 4
-// vectors, FP32: 6.5 and 6.1).  A grid that fills the GPU is bound by the number of loads either
-// way and shares a node's indices and weights (233,000 nodes, FP32: 11.2 and 14.0).
+// 27 loads in flight at once (637 nodes, FP64: 6.6 us per node, 3.4 per DOF).  A grid that fills the GPU
+// in FP32 is bound by the number of loads either way and shares a node's indices and weights
+// (restrict_per_node).
 template <typename T, int NQ>
 __device__ __forceinline__ void restrict_block(const T *__restrict__ rf, int Nfx, int Nfy, int Nfz,
                                                T *__restrict__ bc, int Ncx, int Ncy, int Ncz,
@@ -234,15 +234,13 @@ __global__ __launch_bounds__(NT) void k_restrict(const T *__restrict__ rf, int N
   restrict_block<T, NQ>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, blockIdx.x);
 }
 
-// a thread per DOF, whatever the entries' grids: 1.2 us less per launch on 12 instances' levels of
-// up to 4,000 nodes, 0.3 more on their 39,000
-template <typename T>
+template <typename T, int NQ>
 __global__ __launch_bounds__(NT) void k_restrict_batch(const RestrictLaunch<T> *__restrict__ tab,
                                                        const int *__restrict__ b0, int n)
 {
   const int e = batch_entry(b0, n, blockIdx.x);
   const RestrictLaunch<T> L = tab[e];
-  restrict_block<T, 1>(L.rf, L.Nfx, L.Nfy, L.Nfz, L.bc, L.Ncx, L.Ncy, L.Ncz, L.fs, blockIdx.x - b0[e]);
+  restrict_block<T, NQ>(L.rf, L.Nfx, L.Nfy, L.Nfz, L.bc, L.Ncx, L.Ncy, L.Ncz, L.fs, blockIdx.x - b0[e]);
 }
 
 // x_f(i) += sum over coarse parents J of w(i,J) x_c(J)  (P x_c)
@@ -665,9 +663,14 @@ void cheb_zero_from64(hipStream_t s, const double *b64, float *b32, const float 
   TOFE_LAUNCH_CHECK();
 }
 
-// coarse nodes x vectors from which the restriction takes a thread per node: 72,000 take 6.5 us per
-// node and 6.1 per DOF, 78,000 7.0 and 7.3
-constexpr int64_t kRestrictNode = 75000;
+// coarse nodes x vectors (of every instance of a batch) from which the FP32 restriction takes a thread
+// per node, us per node and per DOF: 38,900 5.0 and 4.9, 61,400 5.1 and 6.0, 233,000 10.4 and 12.9,
+// 932,000 34 and 51.  In FP64 the three components' loads do not stay in flight together and a thread
+// per DOF is the faster one throughout: 4,400 5.2 and 3.8, 61,400 7.4 and 7.0, 233,000 23.4 and 17.9,
+// 932,000 82 and 63.
+constexpr int64_t kRestrictNode = 50000;
+bool restrict_per_node(bool fp32, double nodes) { return fp32 && nodes >= kRestrictNode; }
+int restrict_blocks(int64_t ncn, bool node) { return (int)(((node ? 1 : 3) * ncn + NT - 1) / NT); }
 
 template <typename T>
 void restrict_op(hipStream_t s, const T *rf, int Nfx, int Nfy, int Nfz, T *bc, int Ncx, int Ncy,
@@ -675,10 +678,15 @@ void restrict_op(hipStream_t s, const T *rf, int Nfx, int Nfy, int Nfz, T *bc, i
                  const ReduceTail &tail)
 {
   const int64_t ncn = (int64_t)Ncx * Ncy * Ncz;
-  const bool node = ncn * nvec >= kRestrictNode;
-  const dim3 grid((unsigned)(((node ? 1 : 3) * ncn + NT - 1) / NT + (tail.partial ? 1 : 0)), nvec);
-  if (node) k_restrict<T, 3><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
-  else k_restrict<T, 1><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
+  const bool node = restrict_per_node(sizeof(T) == 4, (double)ncn * nvec);
+  const dim3 grid((unsigned)(restrict_blocks(ncn, node) + (tail.partial ? 1 : 0)), nvec);
+  if constexpr (sizeof(T) == 4)
+    if (node) {
+      k_restrict<T, 3><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
+      TOFE_LAUNCH_CHECK();
+      return;
+    }
+  k_restrict<T, 1><<<grid, dim3(NT), 0, s>>>(rf, Nfx, Nfy, Nfz, bc, Ncx, Ncy, Ncz, fs, tail);
   TOFE_LAUNCH_CHECK();
 }
 
@@ -776,9 +784,16 @@ void fcg_update_xp_batch(hipStream_t s, const FcgPLaunch *tab, const int *b0, in
 
 template <typename T>
 void restrict_batch(hipStream_t s, const RestrictLaunch<T> *tab, const int *b0, int n,
-                    int nblocks_total, int nvec)
+                    int nblocks_total, int nvec, bool node)
 {
-  k_restrict_batch<T><<<dim3(nblocks_total, nvec), dim3(NT), 0, s>>>(tab, b0, n);
+  const dim3 grid(nblocks_total, nvec);
+  if constexpr (sizeof(T) == 4)
+    if (node) {
+      k_restrict_batch<T, 3><<<grid, dim3(NT), 0, s>>>(tab, b0, n);
+      TOFE_LAUNCH_CHECK();
+      return;
+    }
+  k_restrict_batch<T, 1><<<grid, dim3(NT), 0, s>>>(tab, b0, n);
   TOFE_LAUNCH_CHECK();
 }
 
@@ -822,7 +837,7 @@ void lz_p(hipStream_t s, const LzTab<T> &tab, int k)
   template void restrict_op<T>(hipStream_t, const T *, int, int, int, T *, int, int, int,        \
                                const FirstStep<T> &, int, const ReduceTail &);                \
   template void prolong_add<T>(hipStream_t, const T *, int, int, int, T *, int, int, int, int); \
-  template void restrict_batch<T>(hipStream_t, const RestrictLaunch<T> *, const int *, int, int, int); \
+  template void restrict_batch<T>(hipStream_t, const RestrictLaunch<T> *, const int *, int, int, int, bool); \
   template void prolong_batch<T>(hipStream_t, const ProlongLaunch<T> *, const int *, int, int, int); \
 
 TOFE_INST_T(double)

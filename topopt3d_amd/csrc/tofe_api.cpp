@@ -141,8 +141,8 @@ enum BatchKind : int {
   BK_FCG_P = 8,
   BK_REDUCE = 9,
 };
-// kind, precision, element form (fine operator) and epilogue in one key: ops with equal keys
-// share a launch
+// kind, precision, element form (fine operator) and epilogue (restriction: form) in one key: ops with
+// equal keys share a launch
 constexpr int batch_key(int kind, bool fp32, int epi = 0, bool cube = false)
 {
   return (kind << 8) | ((fp32 ? 1 : 0) << 7) | ((cube ? 1 : 0) << 6) | epi;
@@ -799,8 +799,9 @@ void vcycle(tofe_ctx *c, const T *b0, T *x0, VcycleIO *io = nullptr, int nvec = 
       d.rf = lv.r.p; d.Nfx = gf.Nx; d.Nfy = gf.Ny; d.Nfz = gf.Nz;
       d.bc = LV[l + 1]->b.p; d.Ncx = gc.Nx; d.Ncy = gc.Ny; d.Ncz = gc.Nz;
       d.fs = fs;
-      d.nblocks = (int)((gc.ndof() + 255) / 256);
-      rec_push(c, batch_key(BK_RESTRICT, sizeof(T) == 4), d, d.nblocks);
+      const bool node = restrict_per_node(sizeof(T) == 4, (double)gc.nn() * nvec * c->rec->share);
+      d.nblocks = restrict_blocks(gc.nn(), node);
+      rec_push(c, batch_key(BK_RESTRICT, sizeof(T) == 4, node), d, d.nblocks);
     } else {
       const ReduceTail tail = l == 0 && io ? io->tail : ReduceTail();
       restrict_op<T>(s, lv.r.p, gf.Nx, gf.Ny, gf.Nz, LV[l + 1]->b.p, gc.Nx, gc.Ny, gc.Nz, fs, nvec, tail);
@@ -3246,8 +3247,8 @@ struct BatchProgram {
           else stencil_sym_batch<double>(s, (Epi)epi, tab<StencilLaunch<double>>(st), b0, st.n, st.total, nvec);
           break;
         case BK_RESTRICT:
-          if (f32) restrict_batch<float>(s, tab<RestrictLaunch<float>>(st), b0, st.n, st.total, nvec);
-          else restrict_batch<double>(s, tab<RestrictLaunch<double>>(st), b0, st.n, st.total, nvec);
+          if (f32) restrict_batch<float>(s, tab<RestrictLaunch<float>>(st), b0, st.n, st.total, nvec, epi != 0);
+          else restrict_batch<double>(s, tab<RestrictLaunch<double>>(st), b0, st.n, st.total, nvec, epi != 0);
           break;
         case BK_PROLONG:
           if (f32) prolong_batch<float>(s, tab<ProlongLaunch<float>>(st), b0, st.n, st.total, nvec);

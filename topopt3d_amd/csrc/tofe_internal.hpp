@@ -361,8 +361,12 @@ void fcg_update_xp(hipStream_t s, double *p, const double *z, const float *z32, 
                    int64_t n, const double *zq_part, int nparts, double *scal, int nvec = 1);
 void fcg_update_x(hipStream_t s, double *x, const double *p, int64_t n, const double *scal,
                   int nvec = 1);
+// Whether a restriction of so many coarse nodes (times vectors) takes a thread per node, or per DOF;
+// and its blocks per vector.
+bool restrict_per_node(bool fp32, double nodes);
+int restrict_blocks(int64_t ncn, bool node);
 // Batched forms of the V-cycle's transfers and of the flexible-CG updates: one entry per
-// instance, with the blocks per vector of the single launch (restriction: coarse nodes / 256,
+// instance, with the blocks per vector of the single launch (restriction: restrict_blocks,
 // prolongation: fine nodes / 256, fcg_update_r_blocks, fcg_update_xp_blocks, reduction: 1).
 template <typename T>
 struct RestrictLaunch {
@@ -423,7 +427,7 @@ void fcg_update_xp_batch(hipStream_t s, const FcgPLaunch *tab, const int *b0, in
                          int nblocks_total, int nvec);
 template <typename T>
 void restrict_batch(hipStream_t s, const RestrictLaunch<T> *tab, const int *b0, int n,
-                    int nblocks_total, int nvec);
+                    int nblocks_total, int nvec, bool node);
 template <typename T>
 void prolong_batch(hipStream_t s, const ProlongLaunch<T> *tab, const int *b0, int n,
                    int nblocks_total, int nvec);
