@@ -344,10 +344,12 @@ int tofe_time_kernels(tofe_ctx *ctx, int start, tofe_kernel_time *out, int max_k
                       int *nkinds);
 
 /* Launch shapes from measurement (no reference counterpart: PETSc has no such knob): for
- * the precision of the last assemble, times the fine operator's Chebyshev step over
- * candidate z-chunk lengths and every coarse level's stencil kernel one thread per node
- * and split over four wavefronts (nrep launches each), keeps the fastest chunk length and
- * the node-count threshold below which levels run split that minimises their summed time.
+ * the precision of the last assemble, times the fine operator's Chebyshev step at its
+ * current z-chunk length and at 1 to 24 planes, and every coarse level's stencil kernel one
+ * thread per node and split over four wavefronts (nrep launches each); keeps the fastest
+ * chunk length and the node-count threshold below which levels run split that minimises
+ * their summed time, for launches over one vector (several vectors, or a batch's instances,
+ * lengthen short chunks and choose the stencil form by what the launch holds).
  * Outputs (may be NULL): the chunk length and the threshold. */
 int tofe_autotune(tofe_ctx *ctx, int nrep, int *fine_zlen, int64_t *split_nodes);
 

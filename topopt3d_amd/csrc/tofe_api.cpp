@@ -1716,22 +1716,27 @@ double time_level_op(tofe_ctx *c, int level, bool f32, Epi epi, int nrep)
 }
 
 // Launch shapes of the current precision's operators from measurement: the fine operator's
-// z-chunk length (element-centric form) over candidate lengths, and the node-count
-// threshold below which a stencil level runs in the split form, chosen to minimise the
-// summed Chebyshev-step time of the coarse levels.  The chosen shapes stay in the context.
+// z-chunk length (element-centric form) over candidate lengths, the current one first and kept
+// unless another is faster, and the node-count threshold below which a stencil level runs in the
+// split form, chosen to minimise the summed Chebyshev-step time of the coarse levels.  The chosen
+// shapes stay in the context, for launches over one vector; those that hold several vectors or a batch's
+// instances lengthen short chunks and choose the stencil form by their own rules.
 void autotune(tofe_ctx *c, int nrep, int *zlen_out, int64_t *split_out)
 {
   need_assembled(c);
   const bool f32 = c->built_precision == TOFE_PREC_MIXED;
   int best_z = f32 ? c->wht_zlen32 : c->wht_zlen;
   if (c->ke_wht && !c->fine_mfma) {
-    double best = 1e300;
+    // the default rule's lengths among them: 24x12x12 runs its steps at one plane, 5.1 us against 9.1 at
+    // four, and a solve in 0.91 ms against 1.16
     const int keep = best_z;
-    for (int zl : {4, 5, 6, 8, 10, 12, 16, 20, 24}) {
-      if (zl > c->desc.nz + 1 && zl != keep) continue;
+    double best = time_level_op(c, 0, f32, EPI_CHEB, nrep);
+    best = std::min(best, time_level_op(c, 0, f32, EPI_CHEB, nrep));  // the first one starts cold
+    for (int zl : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24}) {
+      if (zl > c->desc.nz + 1 || zl == keep) continue;
       (f32 ? c->wht_zlen32 : c->wht_zlen) = zl;
       const double t = time_level_op(c, 0, f32, EPI_CHEB, nrep);
-      if (t < best * 0.995) {  // a longer chunk must win clearly (fewer blocks, less halo)
+      if (t < best * 0.995) {  // another length must win clearly
         best = t;
         best_z = zl;
       }
