@@ -25,7 +25,6 @@ template <typename T, int EPI>
 __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
                                                    EpiArgs<T> ep, int64_t nn)
 {
-  __shared__ double sred[NT / 64];
   epi_select_vector(ep, u0, 3 * nn, gridDim.x);  // vector blockIdx.y
   const T *__restrict__ u = u0;
   const int64_t n = block_node(blockIdx.x, gridDim.x);
@@ -50,11 +49,10 @@ __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
       const T u0 = u[3 * m], u1 = u[3 * m + 1], u2 = u[3 * m + 2];
 #pragma unroll
       for (int c = 0; c < NA; ++c) {
-        const int a = c;
         T t = acc[c];
-        t += S[(int64_t)(o * 9 + a * 3 + 0) * nn + n] * u0;
-        t += S[(int64_t)(o * 9 + a * 3 + 1) * nn + n] * u1;
-        t += S[(int64_t)(o * 9 + a * 3 + 2) * nn + n] * u2;
+        t += S[(int64_t)(o * 9 + c * 3 + 0) * nn + n] * u0;
+        t += S[(int64_t)(o * 9 + c * 3 + 1) * nn + n] * u1;
+        t += S[(int64_t)(o * 9 + c * 3 + 2) * nn + n] * u2;
         acc[c] = in ? t : acc[c];
       }
     }
@@ -62,15 +60,6 @@ __global__ __launch_bounds__(NT) void k_stencil_op(StencilOp<T> op, const T *u0,
     for (int c = 0; c < NA; ++c) {
       const int64_t dof = 3 * n + c;
       apply_epilogue<T, EPI>(ep, dof, acc[c], u[dof], dsum, dsum2);
-    }
-  }
-  if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2 || EPI == EPI_CHEB_OUT) {
-    const double t = block_sum<NT>(dsum, sred);
-    if (threadIdx.x == 0) ep.partial[blockIdx.x] = t;
-    if constexpr (EPI == EPI_APPLY_DOT2) {
-      __syncthreads();
-      const double t2 = block_sum<NT>(dsum2, sred);
-      if (threadIdx.x == 0) ep.partial2[blockIdx.x] = t2;
     }
   }
 }
@@ -238,10 +227,8 @@ __host__ __device__ inline int64_t su_index(int v, int64_t n)
 // Neighbours per iteration of the rolled neighbour loop (3, 9 or 27).  27 for FP32 selects
 // the fully unrolled form; FP64 keeps one dz plane (9) per iteration, 220 VGPRs and no spills.
 // Level-1 Chebyshev step on the 192x96x96 cantilever: FP32 31 us (27) / 34 us (9 or 3); FP64
-// 62 us (9) / 75 us (3); the fully unrolled FP64 instance spills.  The FP32 one-thread-per-DOF
-// instances take the rolled form's branch-free body with all 27 neighbours unrolled: 5.3 us
-// against 5.8 us per Chebyshev step on level 3 (4,225 nodes); per node that body is slower
-// (33.6 against 31.2 us on level 1).
+// 62 us (9) / 75 us (3); the fully unrolled FP64 instance spills.  (The rolled form's branch-free body
+// with all 27 neighbours unrolled is slower in FP32: 33.6 against 31.2 us on level 1.)
 #ifndef TOFE_SYM32_G
 #define TOFE_SYM32_G 27
 #endif
@@ -258,7 +245,7 @@ __device__ __forceinline__ void epi_dof_load(const EpiArgs<T> &ep, const T *__re
                                              EpiDof<T, EPI> &in)
 {
   if constexpr (EPI != EPI_APPLY && EPI != EPI_RESID) in.u = u[dof];
-  if constexpr (EPI == EPI_APPLY_DOT2 || EPI == EPI_RESID || EPI == EPI_CHEB) in.b = ep.b[dof];
+  if constexpr (EPI == EPI_RESID || EPI == EPI_CHEB) in.b = ep.b[dof];
   if constexpr (EPI == EPI_CHEB) {
     in.dinv = ep.dinv[dof];
     if (ep.c1 != T(0)) in.d = ep.d[dof];
@@ -266,11 +253,10 @@ __device__ __forceinline__ void epi_dof_load(const EpiArgs<T> &ep, const T *__re
 }
 template <typename T, int EPI>
 __device__ __forceinline__ void epi_dof_store(const EpiArgs<T> &ep, int64_t dof, const EpiDof<T, EPI> &in,
-                                              T Au, double &dsum, double &dsum2)
+                                              T Au, double &dsum)
 {
-  if constexpr (EPI == EPI_APPLY || EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) ep.y[dof] = Au;
-  if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) dsum += (double)in.u * (double)Au;
-  if constexpr (EPI == EPI_APPLY_DOT2) dsum2 += (double)in.u * (double)in.b;
+  if constexpr (EPI == EPI_APPLY || EPI == EPI_APPLY_DOT) ep.y[dof] = Au;
+  if constexpr (EPI == EPI_APPLY_DOT) dsum += (double)in.u * (double)Au;
   if constexpr (EPI == EPI_RESID) ep.y[dof] = in.b - Au;
   if constexpr (EPI == EPI_CHEB) {
     const T r = in.dinv * (in.b - Au);
@@ -348,7 +334,7 @@ __device__ __forceinline__ void stencil_split_block(const StencilOp<T> &op, cons
   if (g > 0) return;
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    double dsum = 0, dsum2 = 0;
+    double dsum = 0;
     EpiArgs<T> ep = ep0;
     epi_offset(ep, v0 + v, ndof, nb);
     if (live) {
@@ -357,15 +343,11 @@ __device__ __forceinline__ void stencil_split_block(const StencilOp<T> &op, cons
       for (int o = 0; o < kGroup; ++o) acc += own[v][o];
 #pragma unroll
       for (int o = kGroup; o < 27; ++o) acc += term[v][o - kGroup][lane];
-      epi_dof_store<T, EPI>(ep, dof, ein[v], acc, dsum, dsum2);
+      epi_dof_store<T, EPI>(ep, dof, ein[v], acc, dsum);
     }
-    if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2) {
+    if constexpr (EPI == EPI_APPLY_DOT) {
       const double t = wave_sum(dsum);
       if (lane == 0) ep.partial[blk] = t;
-      if constexpr (EPI == EPI_APPLY_DOT2) {
-        const double t2 = wave_sum(dsum2);
-        if (lane == 0) ep.partial2[blk] = t2;
-      }
     }
   }
 }
@@ -402,14 +384,13 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
         const T u0 = u[3 * m], u1 = u[3 * m + 1], u2 = u[3 * m + 2];
 #pragma unroll
         for (int c = 0; c < NA; ++c) {
-          const int a = c;
           T t;
           if (o >= 13) {
             const T *B = S + su_index((o - 13) * 9, n);
-            t = row3(B[(a * 3 + 0) * 64], B[(a * 3 + 1) * 64], B[(a * 3 + 2) * 64], u0, u1, u2);
+            t = row3(B[(c * 3 + 0) * 64], B[(c * 3 + 1) * 64], B[(c * 3 + 2) * 64], u0, u1, u2);
           } else {
             const T *B = S + su_index((13 - o) * 9, m);  // block (m, 26 - o), transposed
-            t = row3(B[(0 * 3 + a) * 64], B[(1 * 3 + a) * 64], B[(2 * 3 + a) * 64], u0, u1, u2);
+            t = row3(B[(0 * 3 + c) * 64], B[(1 * 3 + c) * 64], B[(2 * 3 + c) * 64], u0, u1, u2);
           }
           acc[c] = in ? acc[c] + t : acc[c];
         }
@@ -440,9 +421,8 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
           const int sr = up ? 3 : 1, sc = up ? 1 : 3;  // strides of (row a, column b)
 #pragma unroll
           for (int c = 0; c < NA; ++c) {
-            const int a = c;
-            const T t = row3(B[(a * sr + 0 * sc) * 64], B[(a * sr + 1 * sc) * 64],
-                             B[(a * sr + 2 * sc) * 64], u0, u1, u2);
+            const T t = row3(B[(c * sr + 0 * sc) * 64], B[(c * sr + 1 * sc) * 64],
+                             B[(c * sr + 2 * sc) * 64], u0, u1, u2);
             acc[c] = __builtin_fma(w, t, acc[c]);
           }
         }
@@ -454,14 +434,9 @@ __device__ __forceinline__ void stencil_sym_block(const StencilOp<T> &op, const 
       apply_epilogue<T, EPI>(ep, dof, acc[c], u[dof], dsum, dsum2);
     }
   }
-  if constexpr (EPI == EPI_APPLY_DOT || EPI == EPI_APPLY_DOT2 || EPI == EPI_CHEB_OUT) {
+  if constexpr (EPI == EPI_APPLY_DOT) {
     const double t = block_sum<NT>(dsum, sred);
     if (threadIdx.x == 0) ep.partial[blk] = t;
-    if constexpr (EPI == EPI_APPLY_DOT2) {
-      __syncthreads();
-      const double t2 = block_sum<NT>(dsum2, sred);
-      if (threadIdx.x == 0) ep.partial2[blk] = t2;
-    }
   }
 }
 
@@ -513,9 +488,8 @@ __device__ __forceinline__ void stencil_sym_block_mv(const StencilOp<T> &op, con
       T bv[NA][3];
 #pragma unroll
       for (int c = 0; c < NA; ++c) {
-        const int a = c;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) bv[c][q] = B[(a * sr + q * sc) * 64];
+        for (int q = 0; q < 3; ++q) bv[c][q] = B[(c * sr + q * sc) * 64];
       }
 #pragma unroll
       for (int jv = 0; jv < V; ++jv) {
@@ -1135,37 +1109,14 @@ int stencil_op_blocks(const StencilOp<T> &op)
   return nn < op.split_nodes ? 3 * (int)((nn + 63) / 64) : (int)((nn + NT - 1) / NT);
 }
 
-#define TOFE_STENCIL_SWITCH(KERNEL)                                                         \
-  do {                                                                                      \
-    const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;                                      \
-    const bool split = nn < op.split_nodes;                                                 \
-    dim3 grid((unsigned)stencil_op_blocks<T>(op), ep.nvec), block(NT);                      \
-    switch (epi) {                                                                          \
-      case EPI_APPLY:                                                                       \
-        if (split) KERNEL<T, EPI_APPLY, true><<<grid, block, 0, s>>>(op, u, ep, nn);        \
-        else KERNEL<T, EPI_APPLY, false><<<grid, block, 0, s>>>(op, u, ep, nn);             \
-        break;                                                                              \
-      case EPI_APPLY_DOT:                                                                   \
-        if (split) KERNEL<T, EPI_APPLY_DOT, true><<<grid, block, 0, s>>>(op, u, ep, nn);    \
-        else KERNEL<T, EPI_APPLY_DOT, false><<<grid, block, 0, s>>>(op, u, ep, nn);         \
-        break;                                                                              \
-      case EPI_APPLY_DOT2:                                                                  \
-        if (split) KERNEL<T, EPI_APPLY_DOT2, true><<<grid, block, 0, s>>>(op, u, ep, nn);   \
-        else KERNEL<T, EPI_APPLY_DOT2, false><<<grid, block, 0, s>>>(op, u, ep, nn);        \
-        break;                                                                              \
-      case EPI_RESID:                                                                       \
-        if (split) KERNEL<T, EPI_RESID, true><<<grid, block, 0, s>>>(op, u, ep, nn);        \
-        else KERNEL<T, EPI_RESID, false><<<grid, block, 0, s>>>(op, u, ep, nn);             \
-        break;                                                                              \
-      case EPI_CHEB:                                                                        \
-        if (split) KERNEL<T, EPI_CHEB, true><<<grid, block, 0, s>>>(op, u, ep, nn);         \
-        else KERNEL<T, EPI_CHEB, false><<<grid, block, 0, s>>>(op, u, ep, nn);              \
-        break;                                                                              \
-      default:                                                                              \
-        throw Error(TOFE_ERR_ARG, "epilogue not available for stencil levels");             \
-    }                                                                                       \
-    TOFE_LAUNCH_CHECK();                                                                    \
-  } while (0)
+template <typename T, int EPI>
+void launch_sym(hipStream_t s, const StencilOp<T> &op, const T *u, const EpiArgs<T> &ep)
+{
+  const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
+  const dim3 grid((unsigned)stencil_op_blocks<T>(op), ep.nvec), block(NT);
+  if (nn < op.split_nodes) k_stencil_op_sym<T, EPI, true><<<grid, block, 0, s>>>(op, u, ep, nn);
+  else k_stencil_op_sym<T, EPI, false><<<grid, block, 0, s>>>(op, u, ep, nn);
+}
 
 template <typename T>
 void stencil_op(hipStream_t s, const StencilOp<T> &op, const T *u, Epi epi, const EpiArgs<T> &ep)
@@ -1249,7 +1200,14 @@ void stencil_op_sym(hipStream_t s, const StencilOp<T> &op0, const T *u, Epi epi,
     TOFE_LAUNCH_CHECK();
     return;
   }
-  TOFE_STENCIL_SWITCH(k_stencil_op_sym);
+  switch (epi) {
+    case EPI_APPLY: launch_sym<T, EPI_APPLY>(s, op, u, ep); break;
+    case EPI_APPLY_DOT: launch_sym<T, EPI_APPLY_DOT>(s, op, u, ep); break;
+    case EPI_RESID: launch_sym<T, EPI_RESID>(s, op, u, ep); break;
+    case EPI_CHEB: launch_sym<T, EPI_CHEB>(s, op, u, ep); break;
+    default: throw Error(TOFE_ERR_ARG, "epilogue not available for stencil levels");
+  }
+  TOFE_LAUNCH_CHECK();
 }
 
 template <typename T, int EPI>

@@ -54,13 +54,6 @@ __global__ __launch_bounds__(NT) void k_masked_kc(const MaskedElems me, const do
   }
 }
 
-__device__ inline int elem_form(int ex, int nel, int Nf)
-{
-  if (ex & 1) return 1;
-  if ((Nf & 1) == 0 && ex == Nf - 2) return 2;
-  return 0;
-}
-
 // Block (I, I + D) of the level-1 operator for the compile-time offset O: the sum over
 // the fine elements whose coarse window holds both nodes, in ascending element order.
 // Per direction the candidate elements are ex = 2 I - 2 + d, d = 0..3 (window start

@@ -323,11 +323,6 @@ __global__ void k_power_start(T *v, int64_t n)
     v[i] = (T)power_start_value(i);
 }
 
-__global__ void k_record(const double *scal, int slot, double *dst)
-{
-  if (threadIdx.x == 0 && blockIdx.x == 0) *dst = scal[slot];
-}
-
 // Sum of nparts per-block partial sums, formed by every block of the consuming kernel
 // in the order k_reduce_final uses (thread-strided, wave butterfly, waves in order), so
 // the value is the same bit for bit without a separate reduction launch.  Valid in all
@@ -735,12 +730,6 @@ template <typename T>
 void power_start(hipStream_t s, T *v, int64_t n)
 {
   k_power_start<T><<<dim3(stride_blocks(n)), dim3(NT), 0, s>>>(v, n);
-  TOFE_LAUNCH_CHECK();
-}
-
-void record_scalar(hipStream_t s, const double *scal, int slot, double *dst)
-{
-  k_record<<<dim3(1), dim3(64), 0, s>>>(scal, slot, dst);
   TOFE_LAUNCH_CHECK();
 }
 

@@ -333,7 +333,6 @@ void cg_update_xp(hipStream_t s, double *p, const double *z, double *x, int64_t 
                   int nparts, double *scal, int nvec = 1);
 template <typename T>
 void power_start(hipStream_t s, T *v, int64_t n);
-void record_scalar(hipStream_t s, const double *scal, int slot, double *dst);
 // Flexible-CG updates that sum the producers' partials themselves: fcg_update_r forms
 // alpha = sum(pr_part) / sum(pq_part) (stored with both sums in scal), r -= alpha q, partials
 // of r.r; fcg_update_xp forms beta = -sum(zq_part) / scal[PQ], applies the iterate's update
