@@ -99,7 +99,7 @@ FineTile fine_tile_choose(int nx, int ny, int nz, int ncu, int hide);
 // Element-centric fine operator in the Walsh-Hadamard basis of KE (k_fine_wht); hide: blocks per CU
 // that overlap for free (measured).
 constexpr int kWhtHide64 = 2, kWhtHide32 = 4;
-int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide, int nvec = 1);
+int fine_wht_zlen(int nx, int ny, int nz, int ncu, int hide, int nvec = 1, int zmax = 24);
 template <typename T>
 int fine_wht_blocks(const FineOp<T> &op);
 // chunk length of a launch that serves nvec vectors of this mesh, or as many nodes of several meshes
