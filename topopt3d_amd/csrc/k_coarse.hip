@@ -1152,23 +1152,29 @@ int stencil_mv_width(int nvec, Epi epi, int64_t nblocks)
 
 // Enough vectors fill the GPU with one thread per node, which reads a stencil value for all three
 // components' sums at once.  V-cycles, level 1 per node over split (time ratio, FP64 / FP32), by
-// nodes / 256 x vectors: up to 2,000 1.10 to 1.16 / 1.07 to 1.15; 2,128 (136,161 nodes) 1.00 / 1.03;
-// 2,216 (70,785) 1.02 / 1.04; 2,256 (47,937) 1.00 / 0.98; 3,008 (47,937) 1.00 / 0.99; 3,192 (136,161)
-// 0.91 / 0.95; 4,432 (70,785) 0.91 / 0.95; 8,512 (136,161) 0.87 / 0.93.  Merged batches follow the
-// rule with what the launch holds (12 and 32 instances of 16 to 96 elements along x, four load
-// cases, ms a solve: split 29.6 and 54.1, this way 28.5 and 51.7; per node from 4,096 nodes on 28.5 and
-// 50.7, FP64 45.3 for 12 against 42.6).  With one vector per thread, where a value serves one vector
-// only, the split form stayed the faster one (12.2 and 13.1).
-constexpr int64_t kNodeFormNodes = 16384, kNodeFormBlocks = 2400;
+// nodes / 256 x vectors in twos to fours per thread: up to 2,000 1.10 to 1.16 / 1.07 to 1.15; 2,128
+// (136,161 nodes) 1.00 / 1.03; 2,256 (47,937) 1.00 / 0.98; 2,576 (41,184) 1.03 / 1.05; 2,784 (44,541)
+// 1.01 / 1.04; 3,008 (47,937) 1.00 / 0.99; 3,192 (136,161) 0.91 / 0.95; 4,432 (70,785) 0.91 / 0.95; 8,512
+// (136,161) 0.87 / 0.93.  A merged batch holds its small grids besides, in as many vectors per thread:
+// 12 and 32 instances of 16 to 96 elements along x, four load cases (2,590 and 7,500), ms a solve:
+// split 29.6 and 54.1, this way 28.5 and 51.7; 4 instances (1,350) 15.7 and 16.0.  5, 7, 11 or 13
+// vectors run one per thread in either form, where the node form reads a third: from 30,625 nodes x 5
+// (600) on 0.86 to 1.00 / 0.92 to 0.99, on 18,081 nodes 0.97 to 1.02 / 0.97 to 1.02; single vectors
+// 0.96 to 1.07 / 0.98 to 1.05, and batches of them, per node from 16,384 nodes on, 1.04 / 1.07.
+constexpr int64_t kNodeFormNodes = 16384, kNodeFormBlocks = 3000, kNodeFormBatch = 2400;
+constexpr int64_t kNodeFormNodes1 = 30000, kNodeFormBlocks1 = 600;  // one vector per thread
 template <typename T>
 int64_t stencil_shared_split(const StencilOp<T> &op, Epi epi, int nvec, double share)
 {
   const int64_t nn = (int64_t)op.Nx * op.Ny * op.Nz;
   const double nb = (double)((nn + NT - 1) / NT) * share;
-  if (op.split_given || nn < kNodeFormNodes || nb * nvec < kNodeFormBlocks ||
-      stencil_mv_width(nvec, epi, (int64_t)nb) == 1)
+  if (op.split_given || nvec * share <= 1 || (epi != EPI_CHEB && epi != EPI_RESID) || nn < kNodeFormNodes)
     return op.split_nodes;
-  return 0;
+  const bool batch = share > 1;
+  if (stencil_mv_width(nvec, epi, INT64_MAX / 64) == 1)
+    return !batch && nn >= kNodeFormNodes1 && nb * nvec >= kNodeFormBlocks1 ? 0 : op.split_nodes;
+  return nb * nvec >= (batch ? kNodeFormBatch : kNodeFormBlocks) && stencil_mv_width(nvec, epi, (int64_t)nb) > 1
+             ? 0 : op.split_nodes;
 }
 
 template <typename T, int EPI, int V>
