@@ -449,21 +449,21 @@ int fine_wht_blocks(const FineOp<T> &op)
 }
 
 // Several vectors, or the instances of a batch, fill the CUs with longer chunks, which form fewer
-// extra element layers: the rule's best of up to eight planes for K, M and Ks (six, seven, eight and ten
+// extra element layers: the rule's best of up to eight planes for K and M (six, seven, eight and ten
 // measured alike over 48x24x24 to 160x80x80, 2 to 16 vectors; the best of all lengths cut at six lost 5 to
 // 10% where that is seven: K on 16 vectors of 61x33x27 42.8 and 38.8 us, on 2 of 200x40x40 33.7 and
-// 32.5) and of up to six for the V-cycle's kernels with their further fields (a Chebyshev step on 16
-// vectors of 160x80x80 670 us at 6, 717 at 14; V-cycle on 16 of 130x50x46 1,323 at up to 6, 1,374 at
-// up to 8).  A merged solve of 32 instances of 16 to 96 elements along x, ms: with their own lengths 57.5
+// 32.5) and of up to six for the kernels with further fields, the V-cycle's and Ks (a Chebyshev step on
+// 16 vectors of 160x80x80 670 us at 6, 717 at 14; V-cycle on 16 of 130x50x46 1,323 at up to 6, 1,374 at
+// up to 8; Ks, K and V-cycle on 10 of 128x64x64 1,367 and 1,398).  A merged solve of 32 instances of 16 to 96 elements along x, ms: with their own lengths 57.5
 // for four load cases each and 35.3 for one, this way 54.1 and 34.4.  The chunk length does not show in
 // the outputs, only in the partial sums of the dot products, where each vector's stay those of its
 // own launch.
-constexpr int kSharedZlenApply = 8, kSharedZlenCheb = 6;
+constexpr int kSharedZlenApply = 8, kSharedZlenFields = 6;
 template <typename T>
 int fine_wht_shared_zlen(const FineOp<T> &op, Epi epi, int nvec)
 {
   const bool sums = epi == EPI_APPLY_DOT || epi == EPI_APPLY_DOT2 || epi == EPI_CHEB_OUT;
-  const int zmax = epi == EPI_APPLY ? kSharedZlenApply : kSharedZlenCheb;
+  const int zmax = epi == EPI_APPLY && !op.H ? kSharedZlenApply : kSharedZlenFields;
   if (sums || nvec <= 1 || op.ncu <= 0 || op.zlen >= zmax) return op.zlen;
   return fine_wht_zlen(op.nx, op.ny, op.nz, op.ncu, sizeof(T) == 8 ? kWhtHide64 : kWhtHide32, nvec, zmax);
 }
