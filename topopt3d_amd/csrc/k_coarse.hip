@@ -1157,7 +1157,8 @@ int stencil_mv_width(int nvec, Epi epi, int64_t nblocks)
 // 1.01 / 1.04; 3,008 (47,937) 1.00 / 0.99; 3,192 (136,161) 0.91 / 0.95; 4,432 (70,785) 0.91 / 0.95; 8,512
 // (136,161) 0.87 / 0.93.  A merged batch holds its small grids besides, in as many vectors per thread:
 // 12 and 32 instances of 16 to 96 elements along x, four load cases (2,590 and 7,500), ms a solve:
-// split 29.6 and 54.1, this way 28.5 and 51.7; 4 instances (1,350) 15.7 and 16.0.  5, 7, 11 or 13
+// split 29.6 and 54.1, this way 28.5 and 51.7, from 4,096 nodes on 28.5 and 50.7 (but 12 in FP64 45.3
+// against 42.6, split 45.7, and from 30,000 on 45.1); 4 instances (1,350) 15.7 and 16.0.  5, 7, 11 or 13
 // vectors run one per thread in either form, where the node form reads a third: from 30,625 nodes x 5
 // (600) on 0.86 to 1.00 / 0.92 to 0.99, on 18,081 nodes 0.97 to 1.02 / 0.97 to 1.02; single vectors
 // 0.96 to 1.07 / 0.98 to 1.05, and batches of them, per node from 16,384 nodes on, 1.04 / 1.07.
